@@ -3,8 +3,8 @@
 // rainfall (added as h += rain*dt right after the update, where the reference adds its
 // point sources), fused into two kernels per step:
 //
-//   K1 (flux + update + rain): a wave marches up a strip of 62 columns x 32 rows, one
-//       lane per column, solving each edge once (X edges with the left cell's values
+//   K1 (flux + update + rain): a wave marches up a strip of 62 columns, one lane per
+//       column, solving each edge once (X edges with the left cell's values
 //       shifted in across lanes, Y edges from the row below kept in registers); every
 //       cell accumulates rhs*0 / rhs*1 from its four edges in the order of the
 //       reference's X-then-Y functors, applies the update with implicit Manning
@@ -41,6 +41,7 @@
 
 #include <algorithm>
 #include <cfloat>
+#include <cmath>
 #include <vector>
 
 using namespace appfis;
@@ -74,7 +75,7 @@ struct Scen {
     const R* z;
     const R* n2;
     int nx, ny;
-    int strips_x;      // strips of MW x MR cells (every kernel of the step works on them)
+    int strips_x;      // strips of MW columns x mr rows (every kernel of the step works on them)
     int strip0;        // first global strip of this scenario
     int nstrips;
     ScenState* st;
@@ -344,9 +345,9 @@ __device__ inline void cell_derive(CellV<R>& c, R hextra)
     velocity(c.h, c.qx, c.qy, hextra, c.u, c.v);
 }
 
-// K1 as a row march.  A wave owns a strip of MW columns x MR rows; lane l holds column
+// K1 as a row march.  A wave owns a strip of MW columns x mr rows; lane l holds column
 // i0-1+l, so lanes 1..MW are the strip's cells and lanes 0 and 63 its halo columns.  The
-// wave walks the rows j0-1 .. j0+MR keeping two rows in registers:
+// wave walks the rows j0-1 .. j0+mr keeping two rows in registers:
 //   X edge of row j between columns (c-1, c): solved by the lane of c, with the left
 //     cell's values shifted in from lane l-1; the cell on the right of the edge takes
 //     rhs*1, the left cell's rhs*0 is shifted back to lane l-1;
@@ -357,12 +358,41 @@ __device__ inline void cell_derive(CellV<R>& c, R hextra)
 // every solve and the order of the rhs accumulation are those of the functors, so the
 // results are those of the per-cell form.  No LDS and no barriers.
 constexpr int MW = 62;            // strip columns (lanes 1..62)
-constexpr int MR = 32;            // strip rows
 constexpr int MWAVES = BT / 64;   // strips per block
 
+// Rows of a strip.  A strip solves its top edge row twice over (once per neighbour), so long
+// strips waste least, but a wave marches its rows one after the other: a grid cut into
+// fewer strips than the chip has SIMDs runs at the latency of one strip however small it is
+// (785 x 785 in FP64: 325 strips of 32 rows, 130 us a step, against 47 with 5 rows).  The
+// blocks of a launch share the CUs, so a step takes about
+//     max(blocks per CU, rounded up, L) * (rows + E)
+// rows' time of a busy SIMD: E is the repeated work of a strip in rows (0.9 FP64, 1.2 FP32:
+// 4096 x 4096 in strips of 4, 8, 16 rows: 861, 776, 744 us; an FP32 ensemble of 8, 16, 32:
+// 813, 749, 734), and a wave alone on its SIMD takes L times a busy one's share of time per
+// row (FP64 3.9 against 2.7 us, FP32 2.4 against 1.0, both kernels of a step).  The choice is
+// the minimum over the lengths below; every value of the fields is the same for all of them.
 template <typename R>
-__global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ sc, int nscen, int nstrips, int par,
-                                                   Params P)
+int strip_rows(int num_cu, int nscen, const int* nx, const int* ny)
+{
+    const double L = sizeof(R) == 8 ? 1.46 : 2.4, E = sizeof(R) == 8 ? 0.9 : 1.2;
+    int best = 32;
+    double least = 0.0;
+    for (int mr : {32, 28, 24, 20, 16, 14, 12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
+        double strips = 0.0;
+        for (int s = 0; s < nscen; s++) strips += (double)ceil_div(nx[s], MW) * ceil_div(ny[s], mr);
+        const double per_cu = std::ceil(std::ceil(strips / MWAVES) / (num_cu > 0 ? num_cu : 1));
+        const double cost = (per_cu > L ? per_cu : L) * (mr + E);
+        if (least == 0.0 || cost < least) {
+            least = cost;
+            best = mr;
+        }
+    }
+    return best;
+}
+
+template <typename R>
+__global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ sc, int nscen, int nstrips, int mr,
+                                                   int par, Params P)
 {
     const int lane = threadIdx.x & 63;
     const int strip = blockIdx.x * MWAVES + (threadIdx.x >> 6);  // uniform per wave
@@ -375,7 +405,7 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
     const int nx = S.nx, ny = S.ny;
     const size_t W = (size_t)nx + 2;
     const int col = tx * MW + lane;  // padded column of this lane
-    const int j0 = ty * MR + 1;
+    const int j0 = ty * mr + 1;
     const bool colmem = col <= nx + 1;
     const bool cell = lane >= 1 && lane <= MW && col <= nx;
     const bool xedge = lane >= 1 && colmem;  // edge (col-1, col) with col-1 <= nx
@@ -391,7 +421,7 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
     const R dt = (R)S.st->dt;
     const R dx = (R)P.dx, hextra = (R)P.hextra, rain = (R)P.rain;
     const R G = (R)9.81, EPS12 = (R)1e-12;
-    const int rend = min(MR, ny + 1 - j0);  // last row offset: rows up to ny+1 exist
+    const int rend = min(mr, ny + 1 - j0);  // last row offset: rows up to ny+1 exist
     const RhsScale<R> scale(dt, dx);
 
     CellV<R> prev, cur, nxt;
@@ -401,13 +431,17 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
     cell_derive(prev, hextra);
     // rhs*0 / rhs*1 of the previous row's cell (h, qx, qy)
     R p0[3] = {(R)0, (R)0, (R)0}, p1[3] = {(R)0, (R)0, (R)0};
+    // Not unrolled and no iteration peeled: a strip's first row would get a copy of the solves
+    // in which the FP32 form's multiply-adds contract differently, and an edge between two
+    // strips would be solved to other bits by each of them.
+#pragma clang loop unroll(disable)
     for (int r = 0; r <= rend; r++) {
         const int j = j0 + r;
         // prefetch row j+1 while row j is solved
         cell_load(nxt, h, qx, qy, z, n2, colc + W * (size_t)min(j + 1, ny + 1));  // unused at r == rend
         cell_derive(cur, hextra);
         R c0[3] = {(R)0, (R)0, (R)0}, c1[3] = {(R)0, (R)0, (R)0};
-        if (r < MR) {  // uniform: row j is a strip row
+        if (r < mr) {  // uniform: row j is a strip row
             CellV<R> L;
             L.h = lane_shift<true>(cur.h);
             L.qx = lane_shift<true>(cur.qx);
@@ -571,8 +605,8 @@ __device__ inline void wave_min_sum(R& m, double& s, double& c)
 // partial per strip, partials[3t .. 3t+2] = (min, sum, compensation).  No LDS and no
 // barriers.  MODE 0: initial CFL only (no fix); MODE 1: end of a step.
 template <typename R, int MODE>
-__global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc, int nscen, int nstrips, int par,
-                                                  Params P)
+__global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc, int nscen, int nstrips, int mr,
+                                                  int par, Params P)
 {
     const int lane = threadIdx.x & 63;
     const int strip = blockIdx.x * MWAVES + (threadIdx.x >> 6);  // uniform per wave
@@ -585,10 +619,10 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
     const int nx = S.nx, ny = S.ny;
     const size_t W = (size_t)nx + 2;
     const int col = tx * MW + lane;  // padded column of this lane
-    const int j0 = ty * MR + 1;
+    const int j0 = ty * mr + 1;
     const bool colmem = col <= nx + 1;
     const bool cell = lane >= 1 && lane <= MW && col <= nx;
-    const int nr = min(MR, ny + 1 - j0);  // cell rows of the strip (j0 <= ny)
+    const int nr = min(mr, ny + 1 - j0);  // cell rows of the strip (j0 <= ny)
     const gmem<R>* h = to_global((const R*)S.h[par]);
     gmem<R>* qx = to_global(S.qx[par]);
     gmem<R>* qy = to_global(S.qy[par]);
@@ -754,13 +788,14 @@ int run_flood(appfis_ctx* ctx, int nscen, const int* nx, const int* ny, void* co
     }
     APPFIS_REQUIRE(prm->dx > 0.0, "dx must be positive");
     // strip work-list
+    const int mr = strip_rows<R>(ctx->num_cu, nscen, nx, ny);
     std::vector<Scen<R>> hs((size_t)nscen);
     long long total_strips = 0;
     size_t field_bytes = 0;
     for (int s = 0; s < nscen; s++) {
         hs[s].nx = nx[s];
         hs[s].ny = ny[s];
-        const int sx = (int)ceil_div(nx[s], MW), sy = (int)ceil_div(ny[s], MR);
+        const int sx = (int)ceil_div(nx[s], MW), sy = (int)ceil_div(ny[s], mr);
         hs[s].strips_x = sx;
         hs[s].strip0 = (int)total_strips;
         hs[s].nstrips = sx * sy;
@@ -861,18 +896,18 @@ int run_flood(appfis_ctx* ctx, int nscen, const int* nx, const int* ny, void* co
     const dim3 grid((unsigned)ceil_div(total_strips, MWAVES));  // MWAVES strips per block
     const int nstrips = (int)total_strips;
     // dt of the first step from the initial state
-    hipLaunchKernelGGL((k_fix_march<R, 0>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, 0, P);
+    hipLaunchKernelGGL((k_fix_march<R, 0>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, 0, P);
     APPFIS_LAUNCH_CHECK();
     hipLaunchKernelGGL((k_finalize<R, 0>), dim3(nscen), dim3(BT), 0, ctx->stream, tab, P);
     APPFIS_LAUNCH_CHECK();
     auto step_pair = [&](int par) -> int {
-        hipLaunchKernelGGL((k_flux_march<R>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, par, P);
+        hipLaunchKernelGGL((k_flux_march<R>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, par, P);
         APPFIS_LAUNCH_CHECK();
         if (nsrc > 0) {
             hipLaunchKernelGGL((k_sources<R>), dim3(nscen), dim3(64), 0, ctx->stream, tab, par ^ 1, P);
             APPFIS_LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL((k_fix_march<R, 1>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, par ^ 1, P);
+        hipLaunchKernelGGL((k_fix_march<R, 1>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, par ^ 1, P);
         APPFIS_LAUNCH_CHECK();
         hipLaunchKernelGGL((k_finalize<R, 1>), dim3(nscen), dim3(BT), 0, ctx->stream, tab, P);
         APPFIS_LAUNCH_CHECK();
@@ -887,6 +922,7 @@ int run_flood(appfis_ctx* ctx, int nscen, const int* nx, const int* ny, void* co
                                            key_ptr(tab),
                                            (uint64_t)nscen,
                                            (uint64_t)nstrips,
+                                           (uint64_t)mr,
                                            (uint64_t)(nsrc > 0),
                                            key_bits(P.dx),
                                            key_bits(P.cn),

@@ -72,6 +72,20 @@ def test_flood_f64_frictionless_bit_exact(ctx, n, wet, steps):
     assert np.allclose(vg, vc, rtol=1e-13, atol=0)
 
 
+@pytest.mark.parametrize("n", [1, 2, 61, 62, 63, 125, 311, 500])
+def test_flood_strip_heights_bit_exact(ctx, n):
+    # the strips' height follows the grid (1 row up to 5 at these sizes): one cell, strips one
+    # column short of, equal to and one past their width, and last strips with fewer rows
+    arrs = scenario(n, 3200 + n, wet=0.1)
+    arrs[4][:] = 0.0
+    g, tg, vg = gpu_run(ctx, arrs, 7)
+    c, tc, vc = cpu_run(arrs, 7)
+    for a, b in zip(g, c):
+        assert np.array_equal(a, b)
+    assert np.array_equal(tg, tc)
+    assert np.allclose(vg, vc, rtol=1e-13, atol=0)
+
+
 @pytest.mark.parametrize("n,wet,steps", [(64, 0.0, 80), (90, 0.3, 50)])
 def test_flood_f64_with_friction(ctx, n, wet, steps):
     arrs = scenario(n, 3100 + n, wet=wet)
