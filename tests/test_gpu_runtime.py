@@ -119,6 +119,31 @@ def test_reduce_matches_oracle(ctx, dt):
             assert abs(w - exact) <= 4 * np.spacing(abs(exact))
 
 
+@pytest.mark.parametrize("dt", [hip.U8, hip.I32, hip.F32, hip.F64])
+@pytest.mark.parametrize("n0", [1, 3, 4, 15, 16, 17, 63, 64, 65, 257, 1023, 1025, 2100, 16387])
+def test_reduce_row_lengths(ctx, dt, n0):
+    # rows shorter than, equal to and longer than one 16-byte load, rows of part of a wave's step,
+    # of one step and of several, starting at an odd element, over one plane and over several,
+    # in one block and in many (16387 x 7 x 60 exceeds the larger blocks' threshold for F64)
+    rng = np.random.default_rng(n0)
+    for n1, n2 in ((1, 1), (5, 3), (7, 60)):
+        shape = (n2 + 2, n1 + 1, n0 + 4)
+        np_dt = hip.NP_DTYPE[dt]
+        a = rng.integers(0, 200, shape).astype(np_dt) if dt in (hip.U8, hip.I32) else rng.random(shape).astype(np_dt) + 1
+        a[:, :, :3] = a[:, :, n0 + 3:] = 250  # outside the box, and above all of it
+        box = [3, n0 + 3, 1, n1 + 1, 1, n2 + 1]
+        part = a[1:n2 + 1, 1:n1 + 1, 3:n0 + 3]
+        d = ctx.from_numpy(a, dt)
+        assert ctx.reduce(d, box, hip.MAX) == part.max()
+        assert ctx.reduce(d, box, hip.MIN) == part.min()
+        total = ctx.reduce_sum_wide(d, box)
+        if dt in (hip.U8, hip.I32):
+            assert total == part.sum(dtype=np.int64)
+        else:  # a compensated sum: within an ulp of the exact one, and the final addition's rounding
+            exact = math.fsum(part.ravel().astype(np.float64))
+            assert abs(total - exact) <= 2 * np.spacing(exact)
+
+
 def test_reduce_max_quirk_and_large(ctx):
     a = -np.ones((64, 64), dtype=np.float32)
     d = ctx.from_numpy(a)
