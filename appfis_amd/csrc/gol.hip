@@ -15,8 +15,8 @@
 //   value new(xw, yw), recomputed from the current buffer whose ring is valid, so the
 //   written buffer leaves with its ring already exchanged: no second launch.
 //
-// CHOSEN: gol_bits.hip (bit-packed copy of the field, 32 cells per word) when nx % 32 == 0,
-//   this byte kernel otherwise.
+// CHOSEN: gol_bits.hip (bit-packed copy of the field, 32 cells per word) from 32 cells a row on,
+//   this byte kernel below.
 #include "common.hpp"
 
 using namespace appfis;
@@ -210,6 +210,8 @@ typedef void (*gol_kernel_t)(const uint8_t*, uint8_t*, int, int, int, int, RowDi
 
 }  // namespace gol
 
+// whether the context's workspace holds the packed board, growing it where it can
+bool gol_bits_workspace(appfis_ctx* ctx, int nx, int ny);
 int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int gens, int force);
 
 extern "C" int appfis_gol(appfis_ctx* ctx, uint8_t* buf0, uint8_t* buf1, int nx, int ny, int gens, int variant,
@@ -226,9 +228,11 @@ extern "C" int appfis_gol(appfis_ctx* ctx, uint8_t* buf0, uint8_t* buf1, int nx,
     APPFIS_REQUIRE(variant >= 0, "gol: unknown variant %d", variant);
     if (variant >= APPFIS_CANDIDATE0)  // a forced blocked candidate of the bit-packed form
         return gol_bits_run(ctx, buf0, buf1, nx, ny, gens, variant - APPFIS_CANDIDATE0);
-    // the bit-packed form needs the periodic wrap on word boundaries; other widths run
-    // the byte kernel, which gives the same bytes
-    if (variant == APPFIS_CHOSEN && nx % 32 == 0) return gol_bits_run(ctx, buf0, buf1, nx, ny, gens, -1);
+    // the bit-packed form needs a word of cells; narrower boards run the byte kernel, which
+    // gives the same bytes, and so do boards whose width is no multiple of 32 where there is
+    // no workspace (a first call while the stream is being captured)
+    if (variant == APPFIS_CHOSEN && nx >= 32 && (nx % 32 == 0 || gol_bits_workspace(ctx, nx, ny)))
+        return gol_bits_run(ctx, buf0, buf1, nx, ny, gens, -1);
     const int W = nx + 2, H = ny + 2;
     const int nbytes = W * H;
     const int nchunks = (nbytes + gol::CHUNK - 1) / gol::CHUNK;

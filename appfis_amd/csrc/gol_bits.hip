@@ -3,10 +3,11 @@
 // The call packs the interior of the uint8 field into 32-bit words (bit b of word w of
 // row y = cell (32w + b, y), interior coordinates), advances the packed field (many
 // generations per launch), and its last launch computes the last generation while
-// unpacking the last two back into the two uint8 buffers, rings exchanged: on return both buffers hold exactly what the PLAIN form
-// leaves (generation `gens` in buf[gens % 2], generation gens-1 in the other).  The
-// packed layout needs nx % 32 == 0 so that the periodic wrap falls on word boundaries;
-// appfis_gol runs the byte kernel for other widths.  Cells must hold 0 or 1.
+// unpacking the last two back into the two uint8 buffers, rings exchanged: on return both
+// buffers hold exactly what the PLAIN form leaves (generation `gens` in buf[gens % 2],
+// generation gens-1 in the other).  A row takes ceil(nx / 32) words; where nx is no multiple
+// of 32 the rest of its last word means nothing, and the kernels join the row's end and start
+// by shifting.  Cells must hold 0 or 1.
 //
 // One generation, per word, with 32 cells evaluated at once by bitwise full adders:
 //   h(row)  = W + C + E                (2-bit horizontal sum of each row; W/E are the
@@ -17,6 +18,9 @@
 // A thread owns one word column over K consecutive rows, so each row's horizontal sum
 // is computed once and used by the three output rows that need it.
 #include "common.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 using namespace appfis;
 
@@ -72,62 +76,28 @@ __global__ __launch_bounds__(256) void k_pack(const uint8_t* __restrict__ u, uin
     P[t] = word;
 }
 
-template <int K>
-__global__ __launch_bounds__(256) void k_step(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q, int NW, int ny,
-                                              unsigned nitems)
-{
-    // consecutive blocks share rows at their band edges: keep them on one XCD
-    const unsigned t = xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-    if (t >= nitems) return;
-    const int band = (int)(t / (unsigned)NW), w = (int)(t - (unsigned)band * NW);
-    const int wl = w == 0 ? NW - 1 : w - 1;
-    const int wr = w == NW - 1 ? 0 : w + 1;
-    const int y0 = band * K;
-    uint32_t h0[K + 2], h1[K + 2], cen[K + 2];
-#pragma unroll
-    for (int r = 0; r < K + 2; r++) {
-        int y = y0 - 1 + r;  // periodic rows; y < ny + K, so the loop ends (once if K <= ny)
-        if (y < 0) y += ny;
-        while (y >= ny) y -= ny;
-        const uint32_t* row = P + (size_t)y * NW;
-        const uint32_t c = row[w], l = row[wl], rr = row[wr];
-        const uint32_t W = __builtin_amdgcn_alignbit(c, l, 31);  // cell x-1 at bit x
-        const uint32_t E = __builtin_amdgcn_alignbit(rr, c, 1);  // cell x+1 at bit x
-        h0[r] = xor3(W, c, E);
-        h1[r] = maj(W, c, E);
-        cen[r] = c;
-    }
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int y = y0 + k;
-        if (y >= ny) break;
-        // S = h[k] + h[k+1] + h[k+2] through the carry-save adders of the two bit-planes
-        const uint32_t s0 = xor3(h0[k], h0[k + 1], h0[k + 2]);
-        const uint32_t c0 = maj(h0[k], h0[k + 1], h0[k + 2]);
-        const uint32_t u1 = xor3(h1[k], h1[k + 1], h1[k + 2]);
-        const uint32_t c1 = maj(h1[k], h1[k + 1], h1[k + 2]);
-        Q[(size_t)y * NW + w] = life_rule(s0, c0, u1, c1, cen[k + 1]);
-    }
-}
-
 constexpr int KROWS = 8;
 
-// One padded uint8 row from a packed word: the 32 cells of word w, and the ring cell
-// that the periodic exchange (X first) copies from it -- ghost column nx+1 holds cell 0,
-// ghost column 0 holds cell nx-1.
-__device__ __forceinline__ void put_word(uint8_t* __restrict__ u, size_t W, int prow, int w, int NW, uint32_t word)
+// 32 cells from cell x on of one padded uint8 row (bit b of word = cell x + b), and the ring
+// cells that the periodic exchange (X first) copies from the row: ghost column nx+1 holds
+// cell 0, ghost column 0 holds cell nx-1.
+__device__ __forceinline__ void put_word(uint8_t* __restrict__ u, size_t W, int prow, int x, bool first, bool last,
+                                         uint32_t word)
 {
     uint8_t* row = u + (size_t)prow * W;
 #pragma unroll
-    for (int b = 0; b < 32; b++) row[1 + 32 * w + b] = (uint8_t)((word >> b) & 1u);
-    if (w == 0) row[W - 1] = (uint8_t)(word & 1u);
-    if (w == NW - 1) row[0] = (uint8_t)(word >> 31);
+    for (int b = 0; b < 32; b++) row[1 + x + b] = (uint8_t)((word >> b) & 1u);
+    if (first) row[W - 1] = (uint8_t)(word & 1u);
+    if (last) row[0] = (uint8_t)(word >> 31);
 }
 
 // The last generation of a call fused with the unpacking: from the packed generation
-// n-1 in P it computes generation n (as k_step does) and writes generation n into `un`
-// and generation n-1 into `uprev`, both with their periodic rings -- what one k_step,
-// unpacking both generations and exchanging both rings would leave, in one pass.  The exchange's Y step copies
+// n-1 in P it computes generation n and writes generation n into `un`
+// and generation n-1 into `uprev`, both with their periodic rings -- what one generation,
+// unpacking both generations and exchanging both rings would leave, in one pass.  Where nx is
+// no multiple of 32 the thread of the last word takes the row's last 32 cells, which overlap
+// the word before it (both write the same bytes there), so that every thread moves whole
+// words.  The exchange's Y step copies
 // padded row ny (ghost columns included) into ghost row 0 and padded row 1 into ghost
 // row ny+1, so the thread of interior row ny-1 also writes row 0 and that of row 0 also
 // writes row ny+1.  Reads only P: `uprev` may be the buffer the call's input came from.
@@ -143,16 +113,23 @@ __global__ __launch_bounds__(256) void k_step_unpack(const uint32_t* __restrict_
     const int wr = w == NW - 1 ? 0 : w + 1;
     const int y0 = band * K;
     const size_t W = (size_t)nx + 2;
+    const unsigned rem = (unsigned)nx & 31u;  // cells of the last word, 0: all 32
+    const bool first = w == 0, last = w == NW - 1, end = last && rem != 0;
+    const int x = end ? nx - 32 : 32 * w;     // first cell of this thread's 32
     uint32_t h0[K + 2], h1[K + 2], cen[K + 2];
 #pragma unroll
     for (int r = 0; r < K + 2; r++) {
-        int y = y0 - 1 + r;
+        int y = y0 - 1 + r;  // periodic rows; y < ny + K, so the loop ends (once if K <= ny)
         if (y < 0) y += ny;
         while (y >= ny) y -= ny;
         const uint32_t* row = P + (size_t)y * NW;
-        const uint32_t c = row[w], l = row[wl], rr = row[wr];
-        const uint32_t Wc = __builtin_amdgcn_alignbit(c, l, 31);
-        const uint32_t Ec = __builtin_amdgcn_alignbit(rr, c, 1);
+        const uint32_t cw = row[w], lw = row[wl], rr = row[wr];
+        const uint32_t c = end ? __builtin_amdgcn_alignbit(cw, lw, rem) : cw;
+        // bit 31 of l is the cell left of the 32: cell nx-1 for the first word, and the last
+        // cell but 32 of a row whose last word is not full
+        const uint32_t l = (first || end) && rem != 0 ? lw << (32u - rem) : lw;
+        const uint32_t Wc = __builtin_amdgcn_alignbit(c, l, 31);   // cell x-1 at bit x
+        const uint32_t Ec = __builtin_amdgcn_alignbit(rr, c, 1);   // cell x+1 at bit x
         h0[r] = xor3(Wc, c, Ec);
         h1[r] = maj(Wc, c, Ec);
         cen[r] = c;
@@ -166,15 +143,15 @@ __global__ __launch_bounds__(256) void k_step_unpack(const uint32_t* __restrict_
         const uint32_t u1 = xor3(h1[k], h1[k + 1], h1[k + 2]);
         const uint32_t c1 = maj(h1[k], h1[k + 1], h1[k + 2]);
         const uint32_t next = life_rule(s0, c0, u1, c1, cen[k + 1]);
-        put_word(un, W, y + 1, w, NW, next);
-        put_word(uprev, W, y + 1, w, NW, cen[k + 1]);
+        put_word(un, W, y + 1, x, first, last, next);
+        put_word(uprev, W, y + 1, x, first, last, cen[k + 1]);
         if (y == ny - 1) {
-            put_word(un, W, 0, w, NW, next);
-            put_word(uprev, W, 0, w, NW, cen[k + 1]);
+            put_word(un, W, 0, x, first, last, next);
+            put_word(uprev, W, 0, x, first, last, cen[k + 1]);
         }
         if (y == 0) {
-            put_word(un, W, ny + 1, w, NW, next);
-            put_word(uprev, W, ny + 1, w, NW, cen[k + 1]);
+            put_word(un, W, ny + 1, x, first, last, next);
+            put_word(uprev, W, ny + 1, x, first, last, cen[k + 1]);
         }
     }
 }
@@ -192,6 +169,8 @@ __global__ __launch_bounds__(256) void k_step_unpack(const uint32_t* __restrict_
 //      barrier
 //   C  vertical combine: the sums of the rows above / below the wave's band come from
 //      the waves above / below (zero outside the window), then the rule.
+// Never chosen any more (48 generations at 16384 x 16384: 441 us, windows 171; at 2048 x 2048
+// 107, windows 24); kept as a forced candidate, the form that spreads a row over waves.
 template <int K, int G, int NWAVES>
 __global__ __launch_bounds__(64 * NWAVES) void k_step_tb(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q,
                                                           int NW, int ny, int WX, int OUT, int gens)
@@ -293,106 +272,6 @@ __global__ __launch_bounds__(64 * NWAVES) void k_step_tb(const uint32_t* __restr
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int r = wy * K + k - G;  // output row within the block's OUT rows
-        const int y = ybase + k;
-        if (r >= 0 && r < OUT && y < ny) Q[y * NW + w] = R[k];
-    }
-}
-
-// One barrier per generation.  Each wave publishes its raw edge words (lanes 0 / 63,
-// all K rows) and its first and last rows into the LDS buffers of the generation's
-// parity; after the barrier every wave computes the horizontal sums of its K rows and
-// of the two rows next to its band (those of the waves above / below, with their edge
-// words) itself.  The buffers alternate by generation, so a wave still reading
-// generation g's buffers is never overwritten: the next writes to them come after the
-// barrier of generation g+1, which every wave reaches only after finishing g.
-template <int K, int G, int NWAVES>
-__global__ __launch_bounds__(64 * NWAVES) void k_step_tb1(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q,
-                                                           int NW, int ny, int WX, int OUT, int gens)
-{
-    __shared__ uint32_t edge_lo[2][NWAVES][K], edge_hi[2][NWAVES][K];  // lane-0 / lane-63 words
-    __shared__ uint32_t row_top[2][NWAVES][64], row_bot[2][NWAVES][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int wx = wv % WX, wy = wv / WX;
-    const int WY = NWAVES / WX;
-    const int w = wx * 64 + lane;
-    const int left = wy * WX + (wx == 0 ? WX - 1 : wx - 1);
-    const int right = wy * WX + (wx == WX - 1 ? 0 : wx + 1);
-    const int band = (int)xcd_tile(blockIdx.x, gridDim.x);  // XCD-contiguous band order
-    const int y0 = band * OUT - G + wy * K;
-    int yw = y0 % ny;
-    if (yw < 0) yw += ny;
-    uint32_t R[K];
-    if (K <= ny) {
-        int y = yw, off = yw * NW + w;
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            R[k] = P[off];
-            ++y;
-            off += NW;
-            if (y == ny) {
-                y = 0;
-                off = w;
-            }
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            int y = yw + k;
-            while (y >= ny) y -= ny;
-            R[k] = P[y * NW + w];
-        }
-    }
-    for (int g = 0; g < gens; g++) {
-        const int b = g & 1;
-        if (lane == 0)
-#pragma unroll
-            for (int k = 0; k < K; k++) edge_lo[b][wv][k] = R[k];
-        if (lane == 63)
-#pragma unroll
-            for (int k = 0; k < K; k++) edge_hi[b][wv][k] = R[k];
-        row_top[b][wv][lane] = R[0];
-        row_bot[b][wv][lane] = R[K - 1];
-        __syncthreads();
-        // horizontal sums of rows -1 .. K (rows -1 / K: the neighbouring waves' band
-        // edges, zero outside the window)
-        uint32_t h0[K + 2], h1[K + 2];
-        auto hsum = [&](uint32_t c, uint32_t lo_edge, uint32_t hi_edge, uint32_t& s0, uint32_t& s1) {
-            const uint32_t l = (uint32_t)__builtin_amdgcn_update_dpp((int)lo_edge, (int)c, 0x138, 0xF, 0xF, false);
-            const uint32_t r = (uint32_t)__builtin_amdgcn_update_dpp((int)hi_edge, (int)c, 0x130, 0xF, 0xF, false);
-            const uint32_t Wc = __builtin_amdgcn_alignbit(c, l, 31);
-            const uint32_t Ec = __builtin_amdgcn_alignbit(r, c, 1);
-            s0 = xor3(Wc, c, Ec);
-            s1 = maj(Wc, c, Ec);
-        };
-#pragma unroll
-        for (int k = 0; k < K; k++) hsum(R[k], edge_hi[b][left][k], edge_lo[b][right][k], h0[k + 1], h1[k + 1]);
-        if (wy > 0) {
-            hsum(row_bot[b][wv - WX][lane], edge_hi[b][left - WX][K - 1], edge_lo[b][right - WX][K - 1], h0[0],
-                 h1[0]);
-        } else {
-            h0[0] = 0u;
-            h1[0] = 0u;
-        }
-        if (wy < WY - 1) {
-            hsum(row_top[b][wv + WX][lane], edge_hi[b][left + WX][0], edge_lo[b][right + WX][0], h0[K + 1],
-                 h1[K + 1]);
-        } else {
-            h0[K + 1] = 0u;
-            h1[K + 1] = 0u;
-        }
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            const uint32_t s0 = xor3(h0[k], h0[k + 1], h0[k + 2]);
-            const uint32_t c0 = maj(h0[k], h0[k + 1], h0[k + 2]);
-            const uint32_t v1 = xor3(h1[k], h1[k + 1], h1[k + 2]);
-            const uint32_t c1 = maj(h1[k], h1[k + 1], h1[k + 2]);
-            R[k] = life_rule(s0, c0, v1, c1, R[k]);
-        }
-    }
-    const int ybase = band * OUT - G + wy * K;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int r = wy * K + k - G;
         const int y = ybase + k;
         if (r >= 0 && r < OUT && y < ny) Q[y * NW + w] = R[k];
     }
@@ -506,11 +385,10 @@ __device__ __forceinline__ void tw_generations(uint32_t (&R)[K][WPL], uint32_t (
 
 template <int WPL, int K, int G, int NWAVES>
 __global__ __launch_bounds__(64 * NWAVES) void k_step_tw(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q,
-                                                          int NW, int ny, int WX, int OUT, int gens)
+                                                          int NW, int ny, int OUT, int gens)
 {
     using VW = WordVec<WPL>;
     using V = typename VW::V;
-    (void)WX;
     // [parity][wave][first / last row][bit-plane][word of the row]
     __shared__ uint32_t hs[2][NWAVES][2][2][64 * WPL];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -636,32 +514,107 @@ __global__ __launch_bounds__(64 * NWAVES) void k_step_tw_io(const uint8_t* __res
     }
 }
 
-typedef void (*tw_io_kernel)(const uint8_t*, const uint32_t*, uint32_t*, uint8_t*, uint8_t*, int, int, int, int);
-struct TbVariant {
+// The blocked form for rows of any width nx >= 32 (NW = ceil(nx / 32) words; bits past cell
+// nx-1 of a row's last word mean nothing).  A wave's K rows span a window of 64*WPL words of
+// which all but the first and the last are stored: G <= 32 generations spoil at most the 32
+// cells of a word at either end, so the wrap of tw_generations' rotation does no harm.  Tile
+// (tx, band) stores words tx*(64*WPL - 2) .. and OUT = NWAVES*K - 2G rows.  The window is
+// periodic in cells, not in words: window word g holds cells 32g .. 32g+31 modulo nx, so where
+// the row's end falls inside a word the fetch joins the cells before it and those from cell 0.
+template <int WPL, int K, int G, int NWAVES>
+__global__ __launch_bounds__(64 * NWAVES) void k_step_win(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q,
+                                                          int nx, int NW, int ny, int tiles_x, int gens)
+{
+    constexpr int OUTW = 64 * WPL - 2, OUT = NWAVES * K - 2 * G;
+    static_assert(G <= 32 && OUT > 0, "a halo of one word and of G rows");
+    __shared__ uint32_t hs[2][NWAVES][2][2][64 * WPL];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int t = (int)xcd_tile(blockIdx.x, gridDim.x);  // x fastest: neighbouring tiles share an L2
+    const int band = t / tiles_x, tx = t - band * tiles_x;
+    const int g0 = tx * OUTW - 1 + WPL * lane;  // word of R[.][0]
+    int yw = (band * OUT - G + wv * K) % ny;
+    if (yw < 0) yw += ny;
+    uint32_t R[K][WPL], Rp[K][WPL];
+    const bool whole = tx > 0 && 32LL * (tx * OUTW + OUTW + 1) <= nx;  // every word a stored one, and full
+    if (whole) {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            int y = yw + k;  // periodic rows (the window may wrap more than once when ny < K)
+            while (y >= ny) y -= ny;
+            const uint32_t* row = P + (size_t)y * NW;
+#pragma unroll
+            for (int w = 0; w < WPL; w++) R[k][w] = row[g0 + w];
+        }
+    } else {
+        // word g: cells s .. of the row (s = 32g modulo nx) down from bit s & 31 of word ia, `low`
+        // of them before the row's end, then cells from 0 on.  Words past the one right of the
+        // row's last are not used and hold its first.
+        int ia[WPL], ib[WPL];
+        unsigned sh[WPL], low[WPL];
+#pragma unroll
+        for (int w = 0; w < WPL; w++) {
+            const int g = g0 + w;
+            int sc = g < 0 ? nx - 32 : g > NW ? 0 : 32 * g;
+            if (sc >= nx) sc -= nx;
+            ia[w] = sc >> 5;
+            ib[w] = ia[w] + 1 < NW ? ia[w] + 1 : ia[w];
+            sh[w] = (unsigned)sc & 31u;
+            low[w] = (unsigned)(nx - sc < 32 ? nx - sc : 32);
+        }
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            int y = yw + k;
+            while (y >= ny) y -= ny;
+            const uint32_t* row = P + (size_t)y * NW;
+            const uint32_t head = row[0];
+#pragma unroll
+            for (int w = 0; w < WPL; w++) {
+                const uint32_t v = __builtin_amdgcn_alignbit(row[ib[w]], row[ia[w]], sh[w]);
+                R[k][w] = low[w] == 32u ? v : (v & ((1u << low[w]) - 1u)) | (head << low[w]);
+            }
+        }
+    }
+    tw_generations<WPL, K, G, NWAVES, false>(R, Rp, hs, lane, wv, gens);
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int r = wv * K + k - G, y = band * OUT + r;  // output row of the block, of the field
+        if (r < 0 || r >= OUT || y >= ny) continue;
+        uint32_t* row = Q + (size_t)y * NW;
+#pragma unroll
+        for (int w = 0; w < WPL; w++) {
+            const int lw = WPL * lane + w;
+            if (lw >= 1 && lw <= OUTW && g0 + w < NW) row[g0 + w] = R[k][w];
+        }
+    }
+}
+
+// Window variants.  Few rows a wave make a generation short (about 0.07 + 0.08 K us for a block
+// alone on its CU, whose waves meet at a barrier each generation), many make the 2G rows that
+// a block repeats cheap, and G spreads the 4.5 us that a launch costs.
+struct WinVariant {
     const char* name;
     void (*kernel)(const uint32_t*, uint32_t*, int, int, int, int, int);
     int k, g, nwaves;
-    int wpl;  // full-row form: words per lane (the wave spans the row); 0: WX waves per row
-    // full-row form: the first launch of a call reading the uint8 field, and the last one
-    // writing both uint8 buffers (k_step_tw_io); null for the other forms
-    tw_io_kernel kin = nullptr, kout = nullptr;
+};
+#define WIN(K, G, NWAVES) {"win k" #K " g" #G " w" #NWAVES, k_step_win<1, K, G, NWAVES>, K, G, NWAVES}
+static const WinVariant kWin[] = {WIN(4, 24, 16), WIN(6, 24, 16), WIN(6, 16, 16), WIN(8, 24, 16), WIN(8, 16, 16),
+                                  WIN(12, 16, 16)};
+constexpr int WIN_WORDS = 62;  // words of a row that a window stores
+constexpr int TB_K = 10, TB_G = 4, TB_WAVES = 16;  // "tb k10 g4 w16"
+
+typedef void (*tw_io_kernel)(const uint8_t*, const uint32_t*, uint32_t*, uint8_t*, uint8_t*, int, int, int, int);
+struct TwVariant {
+    const char* name;
+    void (*kernel)(const uint32_t*, uint32_t*, int, int, int, int);
+    int k, g, nwaves, wpl;  // wpl: words per lane; a wave spans a row of 64 * wpl words
+    // the first launch of a call reading the uint8 field, and the last one writing both
+    // uint8 buffers (k_step_tw_io)
+    tw_io_kernel kin, kout;
 };
 #define TW_IO(WPL, K, G, NWAVES) k_step_tw_io<WPL, K, G, NWAVES, true, false>, k_step_tw_io<WPL, K, G, NWAVES, false, true>
 
-static const TbVariant kTb[] = {
-    {"tb k16 g8 w16", k_step_tb<16, 8, 16>, 16, 8, 16, 0}, {"tb k10 g4 w16", k_step_tb<10, 4, 16>, 10, 4, 16, 0},
-    {"tb k20 g4 w8", k_step_tb<20, 4, 8>, 20, 4, 8, 0},    {"tb k12 g4 w8", k_step_tb<12, 4, 8>, 12, 4, 8, 0},
-    {"tb k24 g8 w16", k_step_tb<24, 8, 16>, 24, 8, 16, 0}, {"tb k8 g4 w16", k_step_tb<8, 4, 16>, 8, 4, 16, 0},
-    {"tb k12 g4 w16", k_step_tb<12, 4, 16>, 12, 4, 16, 0}, {"tb k32 g8 w8", k_step_tb<32, 8, 8>, 32, 8, 8, 0},
-    {"tb k16 g4 w8", k_step_tb<16, 4, 8>, 16, 4, 8, 0},    {"tb k11 g5 w16", k_step_tb<11, 5, 16>, 11, 5, 16, 0},
-    {"tb k13 g6 w16", k_step_tb<13, 6, 16>, 13, 6, 16, 0},
-    {"tb1 k10 g4 w16", k_step_tb1<10, 4, 16>, 10, 4, 16, 0}, {"tb1 k11 g5 w16", k_step_tb1<11, 5, 16>, 11, 5, 16, 0},
-    {"tb1 k13 g6 w16", k_step_tb1<13, 6, 16>, 13, 6, 16, 0}, {"tb1 k16 g8 w16", k_step_tb1<16, 8, 16>, 16, 8, 16, 0},
-    {"tb1 k20 g4 w8", k_step_tb1<20, 4, 8>, 20, 4, 8, 0},    {"tb1 k12 g4 w16", k_step_tb1<12, 4, 16>, 12, 4, 16, 0},
-    // 4K - 2G = 32 output rows per block like k10 g4 (256 blocks fill 256 CUs at 8192
-    // rows), with more generations per launch to spread the launch's fixed load / store
-    {"tb1 k11 g6 w16", k_step_tb1<11, 6, 16>, 11, 6, 16, 0}, {"tb1 k12 g8 w16", k_step_tb1<12, 8, 16>, 12, 8, 16, 0},
-    // full-row waves (nx = 2048 * WPL), also 32 output rows per block at 8192 rows
+static const TwVariant kTw[] = {
+    // 32 output rows per block: 256 blocks fill 256 CUs at 8192 rows
     {"tw4 k3 g8 w16", k_step_tw<4, 3, 8, 16>, 3, 8, 16, 4, TW_IO(4, 3, 8, 16)},
     {"tw4 k4 g8 w12", k_step_tw<4, 4, 8, 12>, 4, 8, 12, 4, TW_IO(4, 4, 8, 12)},
     {"tw2 k3 g8 w16", k_step_tw<2, 3, 8, 16>, 3, 8, 16, 2, TW_IO(2, 3, 8, 16)},
@@ -672,45 +625,82 @@ static const TbVariant kTb[] = {
 
 namespace {
 
-// `gens` generations from P[*cur] with the one-generation kernel
-int run_step(appfis_ctx* ctx, uint32_t* const P[2], int* cur, int NW, int ny, int gens)
+// `gens` generations from P[*cur] in windows of variant v
+int run_win(appfis_ctx* ctx, const golbits::WinVariant& v, uint32_t* const P[2], int* cur, int nx, int ny, int gens,
+            int* launches)
 {
-    const int nbands = (ny + golbits::KROWS - 1) / golbits::KROWS;
-    const unsigned nitems = (unsigned)NW * (unsigned)nbands;
-    for (int g = 0; g < gens; g++) {
-        hipLaunchKernelGGL(golbits::k_step<golbits::KROWS>, dim3(ceil_div(nitems, 256)), dim3(256), 0, ctx->stream,
-                           P[*cur], P[*cur ^ 1], NW, ny, nitems);
+    const int NW = (nx + 31) / 32, tiles_x = (int)ceil_div(NW, golbits::WIN_WORDS);
+    const unsigned bands = ceil_div(ny, v.nwaves * v.k - 2 * v.g);
+    *launches = 0;
+    for (int done = 0; done < gens;) {
+        const int n = std::min(gens - done, v.g);
+        hipLaunchKernelGGL(v.kernel, dim3(bands * tiles_x), dim3(64 * v.nwaves), 0, ctx->stream, P[*cur], P[*cur ^ 1],
+                           nx, NW, ny, tiles_x, n);
         APPFIS_LAUNCH_CHECK();
         *cur ^= 1;
+        done += n;
+        ++*launches;
     }
     return APPFIS_OK;
 }
 
-// rows of a block's window: the full-row form stacks NWAVES bands; the other forms
-// spread each row over WX = NW / 64 waves
-int tb_rows(const golbits::TbVariant& v, int NW)
+// The window variant for `gens` generations of an nx x ny board, by the cost that its table
+// states: blocks that share a CU take about 0.8 of their times' sum.  Measured (48 generations,
+// us; k4 g24, k6 g24, k6 g16, k8 g24, k8 g16, k12 g16): 1000 x 1000 23 30 34 37 43 56; 3000 x 3000
+// 34 30 34 37 42 57; 8191 x 8191 139 88 79 86 71 92; 16384 x 16384 457 247 199 201 196 171.
+const golbits::WinVariant& win_for(const appfis_ctx* ctx, int nx, int ny, int gens)
 {
-    return v.wpl > 0 ? v.nwaves * v.k : (v.nwaves / (NW / 64)) * v.k;
+    const double cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
+    const golbits::WinVariant* best = nullptr;
+    double least = 0.0;
+    for (const golbits::WinVariant& v : golbits::kWin) {
+        const double blocks = (double)ceil_div((nx + 31) / 32, golbits::WIN_WORDS) * ceil_div(ny, v.nwaves * v.k - 2 * v.g);
+        const double load = blocks <= cus ? 1.0 : 0.8 * std::ceil(blocks / cus);
+        const double cost = 4.5 * ceil_div(gens, v.g) + gens * (0.07 + 0.0775 * v.k) * load;
+        if (!best || cost < least) {
+            best = &v;
+            least = cost;
+        }
+    }
+    return *best;
 }
 
-bool tb_fits(const golbits::TbVariant& v, int NW)
+// `gens` generations from P[*cur] with k_step_tb, rows spread over NW / 64 waves
+int run_tb(appfis_ctx* ctx, uint32_t* const P[2], int* cur, int NW, int ny, int gens, int* launches)
 {
-    if (v.wpl > 0) return NW == 64 * v.wpl && v.nwaves * v.k > 2 * v.g;
-    if (NW % 64) return false;
-    const int WX = NW / 64;
-    return WX <= v.nwaves && v.nwaves % WX == 0 && (v.nwaves / WX) * v.k > 2 * v.g;
-}
-
-// `gens` generations from P[*cur] with temporal-blocking variant v (G per launch)
-int run_tb(appfis_ctx* ctx, const golbits::TbVariant& v, uint32_t* const P[2], int* cur, int NW, int ny, int gens)
-{
-    const int WX = NW / 64;
-    const int OUT = tb_rows(v, NW) - 2 * v.g;
-    const unsigned blocks = ceil_div((size_t)ny, (size_t)OUT);
+    using namespace golbits;
+    const int WX = NW / 64, OUT = TB_WAVES / WX * TB_K - 2 * TB_G;
+    *launches = 0;
     for (int done = 0; done < gens;) {
-        const int n = gens - done < v.g ? gens - done : v.g;
-        hipLaunchKernelGGL(v.kernel, dim3(blocks), dim3(64 * v.nwaves), 0, ctx->stream, P[*cur], P[*cur ^ 1], NW, ny,
-                           WX, OUT, n);
+        const int n = std::min(gens - done, TB_G);
+        hipLaunchKernelGGL((k_step_tb<TB_K, TB_G, TB_WAVES>), dim3(ceil_div(ny, OUT)), dim3(64 * TB_WAVES), 0,
+                           ctx->stream, P[*cur], P[*cur ^ 1], NW, ny, WX, OUT, n);
+        APPFIS_LAUNCH_CHECK();
+        *cur ^= 1;
+        done += n;
+        ++*launches;
+    }
+    return APPFIS_OK;
+}
+
+// a row is whole waves, a divisor of the block's, and the rows left hold more than the halo
+bool tb_fits(int nx)
+{
+    using namespace golbits;
+    const int WX = nx / 2048;
+    return nx % 2048 == 0 && WX <= TB_WAVES && TB_WAVES % WX == 0 && TB_WAVES / WX * TB_K > 2 * TB_G;
+}
+
+int tw_out(const golbits::TwVariant& v) { return v.nwaves * v.k - 2 * v.g; }
+
+// `gens` generations from P[*cur] with full-row variant v (G per launch)
+int run_tw(appfis_ctx* ctx, const golbits::TwVariant& v, uint32_t* const P[2], int* cur, int NW, int ny, int gens)
+{
+    const int OUT = tw_out(v);
+    for (int done = 0; done < gens;) {
+        const int n = std::min(gens - done, v.g);
+        hipLaunchKernelGGL(v.kernel, dim3(ceil_div(ny, OUT)), dim3(64 * v.nwaves), 0, ctx->stream, P[*cur], P[*cur ^ 1],
+                           NW, ny, OUT, n);
         APPFIS_LAUNCH_CHECK();
         *cur ^= 1;
         done += n;
@@ -718,63 +708,81 @@ int run_tb(appfis_ctx* ctx, const golbits::TbVariant& v, uint32_t* const P[2], i
     return APPFIS_OK;
 }
 
+size_t packed_bytes(int nx, int ny) { return ((size_t)((nx + 31) / 32) * ny * 4 + 255) / 256 * 256; }
+
 }  // namespace
 
-// Runs `gens` >= 1 generations of the nx x ny periodic field (nx % 32 == 0) held in
-// buf0; see the file comment for what the two buffers hold on return.  When the packed
-// row width is a multiple of 64 words (and at most 1024), the generations run
-// temporally blocked (tile height and depth autotuned per shape).  With a full-row
-// variant and two or more generations, all of them run in its launches (at least two),
-// the first reading the uint8 field and the last writing both uint8 buffers; otherwise
-// k_pack packs the field, generations 1 .. gens-1 run blocked, and the last one runs
-// fused with the unpacking (k_step_unpack), so that generation gens-1 is still at hand.
+bool gol_bits_workspace(appfis_ctx* ctx, int nx, int ny)
+{
+    if (ensure_work(ctx, 2 * packed_bytes(nx, ny)) == APPFIS_OK) return true;
+    (void)hipGetLastError();  // an allocation that failed is no error of the launches that follow
+    return false;
+}
+
+// Runs `gens` >= 1 generations of the nx x ny periodic field (nx >= 32) held in buf0; see the
+// file comment for what the two buffers hold on return.  Two blocked forms advance the packed
+// field: windows (k_step_win) for any width, their shape chosen by win_for, and, where a wave
+// spans the row (nx = 2048, 4096 or 8192), full-row waves (k_step_tw), which the tuner times
+// against the window (at 8192 x 8192 63 us for 48 generations against 69, at 2048 x 2048 31
+// against 24).  With full-row waves and two or more generations, all of them run in their
+// launches (at least two), the first reading the uint8 field and the last writing both uint8
+// buffers; otherwise k_pack packs the field, generations 1 .. gens-1 run blocked, and the last
+// one runs fused with the unpacking (k_step_unpack), so that generation gens-1 is still at hand.
 int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int gens, int force)
 {
-    APPFIS_REQUIRE(nx % 32 == 0, "gol: the bit-packed form needs nx %% 32 == 0 (nx = %d)", nx);
-    const int NW = nx / 32;
-    const int ntb = (int)(sizeof(golbits::kTb) / sizeof(golbits::kTb[0]));
+    const int NW = (nx + 31) / 32;
+    const int ntw = (int)(sizeof(golbits::kTw) / sizeof(golbits::kTw[0]));
+    const int nwin = (int)(sizeof(golbits::kWin) / sizeof(golbits::kWin[0]));
+    const auto fits = [&](int i) { return nx % 32 == 0 && NW == 64 * golbits::kTw[i].wpl; };
     if (force >= 0) {
-        APPFIS_REQUIRE(force < ntb, "gol: candidate %d out of range (%d candidates)", force, ntb);
-        APPFIS_REQUIRE(tb_fits(golbits::kTb[force], NW),
-                       "gol: candidate %s needs nx that its block of waves spans (nx = %d)",
-                       golbits::kTb[force].name, nx);
+        APPFIS_REQUIRE(nx >= 32, "gol: the bit-packed form needs nx >= 32 (nx = %d)", nx);
+        APPFIS_REQUIRE(force <= ntw + nwin, "gol: candidate %d out of range (%d candidates)", force, ntw + nwin + 1);
+        APPFIS_REQUIRE(force >= ntw || fits(force), "gol: candidate %s needs nx that its waves span (nx = %d)",
+                       golbits::kTw[force].name, nx);
+        APPFIS_REQUIRE(force < ntw + nwin || tb_fits(nx), "gol: candidate tb needs nx that its block spans (nx = %d)", nx);
     }
-    const size_t words = (size_t)NW * ny;
-    const size_t half = (words * 4 + 255) / 256 * 256;
+    const size_t half = packed_bytes(nx, ny);
     int st = ensure_work(ctx, 2 * half);
     if (st) return st;
     uint32_t* const P[2] = {(uint32_t*)ctx->work, (uint32_t*)((char*)ctx->work + half)};
-    // autotune the blocked variant on the two packed buffers before they hold the field
-    // (timing does not depend on the cell values)
-    std::vector<int> cand;
-    std::vector<const char*> names;
-    for (int i = 0; i < ntb; i++)
-        if (tb_fits(golbits::kTb[i], NW)) {
-            cand.push_back(i);
-            names.push_back(golbits::kTb[i].name);
+    const golbits::WinVariant* win = force >= ntw && force < ntw + nwin ? &golbits::kWin[force - ntw] : nullptr;
+    const golbits::TwVariant* tw = force >= 0 && force < ntw ? &golbits::kTw[force] : nullptr;
+    if (force < 0) {
+        win = &win_for(ctx, nx, ny, gens > 1 ? gens - 1 : 1);
+        std::vector<const golbits::TwVariant*> cand;
+        std::vector<const char*> names;
+        for (int i = 0; i < ntw; i++)
+            if (fits(i)) {
+                cand.push_back(&golbits::kTw[i]);
+                names.push_back(golbits::kTw[i].name);
+            }
+        if (!cand.empty() && gens > 1) {
+            // on the two packed buffers before they hold the field (timing does not depend on
+            // the cell values); the window is the rule's for the 48 timed generations
+            const golbits::WinVariant& wt = win_for(ctx, nx, ny, 48);
+            names.push_back(wt.name);
+            const int key[6] = {4, APPFIS_U8, nx, ny, 0, 0};
+            int c = 0;
+            st = tune_select(ctx, key, (int)names.size(), names.data(),
+                             [&](int i) {
+                                 int tmp = 0, n = 0;
+                                 return i < (int)cand.size() ? run_tw(ctx, *cand[i], P, &tmp, NW, ny, 48)
+                                                             : run_win(ctx, wt, P, &tmp, nx, ny, 48, &n);
+                             },
+                             4, &c);
+            if (st) return st;
+            if (c < (int)cand.size()) tw = cand[c];
         }
-    int pick = force;
-    if (force < 0 && !cand.empty() && gens > 1) {
-        const int key[6] = {4, APPFIS_U8, nx, ny, 0, 0};
-        int c = 0;
-        st = tune_select(ctx, key, (int)cand.size(), names.data(),
-                         [&](int i) {
-                             int tmp = 0;
-                             return run_tb(ctx, golbits::kTb[cand[i]], P, &tmp, NW, ny, 48);
-                         },
-                         4, &c);
-        if (st) return st;
-        pick = cand[c];
     }
     uint8_t* buf[2] = {b0, b1};
-    if (pick >= 0 && golbits::kTb[pick].kin && gens >= 2) {
+    if (tw && gens >= 2) {
         // full-row form over two or more launches: the first packs the uint8 field as it
         // loads its window, the last writes generations gens and gens-1 back as uint8
         // (rings included) -- after the first has finished reading b0, which it may
         // overwrite.  Up to G generations: gens-1 in the first launch, 1 in the last;
         // beyond: G per launch, the rest in the last.
-        const golbits::TbVariant& v = golbits::kTb[pick];
-        const int OUT = tb_rows(v, NW) - 2 * v.g;
+        const golbits::TwVariant& v = *tw;
+        const int OUT = tw_out(v);
         const dim3 grid(ceil_div((size_t)ny, (size_t)OUT)), block(64 * v.nwaves);
         const int L = gens <= v.g ? 2 : (gens + v.g - 1) / v.g;
         const int first = gens <= v.g ? gens - 1 : v.g;
@@ -786,7 +794,7 @@ int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int 
         APPFIS_LAUNCH_CHECK();
         int cur = 0;
         for (int l = 1; l < L - 1; l++) {
-            hipLaunchKernelGGL(v.kernel, grid, block, 0, ctx->stream, P[cur], P[cur ^ 1], NW, ny, NW / 64, OUT, v.g);
+            hipLaunchKernelGGL(v.kernel, grid, block, 0, ctx->stream, P[cur], P[cur ^ 1], NW, ny, OUT, v.g);
             APPFIS_LAUNCH_CHECK();
             cur ^= 1;
         }
@@ -795,20 +803,17 @@ int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int 
         APPFIS_LAUNCH_CHECK();
         return ktime_end(ctx, L, gens);
     }
-    const unsigned pblocks = ceil_div(words, 256);
+    const unsigned pblocks = ceil_div((size_t)NW * ny, 256);
     hipLaunchKernelGGL(golbits::k_pack, dim3(pblocks), dim3(256), 0, ctx->stream, b0, P[0], nx, ny, NW);
     APPFIS_LAUNCH_CHECK();
-    int cur = 0;
+    int cur = 0, launches = 0;
     st = ktime_begin(ctx);
     if (st) return st;
-    int launches = gens - 1;
-    if (pick >= 0 && gens > 1) {
-        st = run_tb(ctx, golbits::kTb[pick], P, &cur, NW, ny, gens - 1);
-        launches = (gens - 1 + golbits::kTb[pick].g - 1) / golbits::kTb[pick].g;
-    } else {
-        st = run_step(ctx, P, &cur, NW, ny, gens - 1);
+    if (gens > 1) {
+        st = win ? run_win(ctx, *win, P, &cur, nx, ny, gens - 1, &launches)
+                 : run_tb(ctx, P, &cur, NW, ny, gens - 1, &launches);
+        if (st) return st;
     }
-    if (st) return st;
     st = ktime_end(ctx, launches, gens - 1);
     if (st) return st;
     // generation gens-1 is in P[cur]: the last generation runs fused with the unpacking
@@ -824,9 +829,11 @@ int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int 
 
 extern "C" int appfis_gol_candidates(char* names, int len)
 {
-    const int ntb = (int)(sizeof(golbits::kTb) / sizeof(golbits::kTb[0]));
     std::string all;
-    for (int i = 0; i < ntb; i++) all += std::string(golbits::kTb[i].name) + "\n";
+    int n = 0;
+    for (const golbits::TwVariant& v : golbits::kTw) all += std::string(v.name) + "\n", n++;
+    for (const golbits::WinVariant& v : golbits::kWin) all += std::string(v.name) + "\n", n++;
+    all += "tb k10 g4 w16\n";
     if (names && len > 0) snprintf(names, (size_t)len, "%s", all.c_str());
-    return ntb;
+    return n + 1;
 }

@@ -215,16 +215,18 @@ int appfis_heat2d_ensemble(appfis_ctx* ctx, int dtype, int ngrid, const int* nx,
  *      game_appfis.hpp:121-135 plus the periodic exchange of Communication.hpp:613-678).
  * bufs as for heat2d (ghost 1, padded (nx+2)*(ny+2)).  The ghost ring of the
  * written buffer is refreshed every generation.  PLAIN: one generation per launch;
- * CHOSEN (nx % 32 == 0): the generations run on a bit-packed copy of the field (32
- * cells per word), both buffers are left exactly as PLAIN leaves them; other widths
- * run the PLAIN kernel.  `tsteps` is reserved (pass 0).  Cells must hold 0 or 1.
+ * CHOSEN (nx >= 32): the generations run on a bit-packed copy of the field (32
+ * cells per word), both buffers are left exactly as PLAIN leaves them; narrower boards
+ * run the PLAIN kernel, and so does a first call under graph capture where nx is no
+ * multiple of 32.  `tsteps` is reserved (pass 0).  Cells must hold 0 or 1.
  * APPFIS_CANDIDATE0 + i: the bit-packed form with blocked candidate i forced. */
 int appfis_gol(appfis_ctx* ctx, uint8_t* buf0, uint8_t* buf1, int nx, int ny, int gens,
                int variant, int tsteps);
 
 /* Blocked kernels of the bit-packed GoL form (variant APPFIS_CANDIDATE0 + i forces
- * candidate i; it needs nx a multiple of 2048 spanned by its block), one name per
- * line; returns their number. */
+ * candidate i; "tw" needs nx = 2048, 4096 or 8192, spanned by its waves, "win" nx >= 32,
+ * "tb" nx a multiple of 2048 spanned by its block), one name per line; returns their
+ * number. */
 int appfis_gol_candidates(char* names, int len);
 
 /* ---- FDTD3d radius-4 star (config form of FDTD3d/src/fdtd3d_appfis.hpp:129-143):

@@ -231,6 +231,25 @@ def test_gol_every_blocked_candidate(ctx, nx, ny, gens):
     assert len(ran) >= 3
 
 
+@pytest.mark.parametrize("nx,ny,gens", [(32, 3, 20), (33, 5, 9), (40, 2, 26), (63, 64, 17), (64, 97, 33), (65, 17, 25),
+                                        (1000, 77, 49), (1983, 40, 20), (1984, 33, 9), (1985, 50, 18), (2016, 20, 17),
+                                        (4031, 49, 34), (6144, 30, 19), (8191, 100, 33), (31, 12, 9)])
+def test_gol_windows_of_any_width(ctx, nx, ny, gens):
+    # every window shape forced, and the one the rule takes, where the row ends inside, at and
+    # just past a word and a window (62 stored words), in boards narrower than a window and
+    # lower than a block (both wrap around several times); 31 cells run the byte kernel
+    a, d0, d1 = _gol_pair(ctx, nx, ny, seed=nx * 11 + gens)
+    ref = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens)
+    prev = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens - 1)
+    wins = [hip.CANDIDATE0 + i for i, name in enumerate(hip.gol_candidates()) if name.startswith("win ")]
+    assert len(wins) >= 3
+    for variant in [hip.CHOSEN] + (wins if nx >= 32 else []):
+        d0.upload(a)
+        ctx.gol(d0, d1, nx, ny, gens, variant)
+        assert np.array_equal((d0, d1)[gens % 2].download(), ref), variant
+        assert np.array_equal((d0, d1)[(gens + 1) % 2].download(), prev), variant
+
+
 @pytest.mark.parametrize("gens", [2, 7, 8, 9, 16, 17, 24, 25])
 def test_gol_full_row_launch_split(ctx, gens):
     # the full-row form runs a call's generations in at least two launches, the first
