@@ -15,6 +15,9 @@
 // partial per block, and the last block to arrive (atomic ticket) sums the partials in
 // block order into gosa[it] -- deterministic, on the device, no host round trip.
 //
+// Sweeps run in pairs where they can (k_himeno_two): one pass over the coefficients serves two
+// sweeps.
+//
 // PLAIN (F32 or F64): the reference operation order, no FMA contraction.
 // CHOSEN (defect correction, F64 problem): p = B + q with a FP64 base B and a FP32
 //   correction q.  Because the sweep is affine, ss(B + q) = ss(B) + L q with
@@ -26,6 +29,7 @@
 //   made once per call, inside the call, blocked by 64 points (Coef::inter).
 #include "common.hpp"
 
+#include <algorithm>
 #include <vector>
 
 using namespace appfis;
@@ -73,41 +77,59 @@ __device__ inline void tile_of(int nx, int ny, int ry, int& bx, int& by, int& bz
     bz = r / gy;
 }
 
-__device__ inline double block_sum_last(double v, double* partials, unsigned* ticket, double* out, double* lds)
+// Adds the block's sums of v[0 .. NV-1] to partials[bid * NV ..]; the last block to arrive sums
+// the partials in block order into out[0 .. NV-1].
+template <int NT, int NV>
+__device__ inline void block_sum_last(const double (&v)[NV], double* partials, unsigned* ticket, double* out,
+                                      double* lds)
 {
     const auto add = [](double a, double b) { return a + b; };
-    v = wave_reduce(v, 0.0, add);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     __shared__ bool last;
-    const unsigned nblk = gridDim.x * gridDim.y * gridDim.z;
-    const unsigned bid = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    if (lane == WAVE_TOTAL_LANE) lds[wid] = v;
+    const unsigned nblk = gridDim.x, bid = blockIdx.x;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const double w = wave_reduce(v[i], 0.0, add);
+        if (lane == WAVE_TOTAL_LANE) lds[NV * wid + i] = w;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < TX / 64; w++) s += lds[w];
-        partials[bid] = s;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            double s = 0.0;
+            for (int w = 0; w < NT / 64; w++) s += lds[NV * w + i];
+            partials[(size_t)bid * NV + i] = s;
+        }
         __threadfence();
         unsigned prev = atomicAdd(ticket, 1u);
         last = (prev == nblk - 1);
     }
     __syncthreads();
-    if (!last) return 0.0;
+    if (!last) return;
     __threadfence();
-    double acc = 0.0;
-    for (unsigned p = threadIdx.x; p < nblk; p += TX)
-        acc += __hip_atomic_load(partials + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    acc = wave_reduce(acc, 0.0, add);
+    double acc[NV];
+#pragma unroll
+    for (int i = 0; i < NV; i++) acc[i] = 0.0;
+    for (unsigned p = threadIdx.x; p < nblk; p += NT)
+#pragma unroll
+        for (int i = 0; i < NV; i++)
+            acc[i] += __hip_atomic_load(partials + (size_t)p * NV + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    if (lane == WAVE_TOTAL_LANE) lds[wid] = acc;
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+        const double w = wave_reduce(acc[i], 0.0, add);
+        if (lane == WAVE_TOTAL_LANE) lds[NV * wid + i] = w;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int w = 0; w < TX / 64; w++) s += lds[w];
-        *out = s;
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            double s = 0.0;
+            for (int w = 0; w < NT / 64; w++) s += lds[NV * w + i];
+            out[i] = s;
+        }
         *ticket = 0u;
     }
-    return 0.0;
 }
 
 // Buffer accesses: every load and store of the sweep is a buffer instruction on a
@@ -262,7 +284,7 @@ __global__ __launch_bounds__(TX) void k_himeno(const T* __restrict__ p, T* __res
     T cr[NS][RY][NC];
 #pragma unroll
     for (int s = 0; s < D; s++) coef_load(min(k0 + s, nz - 2), cr[s]);
-    double g = 0.0;
+    double g[1] = {0.0};
     for (int kb = k0; kb < k1; kb += NS) {
 #pragma unroll
         for (int s = 0; s < NS; s++) {
@@ -309,11 +331,208 @@ __global__ __launch_bounds__(TX) void k_himeno(const T* __restrict__ p, T* __res
                 } else {
                     st<T>(rw, so, pc + omega * ss);
                 }
-                g += (double)ss * (double)ss;
+                g[0] += (double)ss * (double)ss;
             }
         }
     }
-    block_sum_last(g, partials, ticket, gosa_out, red);
+    block_sum_last<TX, 1>(g, partials, ticket, gosa_out, red);
+}
+
+// Tiles of the two-sweep kernel: windows of BX columns and WR rows.  A tile's sweep 2 needs sweep 1
+// one cell further out, so it stores the window less its outer ring -- except the left column
+// of the first tile in x, whose neighbour is the shell: rows of 2^n + 1 cells (2^n - 1 updated
+// ones) are then one tile of 2^n columns.
+__host__ __device__ inline int two_tiles_x(int nx, int bx) { return nx - 2 <= bx - 1 ? 1 : 1 + (nx - 2 - (bx - 1) + bx - 3) / (bx - 2); }
+__host__ __device__ inline int two_tiles_y(int ny, int wr) { return (ny - 2 + wr - 3) / (wr - 2); }
+
+// Two sweeps in one pass over the coefficients (12 of the 14 streams of a sweep).  A block marches
+// its window of BX columns and WR = NWY * RY rows along k; at step k it computes sweep 1 of
+// plane k from the staged planes k-1, k, k+1 into a second LDS ring, and sweep 2 of plane k-1
+// from that ring's planes k-2, k-1, k.  The coefficients of plane k-1 are still in registers from
+// the step before, those of plane k+1 are in flight (a ring of three).  A chunk of zc planes
+// computes sweep 1 on one plane more at either end.  Same operation order per sweep as k_himeno:
+// bit-identical.  Between the sweeps of a PLAIN call the shell changes from p0's to p1's: sha
+// holds the shell that sweep 1 reads and shb the one that sweep 2 reads (p's interior lies in
+// whichever buffer the last launch wrote).  gosa_out[0], [1]: the two sweeps' residuals.
+//
+// What bounds it is the memory side: at 257 x 257 x 513 in FP32 a launch moves 2.0 GB (14 streams
+// once, and 7% for halo rows that L2 did not hold: neighbouring tiles share an XCD) in 475 us,
+// 4.2 TB/s, against 1.9 GB in 372 us for one sweep; the arithmetic takes about 100 us of it.  The
+// coefficients of plane k+1 are requested half before the first barrier and half before the
+// second, so that requests do not come in one burst a plane (254 -> 238 us a sweep).  Two
+// shapes of the loop measured the same: one barrier per plane with sweep 2 lagging two planes,
+// and twice the rows per thread in half the waves.
+template <typename T, int MODE, int BX, int NWY, int RY>
+__global__ __launch_bounds__(BX* NWY) void k_himeno_two(const T* __restrict__ p, T* __restrict__ pn,
+                                                        const T* __restrict__ sha, const T* __restrict__ shb, Coef cf,
+                                                        int nx, int ny, int nz, int zc, T omega, double* partials,
+                                                        unsigned* ticket, double* gosa_out)
+{
+    static_assert(MODE == 0 || (MODE == 2 && sizeof(T) == 4), "PLAIN, or the FP32 inner sweep");
+    constexpr int NT = BX * NWY, WR = NWY * RY, OUT = WR - 2;
+    constexpr int LX = BX + 2, LH = WR + 2;       // staged row and rows: the window and its halo
+    constexpr int PPT = (LX * LH + NT - 1) / NT;  // staged values per thread
+    constexpr int NC = 12, NS = 3;
+    __shared__ T ring0[NS][LH][LX];
+    __shared__ T ring1[NS][WR][LX];
+    __shared__ double red[2 * NT / 64];
+    const int tx = threadIdx.x % BX, ty = threadIdx.x / BX;
+    const int gx = two_tiles_x(nx, BX), gy = two_tiles_y(ny, WR);
+    const int t = (int)xcd_tile(blockIdx.x, gridDim.x);  // x fastest, then y: neighbours share an L2
+    const int bx = t % gx, by = t / gx % gy, bz = t / gx / gy;
+    const int xs = bx == 0 ? 1 : BX + (bx - 1) * (BX - 2) - 1;  // first window column
+    const int ys = by * OUT;                                    // first window row
+    const int k0 = bz * zc + 1, k1 = min(k0 + zc, nz - 1);      // planes stored
+    const int sy = nx, sz = nx * ny;                            // < 2^31 elements (checked on the host)
+    const uint32_t pbytes = (uint32_t)sz * (uint32_t)sizeof(T);  // < 2^31 (checked on the host)
+    const int i = xs + tx, j0 = ys + ty * RY;
+    const T* arr[NC] = {(const T*)cf.a0, (const T*)cf.a1, (const T*)cf.a2, (const T*)cf.a3, (const T*)cf.b0,
+                        (const T*)cf.b1, (const T*)cf.b2, (const T*)cf.c0, (const T*)cf.c1, (const T*)cf.c2,
+                        (const T*)cf.bnd, (const T*)cf.wrk1};
+    // staged cells of this thread (cell e of the staged window: e = threadIdx.x + q * NT), as
+    // pointers into plane 0 of the array that sweep 1 reads them from; cells outside the array
+    // feed nothing that is stored and read the plane's first cell
+    const gmem<T>* src[PPT];
+    const long long to_sha = sha - p;  // from a cell of p to the same cell of sha
+    uint32_t in_p = 0;                 // bit q: src[q] points into p
+#pragma unroll
+    for (int q = 0; q < PPT; q++) {
+        const int e = (int)threadIdx.x + q * NT;
+        const int ly = e / LX, lx = e - ly * LX;
+        const int x = xs - 1 + lx, y = ys - 1 + ly;
+        const bool in = e < LX * LH && x < nx && y >= 0 && y < ny;  // x >= 0
+        const bool shell = x == 0 || x == nx - 1 || y == 0 || y == ny - 1;
+        src[q] = to_global(p) + (in ? x + sy * y : 0);
+        if (in && !shell) in_p |= 1u << q;
+        else src[q] += to_sha;
+    }
+    // own cells: inside (updated by both sweeps) and stored; a cell that is not inside takes the
+    // value of the shell that sweep 2 reads, and so does the column left of the first tile, whose
+    // rows the first WR threads hold
+    bool inside[RY], stored[RY];
+    uint32_t own[RY];
+#pragma unroll
+    for (int r = 0; r < RY; r++) {
+        const int j = j0 + r, wr = ty * RY + r;
+        inside[r] = i <= nx - 2 && j >= 1 && j <= ny - 2;
+        stored[r] = inside[r] && wr >= 1 && wr <= WR - 2 && tx <= BX - 2 && (bx == 0 || tx >= 1);
+        const bool in = i <= nx - 1 && j <= ny - 1;
+        own[r] = in ? (uint32_t)(i + sy * j) * (uint32_t)sizeof(T) : kOut;
+    }
+    const bool left = bx == 0 && (int)threadIdx.x < WR;
+    const uint32_t lsh = left && ys + (int)threadIdx.x <= ny - 1
+                             ? (uint32_t)(sy * (ys + (int)threadIdx.x)) * (uint32_t)sizeof(T) : kOut;
+    T* const r0 = &ring0[0][0][0] + threadIdx.x;
+    auto stage_load = [&](int k, T(&v)[PPT]) {
+        const int kc = min(max(k, 0), nz - 1);  // planes outside the array feed nothing
+        if (kc == 0 || kc == nz - 1) {
+#pragma unroll
+            for (int q = 0; q < PPT; q++) v[q] = src[q][(long long)sz * kc + (in_p >> q & 1u ? to_sha : 0)];
+        } else {
+#pragma unroll
+            for (int q = 0; q < PPT; q++) v[q] = src[q][(long long)sz * kc];
+        }
+    };
+    auto stage_store = [&](int slot, const T(&v)[PPT]) {
+#pragma unroll
+        for (int q = 0; q < PPT; q++)
+            if ((q + 1) * NT <= LX * LH || (int)threadIdx.x < LX * LH - q * NT) r0[slot * (LH * LX) + q * NT] = v[q];
+    };
+    auto coef_load = [&](int k, T(&c)[RY][NC], int ra, int rb) {
+        const int kc = min(max(k, 1), nz - 2);
+        if constexpr (MODE == 2) {
+            const int b = sz * kc;
+            const auto rs = rsrc((const float*)cf.inter + (size_t)(b >> 6) * BLK,
+                                 (uint32_t)((sz >> 6) + 2) * (uint32_t)(BLK * 4));
+#pragma unroll
+            for (int r = ra; r < rb; r++) {
+                const int q = i + sy * (j0 + r) + b;
+                const uint32_t o = inside[r] ? (uint32_t)(((q >> 6) - (b >> 6)) * BLK + (q & 63)) * 4u : kOut;
+#pragma unroll
+                for (int a = 0; a < NC; a++) c[r][a] = ld<T>(rs, o + (uint32_t)(a * 256));
+            }
+        } else {
+#pragma unroll
+            for (int a = 0; a < NC; a++) {
+                const auto rs = rsrc(arr[a] + (long long)sz * kc, pbytes);
+#pragma unroll
+                for (int r = ra; r < rb; r++) c[r][a] = ld<T>(rs, inside[r] ? own[r] : kOut);
+            }
+        }
+    };
+    // the shell values of plane k that sweep 2 reads: the whole window of planes 0 and nz-1
+    auto shell_load = [&](int k, T(&v)[RY], T& l) {
+        const int kc = min(max(k, 0), nz - 1);
+        const bool all = kc == 0 || kc == nz - 1;
+        const auto rs = rsrc(shb + (long long)sz * kc, pbytes);
+#pragma unroll
+        for (int r = 0; r < RY; r++) v[r] = ld<T>(rs, all || !inside[r] ? own[r] : kOut);
+        l = ld<T>(rs, lsh);
+    };
+    // ss of one point: m, z, q the planes below, of and above it (rows of LX values), at their
+    // centre
+    auto residual = [&](const T* m, const T* z, const T* q, const T(&c)[NC]) -> T {
+        T s0 = c[0] * z[1] + c[1] * z[LX] + c[2] * q[0]
+               + c[4] * (z[LX + 1] - z[-LX + 1] - z[LX - 1] + z[-LX - 1])
+               + c[5] * (q[LX] - q[-LX] - m[LX] + m[-LX])
+               + c[6] * (q[1] - q[-1] - m[1] + m[-1])
+               + c[7] * z[-1] + c[8] * z[-LX] + c[9] * m[0];
+        if constexpr (MODE == 2) return c[11] + (s0 * c[3] - z[0]) * c[10];
+        s0 = s0 + c[11];
+        return (s0 * c[3] - z[0]) * c[10];
+    };
+    const int ka = k0 - 1;  // first plane of sweep 1; slot of plane k: (k - ka) % 3
+    T pnext[PPT], cr[NS][RY][NC], shv[RY], shl;
+    stage_load(ka - 1, pnext);
+    stage_store(2, pnext);
+    stage_load(ka, pnext);
+    stage_store(0, pnext);
+    stage_load(ka + 1, pnext);
+    coef_load(ka, cr[0], 0, RY);
+    shell_load(ka, shv, shl);
+    double g[2] = {0.0, 0.0};
+    for (int kb = ka; kb <= k1; kb += NS) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            const int k = kb + s;
+            if (k > k1) break;
+            stage_store((s + 1) % NS, pnext);
+            stage_load(k + 2, pnext);
+            coef_load(k + 1, cr[(s + 1) % NS], 0, RY / 2);
+            __syncthreads();
+            {
+                const bool plane = k >= 1 && k <= nz - 2;
+                const bool count = k >= k0 && k < k1;
+#pragma unroll
+                for (int r = 0; r < RY; r++) {
+                    const int wr = ty * RY + r;
+                    const T* z = &ring0[s][wr + 1][tx + 1];
+                    const T ss = residual(&ring0[(s + 2) % NS][wr + 1][tx + 1], z, &ring0[(s + 1) % NS][wr + 1][tx + 1],
+                                          cr[s][r]);
+                    ring1[s][wr][tx + 1] = plane && inside[r] ? z[0] + omega * ss : shv[r];
+                    if (count && stored[r]) g[0] += (double)ss * (double)ss;
+                }
+                if (left) ring1[s][threadIdx.x][0] = shl;
+            }
+            shell_load(k + 1, shv, shl);
+            coef_load(k + 1, cr[(s + 1) % NS], RY / 2, RY);
+            __syncthreads();
+            if (k > k0) {
+                const auto rw = rsrc(pn + (long long)sz * (k - 1), pbytes);
+                constexpr int F = 1;
+#pragma unroll
+                for (int r = 0; r < RY; r++) {
+                    // the window's first and last rows have no neighbours here and are not stored
+                    const int wr = min(max(ty * RY + r, F), WR - 1 - F);
+                    const T* z = &ring1[(s + 2) % NS][wr][tx + 1];
+                    const T ss = residual(&ring1[(s + 1) % NS][wr][tx + 1], z, &ring1[s][wr][tx + 1], cr[(s + 2) % NS][r]);
+                    st<T>(rw, stored[r] ? own[r] : kOut, z[0] + omega * ss);
+                    if (stored[r]) g[1] += (double)ss * (double)ss;
+                }
+            }
+        }
+    }
+    block_sum_last<NT, 2>(g, partials, ticket, gosa_out, red);
 }
 
 // The FP32 blocked coefficients of the inner sweep (see Coef::inter) from the FP64
@@ -388,15 +607,61 @@ void launch_sweep(appfis_ctx* ctx, SweepShape sh, const T* pin, T* pout, const C
     }
 }
 
+// Shape of the two-sweep kernel: the window width whose tiles leave the fewest lanes without a
+// column (of equal ones the widest, for FP64 128 columns), RY rows per thread and NWY thread
+// rows as the registers of three planes of coefficients allow, and as many chunks in z as give
+// about one block to a CU: the chunks at either end repeat planes, and fewer regions of the
+// arrays streamed at once run faster (257 x 257 x 513 FP32, us a sweep: 5 chunks 236, 10 chunks
+// 242, 16 chunks 263).  It beats the best one-sweep shape on every grid tried (us a sweep, FP32
+// one / two: 33 x 33 x 65 13.5 / 9.6, 65 x 65 x 129 21.5 / 13.9, 129 x 129 x 257 54.8 / 35.1,
+// 100 x 180 x 240 68.2 / 38.2, 257 x 257 x 513 372 / 236; FP64 32.4 / 18.9, 137 / 74, 180 / 78,
+// 700 / 470), so pairs of sweeps always run it.
+struct TwoShape {
+    int bx, wr, zc;
+    unsigned blocks;
+};
+template <typename T>
+TwoShape two_shape(int num_cu, int nx, int ny, int nz)
+{
+    const bool wide = sizeof(T) == 4;
+    TwoShape sh{wide ? 256 : 128, 0, 0, 0};
+    for (int bx : {256, 128, 64})
+        if (two_tiles_x(nx, bx) * bx < two_tiles_x(nx, sh.bx) * sh.bx) sh.bx = bx;
+    sh.wr = !wide && sh.bx == 256 ? 4 : 8;
+    const int tiles = two_tiles_x(nx, sh.bx) * two_tiles_y(ny, sh.wr);
+    const int chunks = std::max(1, std::min((num_cu > 0 ? num_cu : 256) / tiles, (nz - 2 + 3) / 4));
+    sh.zc = (int)ceil_div(nz - 2, chunks);
+    sh.blocks = (unsigned)tiles * ceil_div(nz - 2, sh.zc);
+    return sh;
+}
+
+template <typename T, int MODE>
+void launch_two(appfis_ctx* ctx, const T* pin, T* pout, const T* sha, const T* shb, const Coef& cf, int nx, int ny,
+                int nz, T omega, double* partials, unsigned* ticket, double* gosa)
+{
+    const TwoShape sh = two_shape<T>(ctx->num_cu, nx, ny, nz);
+    auto go = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(sh.blocks), dim3(threads), 0, ctx->stream, pin, pout, sha, shb, cf, nx, ny, nz,
+                           sh.zc, omega, partials, ticket, gosa);
+    };
+    constexpr bool wide = sizeof(T) == 4;
+    switch (sh.bx) {
+    case 256: go(k_himeno_two<T, MODE, 256, 4, wide ? 2 : 1>, 1024); break;
+    case 128: go(k_himeno_two<T, MODE, 128, 4, 2>, 512); break;
+    default: go(k_himeno_two<T, MODE, 64, 4, 2>, 256); break;
+    }
+}
+
 }  // namespace
 
 extern "C" int appfis_himeno_candidates(char* names, int len)
 {
     std::string all;
     for (int f = 0; f < 2; f++)
-        for (int i = 0; i < NSHAPE; i++) all += std::string(f ? "dc " : "plain ") + kShapeNames[i] + "\n";
+        for (int i = 0; i <= NSHAPE; i++)
+            all += std::string(f ? "dc " : "plain ") + (i < NSHAPE ? kShapeNames[i] : "two") + "\n";
     if (names && len > 0) snprintf(names, (size_t)len, "%s", all.c_str());
-    return 2 * NSHAPE;
+    return 2 * (NSHAPE + 1);
 }
 
 extern "C" int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, int nx, int ny, int nz, double omega,
@@ -412,7 +677,10 @@ extern "C" int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, in
     APPFIS_REQUIRE((double)nx * ny * (dtype == APPFIS_F32 ? 4.0 : 8.0) < 2147483648.0,
                    "a plane of the grid exceeds 2 GiB (32-bit buffer offsets)");
     if (iters == 0) return APPFIS_OK;
-    const size_t nblk = grid_of(nx, ny, nz, kMinZc, kMinRy).x;  // at least the blocks any candidate launches
+    // at least the sums any candidate leaves: one per block, two per block of the two-sweep kernel
+    size_t nblk = grid_of(nx, ny, nz, kMinZc, kMinRy).x;
+    nblk = std::max(nblk, 2 * (size_t)two_shape<float>(ctx->num_cu, nx, ny, nz).blocks);
+    nblk = std::max(nblk, 2 * (size_t)two_shape<double>(ctx->num_cu, nx, ny, nz).blocks);
     // scratch: ticket | partials[nblk] | gosa[iters]
     const size_t off_part = 256, off_gosa = off_part + ((nblk * 8 + 255) / 256) * 256;
     int st = ensure_scratch(ctx, off_gosa + (size_t)iters * 8 + 256);
@@ -423,14 +691,19 @@ extern "C" int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, in
     Coef cf{arrays[2], arrays[3], arrays[4], arrays[5], arrays[6], arrays[7], arrays[8],
             arrays[9], arrays[10], arrays[11], arrays[12], arrays[13]};
 
-    // APPFIS_CANDIDATE0 + i: the PLAIN sweep with shape i forced (i < NSHAPE), or the
-    // defect correction with inner-sweep shape i - NSHAPE forced
+    // APPFIS_CANDIDATE0 + i: the PLAIN form (i <= NSHAPE), or the defect correction (the same
+    // list again), with every sweep in a launch of its own of shape i, or, for the last of the
+    // list, in pairs where the form allows it and in launches of a fixed shape where not
     int forced = -1;
+    bool pairs = true;
     if (variant >= APPFIS_CANDIDATE0) {
         forced = variant - APPFIS_CANDIDATE0;
-        APPFIS_REQUIRE(forced < 2 * NSHAPE, "himeno: candidate %d out of range (%d candidates)", forced, 2 * NSHAPE);
-        variant = forced < NSHAPE ? APPFIS_PLAIN : APPFIS_CHOSEN;
-        forced %= NSHAPE;
+        constexpr int N = NSHAPE + 1;
+        APPFIS_REQUIRE(forced < 2 * N, "himeno: candidate %d out of range (%d candidates)", forced, 2 * N);
+        variant = forced < N ? APPFIS_PLAIN : APPFIS_CHOSEN;
+        forced %= N;
+        pairs = forced == NSHAPE;
+        if (pairs) forced = 2;
     }
     // sweep shape: timed once per (dtype, form, grid shape) -- a sweep from p0 into p1
     // (PLAIN; the first real sweep rewrites p1) or between the correction buffers (CHOSEN)
@@ -462,7 +735,23 @@ extern "C" int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, in
         SweepShape sh;
         st = tune_shape(0, [&](int c) { return sweep(kShapes[c], 0); }, &sh);
         if (st) return st;
-        for (int it = 0; it < iters; it++) {
+        // Sweeps in pairs, then the last 1 to 4 one by one: an even number of pairs brings the
+        // field back to p0, so that every sweep that follows reads and writes the buffer of its
+        // parity and the call leaves the last two sweeps in p0 and p1.
+        int it = 0;
+        for (const int paired = pairs ? (iters - 1) / 4 * 4 : 0; it < paired; it += 2) {
+            void* pin = arrays[(it >> 1) & 1];
+            void* pout = arrays[((it >> 1) & 1) ^ 1];
+            if (dtype == APPFIS_F32)
+                launch_two<float, 0>(ctx, (const float*)pin, (float*)pout, (const float*)arrays[0],
+                                     (const float*)arrays[1], cf, nx, ny, nz, (float)omega, partials, ticket,
+                                     gosa_dev + it);
+            else
+                launch_two<double, 0>(ctx, (const double*)pin, (double*)pout, (const double*)arrays[0],
+                                      (const double*)arrays[1], cf, nx, ny, nz, omega, partials, ticket, gosa_dev + it);
+            APPFIS_LAUNCH_CHECK();
+        }
+        for (; it < iters; it++) {
             st = sweep(sh, it);
             if (st) return st;
         }
@@ -523,6 +812,11 @@ extern "C" int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, in
                 launch_sweep<double, 1>(ctx, sh, B[bi], B[bi ^ 1], cr, nx, ny, nz, omega, partials, ticket,
                                         gosa_dev + it);
                 bi ^= 1;
+            } else if (pairs && it + 1 < iters && (it + 1) % K != 0) {
+                // the shells of the two correction buffers are both zero
+                launch_two<float, 2>(ctx, q[qi], q[qi ^ 1], q[qi], q[qi], c32s, nx, ny, nz, (float)omega, partials,
+                                     ticket, gosa_dev + it);
+                it++;
             } else {
                 launch_sweep<float, 2>(ctx, sh, q[qi], q[qi ^ 1], c32s, nx, ny, nz, (float)omega, partials, ticket,
                                        gosa_dev + it);

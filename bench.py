@@ -506,8 +506,12 @@ def bench_himeno(ctx, hip, nx=257, ny=257, nz=513, iters=200):
         ry = int(shape.split()[2][2:]) if len(shape.split()) > 2 else 2
         r["tiling"] = shape
         if bpl:
+            # the sweeps but the last 1 to 4 run two to a launch (k_himeno_two): launches per sweep
+            t, rows = ("float", 2) if dt == hip.F32 else ("double", 1)
+            pairs = (iters - 1) // 4 * 2
             r["roofline"] = roofline(float(bpl) * pts, ms / iters,
-                                     f"k_himeno<{'float' if dt == hip.F32 else 'double'}, 0, {d}, {ry}>")
+                                     {f"k_himeno_two<{t}, 0, 256, 4, {rows}>": pairs / iters,
+                                      f"k_himeno<{t}, 0, {d}, {ry}>": (iters - 2 * pairs) / iters})
         else:
             # defect correction, per sweep on average over one outer cycle of K sweeps
             # (the library's default K = 16): K-1 FP32 inner sweeps (11 coefficients, read
@@ -515,8 +519,10 @@ def bench_himeno(ctx, hip, nx=257, ny=257, nz=513, iters=200):
             # rebase (11 coefficients, wrk1, B read, q read 4 B, B / r / q written
             # 8 + 4 + 4 B: 124 B/LUP)
             K = HIMENO_DC_OUTER
+            # The inner sweeps run two to a launch, but for the one left over.
             r["roofline"] = roofline(((K - 1) * 56.0 + 124.0) / K * pts, ms / iters,
-                                     {f"k_himeno<float, 2, {d}, {ry}>": (K - 1) / K,
+                                     {"k_himeno_two<float, 2, 256, 4, 2>": (K - 1) // 2 / K,
+                                      f"k_himeno<float, 2, {d}, {ry}>": (K - 1) % 2 / K,
                                       f"k_himeno<double, 1, {d}, {ry}>": 1 / K})
         out[name] = r
         for a in arrs:

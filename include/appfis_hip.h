@@ -258,10 +258,13 @@ int appfis_fdtd3d_candidates(int dtype, char* names, int len);
  * Field in p[iters % 2] at exit.  gosa_host (iters doubles) receives each sweep's
  * gosa.  variant PLAIN: dtype F32 or F64, reference operation order.
  * variant CHOSEN (defect correction): dtype F64 inputs; FP32 inner sweeps on the
- * correction, FP64 outer residual every `outer` sweeps (<=0: every 16).  Both tune
- * the sweep shape (planes per block, coefficient prefetch depth) on first use per
+ * correction, FP64 outer residual every `outer` sweeps (<=0: every 16).  Both run
+ * sweeps in pairs, one launch for two, where they can (PLAIN: all but the last 1 to 4,
+ * so that p0 and p1 hold the last two sweeps; CHOSEN: the inner sweeps) and tune the
+ * shape of the others (planes per block, coefficient prefetch depth) on first use per
  * shape.  APPFIS_CANDIDATE0 + i runs candidate i of appfis_himeno_candidates: the
- * PLAIN form or the defect correction with that sweep shape forced (same values).
+ * PLAIN form or the defect correction with one launch per sweep of that shape, or, for
+ * "two", in pairs (same values).
  * A plane of the grid must stay under 2 GiB.  */
 int appfis_himeno(appfis_ctx* ctx, int dtype, void* const* arrays, int nx, int ny, int nz,
                   double omega, int iters, int variant, int outer, double* gosa_host);

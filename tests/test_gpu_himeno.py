@@ -188,3 +188,41 @@ def test_himeno_every_candidate(ctx, dtype, shape):
             assert np.max(np.abs(gosa - ref_g) / ref_g) < HIMENO_DC_GOSA_RTOL
         assert np.array_equal(p, first[0]), names[i]
         assert np.allclose(gosa, first[1], rtol=1e-12, atol=0), names[i]
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("shape", [(3, 3, 3), (5, 4, 7), (65, 9, 12), (66, 40, 20), (129, 14, 33), (130, 21, 9),
+                                   (256, 8, 30), (257, 20, 70), (258, 11, 30), (300, 17, 29)])
+def test_himeno_pairs_of_sweeps(ctx, dtype, shape):
+    # the two-sweep launches: windows of 64, 128 and 256 columns with rows of one tile, of one
+    # column more and of several tiles, tiles cut short in y, chunks of a few planes; 5 sweeps
+    # are two pairs and a single one, 8 two pairs and four, 9 four pairs and one.  Random values
+    # in every array, so that p0 and p1 have different shells and each sweep must read its own.
+    # Both buffers hold what the oracle's sweeps leave, gosa to 1e-11 (sums of squares in
+    # another order: at most n * 2^-53 relative, n < 2^20 points).
+    nx, ny, nz = shape
+    rng = np.random.default_rng(nx + ny)
+    arrs = [rng.random((nz, ny, nx)).astype(dtype) for _ in range(14)]
+    arrs[5] /= 6
+    for iters in (5, 8, 9):
+        ref = [a.copy() for a in arrs]
+        ref_gosa = oracle.himeno(ref, nx, ny, nz, 0.8, iters)
+        dt = hip.F64 if dtype == np.float64 else hip.F32
+        for variant in (hip.PLAIN, hip.CANDIDATE0 + hip.himeno_candidates().index("plain two")):
+            dev = [ctx.from_numpy(a, dt) for a in arrs]
+            gosa = ctx.himeno(dev, nx, ny, nz, 0.8, iters, variant)
+            assert np.array_equal(dev[0].download(), ref[0]) and np.array_equal(dev[1].download(), ref[1])
+            assert np.allclose(gosa, ref_gosa, rtol=1e-11, atol=0)
+
+
+@pytest.mark.parametrize("shape,iters,outer", [((65, 30, 40), 37, 0), ((130, 21, 33), 20, 4), ((257, 20, 40), 18, 3)])
+def test_himeno_defect_correction_pairs(ctx, shape, iters, outer):
+    # inner sweeps in pairs between rebases (an odd one left over or not) give the same field, bit
+    # for bit, as one launch each, and gosa to 1e-12
+    nx, ny, nz = shape
+    arrs = himeno_arrays(nx, ny, nz, np.float64, seed=2001)
+    names = hip.himeno_candidates()
+    one = run_gpu(ctx, arrs, nx, ny, nz, iters, hip.CANDIDATE0 + names.index("dc zc32 d1"), outer)
+    two = run_gpu(ctx, arrs, nx, ny, nz, iters, hip.CANDIDATE0 + names.index("dc two"), outer)
+    assert np.array_equal(one[0], two[0])
+    assert np.allclose(one[1], two[1], rtol=1e-12, atol=0)
