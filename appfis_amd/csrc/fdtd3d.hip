@@ -6,7 +6,7 @@
 //   u'  = (((c0*u + c1*s_1) + c2*s_2) + c3*s_3) + c4*s_4        (no FMA contraction)
 //
 // 2.5D k-march.  A block of 64 x TY threads owns a (64*VX) x (TY*RY) column of the x-y
-// plane and a chunk of ZC planes.  Each thread owns VX x RY points of the plane and keeps
+// plane and a chunk of zc planes.  Each thread owns VX x RY points of the plane and keeps
 // a 9-deep register queue along z for each of them, so the z neighbours cost nothing;
 // the y neighbours inside the thread's own RY rows come from the same registers; only
 // the x neighbours and the y neighbours across thread rows are read from the plane
@@ -20,6 +20,9 @@
 // dtype F32 / F64: storage and arithmetic in that type.  F16 / BF16: storage only,
 // arithmetic in FP32, round-to-nearest-even on store.
 #include "common.hpp"
+
+#include <algorithm>
+#include <cmath>
 
 using namespace appfis;
 
@@ -165,8 +168,8 @@ __device__ inline void tile_of(int& bx, int& by, int& bz)
     bz = r / gy;
 }
 
-template <typename S, int VX, int TY, int RY, int ZC, int D, int U>
-__global__ __launch_bounds__(TXT* TY) void k_fdtd3d(const S* __restrict__ u, S* __restrict__ v, int nx, int ny, int nz,
+template <typename S, int VX, int TY, int RY, int D, int U>
+__global__ __launch_bounds__(TXT* TY) void k_fdtd3d(const S* __restrict__ u, S* __restrict__ v, int nx, int ny, int nz, int zc,
                                                      typename Cvt<S>::C c0, typename Cvt<S>::C c1,
                                                      typename Cvt<S>::C c2, typename Cvt<S>::C c3,
                                                      typename Cvt<S>::C c4)
@@ -192,8 +195,8 @@ __global__ __launch_bounds__(TXT* TY) void k_fdtd3d(const S* __restrict__ u, S* 
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int tid = ty * TXT + tx;
     const int bx = tbx * PX + R, by = tby * PY + R;  // padded origin of the tile
-    const int z0 = tbz * ZC + R;
-    const int z1 = min(z0 + ZC, nz + R);
+    const int z0 = tbz * zc + R;
+    const int z1 = min(z0 + zc, nz + R);
     const C cc[5] = {c0, c1, c2, c3, c4};
 
     // own point group: x = gx .. gx+VX-1, rows y = gy0 + r
@@ -380,9 +383,9 @@ __device__ inline void load_lds16(__amdgpu_buffer_rsrc_t r, void* lds, uint32_t 
     __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, off, 0, 0, 0);
 }
 
-template <typename S, int TY, int RY, int ZC, int D>
+template <typename S, int TY, int RY, int D>
 __global__ __launch_bounds__(TXT* TY) void k_fdtd3d_dma(const S* __restrict__ u, S* __restrict__ v, int nx, int ny,
-                                                         int nz, S c0, S c1, S c2, S c3, S c4)
+                                                         int nz, int zc, S c0, S c1, S c2, S c3, S c4)
 {
     static_assert(sizeof(S) == 4, "FP32 storage");
     using C = S;
@@ -408,8 +411,8 @@ __global__ __launch_bounds__(TXT* TY) void k_fdtd3d_dma(const S* __restrict__ u,
     const int plane_bytes = (int)(szl * (long long)sizeof(S));
     const int tx = threadIdx.x, ty = threadIdx.y;
     const int bx = tbx * TXT + R, by = tby * PY + R;  // padded origin of the tile
-    const int z0 = tbz * ZC + R;
-    const int z1 = min(z0 + ZC, nz + R);
+    const int z0 = tbz * zc + R;
+    const int z1 = min(z0 + zc, nz + R);
     const int zlast = z1 + R - 1;  // the last plane the chunk reads
     const C cc[5] = {c0, c1, c2, c3, c4};
     const int gx = bx + tx;
@@ -521,114 +524,162 @@ __global__ __launch_bounds__(TXT* TY) void k_fdtd3d_dma(const S* __restrict__ u,
     }
 }
 
-template <typename S, int TY, int RY, int ZC, int D>
-int run_dma(appfis_ctx* ctx, S* b0, S* b1, int nx, int ny, int nz, const double* cf, int steps)
+template <typename S, int TY, int RY, int D>
+int run_dma(appfis_ctx* ctx, S* b0, S* b1, int nx, int ny, int nz, const double* cf, int steps, int zc)
 {
-    dim3 block(TXT, TY), grid(ceil_div(nx, TXT), ceil_div(ny, TY * RY), ceil_div(nz, ZC));
+    dim3 block(TXT, TY), grid(ceil_div(nx, TXT), ceil_div(ny, TY * RY), ceil_div(nz, zc));
     S* buf[2] = {b0, b1};
     for (int s = 0; s < steps; s++) {
-        hipLaunchKernelGGL((k_fdtd3d_dma<S, TY, RY, ZC, D>), grid, block, 0, ctx->stream, buf[s & 1],
-                           buf[(s + 1) & 1], nx, ny, nz, (S)cf[0], (S)cf[1], (S)cf[2], (S)cf[3], (S)cf[4]);
+        hipLaunchKernelGGL((k_fdtd3d_dma<S, TY, RY, D>), grid, block, 0, ctx->stream, buf[s & 1], buf[(s + 1) & 1],
+                           nx, ny, nz, zc, (S)cf[0], (S)cf[1], (S)cf[2], (S)cf[3], (S)cf[4]);
         APPFIS_LAUNCH_CHECK();
     }
     return APPFIS_OK;
 }
 
-template <typename S, int VX, int TY, int RY, int ZC, int D, int U>
-int run(appfis_ctx* ctx, S* b0, S* b1, int nx, int ny, int nz, const double* cf, int steps)
+template <typename S, int VX, int TY, int RY, int D, int U>
+int run(appfis_ctx* ctx, S* b0, S* b1, int nx, int ny, int nz, const double* cf, int steps, int zc)
 {
     using C = typename Cvt<S>::C;
-    dim3 block(TXT, TY), grid(ceil_div(nx, TXT * VX), ceil_div(ny, TY * RY), ceil_div(nz, ZC));
+    dim3 block(TXT, TY), grid(ceil_div(nx, TXT * VX), ceil_div(ny, TY * RY), ceil_div(nz, zc));
     S* buf[2] = {b0, b1};
     for (int s = 0; s < steps; s++) {
-        hipLaunchKernelGGL((k_fdtd3d<S, VX, TY, RY, ZC, D, U>), grid, block, 0, ctx->stream, buf[s & 1],
-                           buf[(s + 1) & 1], nx, ny, nz, (C)cf[0], (C)cf[1], (C)cf[2], (C)cf[3], (C)cf[4]);
+        hipLaunchKernelGGL((k_fdtd3d<S, VX, TY, RY, D, U>), grid, block, 0, ctx->stream, buf[s & 1],
+                           buf[(s + 1) & 1], nx, ny, nz, zc, (C)cf[0], (C)cf[1], (C)cf[2], (C)cf[3], (C)cf[4]);
         APPFIS_LAUNCH_CHECK();
     }
     return APPFIS_OK;
 }
 
-typedef int (*fdtd_fn)(appfis_ctx*, void*, void*, int, int, int, const double*, int);
+typedef int (*fdtd_fn)(appfis_ctx*, void*, void*, int, int, int, const double*, int, int);
 struct FdtdVariant {
     const char* name;
     fdtd_fn fn;
+    int ty, ry;    // thread rows (one wave each), rows per thread: a tile is 64*vx x ty*ry points
+    int zc;        // planes per block where the candidate is forced
     bool pairs;    // 16-bit storage moved in 32-bit pairs: needs 4-byte aligned buffers
     int vx;        // x points per thread: needs nx % vx == 0 (a lane stores all vx or none)
     int wmod = 0;  // tile rows loaded as 16-byte chunks: nx + 8 a multiple of wmod, 16-byte
                    // aligned buffers (0: no such needs)
-    bool plain = false;  // PLAIN's fixed tiling where it fits (else row 0)
 };
 
-template <typename S, int VX, int TY, int RY, int ZC, int D, int U>
-int run_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const double* cf, int steps)
+template <typename S, int VX, int TY, int RY, int D, int U>
+int run_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const double* cf, int steps, int zc)
 {
-    return run<S, VX, TY, RY, ZC, D, U>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps);
+    return run<S, VX, TY, RY, D, U>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps, zc);
 }
 
-template <typename S, int TY, int RY, int ZC, int D>
-int run_dma_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const double* cf, int steps)
+template <typename S, int TY, int RY, int D>
+int run_dma_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const double* cf, int steps, int zc)
 {
-    return run_dma<S, TY, RY, ZC, D>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps);
+    return run_dma<S, TY, RY, D>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps, zc);
 }
 
-// Candidate tilings (VX x-points per thread, TY thread rows, RY rows per thread, ZC
-// planes per block, D-deep prefetch, U-step unroll: 18 rotates the queue).  Index 0 of
-// each table is the PLAIN default: the fastest measured tiling that fits any shape;
-// PLAIN takes the row marked plain instead where the shape and buffers allow it.
+// Candidate tilings (VX x-points per thread, TY thread rows, RY rows per thread, zc
+// planes per block, D-deep prefetch, U-step unroll: 18 rotates the queue).
 static const FdtdVariant kF32[] = {
-    {"vx1 ty16 ry2 zc256 d4 u4", run_v<float, 1, 16, 2, 256, 4, 4>, false, 1},
-    {"vx1 ty8 ry4 zc256 d2 u2", run_v<float, 1, 8, 4, 256, 2, 2>, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<float, 1, 4, 4, 64, 2, 2>, false, 1},
-    {"vx1 ty8 ry4 zc64 d2 u2", run_v<float, 1, 8, 4, 64, 2, 2>, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u18", run_v<float, 1, 4, 4, 64, 2, 18>, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<float, 1, 4, 2, 64, 2, 18>, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u18", run_v<float, 1, 8, 2, 64, 2, 18>, false, 1},
-    {"vx1 ty4 ry4 zc32 d2 u2", run_v<float, 1, 4, 4, 32, 2, 2>, false, 1},
-    {"vx1 ty8 ry4 zc128 d2 u2", run_v<float, 1, 8, 4, 128, 2, 2>, false, 1},
-    {"vx1 ty4 ry4 zc64 d3 u6", run_v<float, 1, 4, 4, 64, 3, 6>, false, 1},
-    {"vx1 ty16 ry2 zc64 d2 u2", run_v<float, 1, 16, 2, 64, 2, 2>, false, 1},
-    {"vx1 ty8 ry4 zc128 d3 u6", run_v<float, 1, 8, 4, 128, 3, 6>, false, 1},
-    {"vx1 ty16 ry2 zc256 d2 u2", run_v<float, 1, 16, 2, 256, 2, 2>, false, 1},
-    {"vx1 ty8 ry4 zc256 d4 u4", run_v<float, 1, 8, 4, 256, 4, 4>, false, 1},
-    {"vx1 ty8 ry4 zc256 d6 u6", run_v<float, 1, 8, 4, 256, 6, 6>, false, 1},
-    {"vx1 ty8 ry2 zc256 d4 u4", run_v<float, 1, 8, 2, 256, 4, 4>, false, 1},
-    {"vx2 ty8 ry2 zc256 d4 u4", run_v<float, 2, 8, 2, 256, 4, 4>, false, 2},
-    {"vx2 ty16 ry1 zc256 d4 u4", run_v<float, 2, 16, 1, 256, 4, 4>, false, 2},
-    {"vx2 ty16 ry1 zc256 d6 u6", run_v<float, 2, 16, 1, 256, 6, 6>, false, 2},
+    {"vx1 ty16 ry2 zc256 d4 u4", run_v<float, 1, 16, 2, 4, 4>, 16, 2, 256, false, 1},
+    {"vx1 ty8 ry4 zc256 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 256, false, 1},
+    {"vx1 ty4 ry4 zc64 d2 u2", run_v<float, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},
+    {"vx1 ty8 ry4 zc64 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 64, false, 1},
+    {"vx1 ty4 ry4 zc64 d2 u18", run_v<float, 1, 4, 4, 2, 18>, 4, 4, 64, false, 1},
+    {"vx1 ty4 ry2 zc64 d2 u18", run_v<float, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},
+    {"vx1 ty8 ry2 zc64 d2 u18", run_v<float, 1, 8, 2, 2, 18>, 8, 2, 64, false, 1},
+    {"vx1 ty4 ry4 zc32 d2 u2", run_v<float, 1, 4, 4, 2, 2>, 4, 4, 32, false, 1},
+    {"vx1 ty8 ry4 zc128 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 128, false, 1},
+    {"vx1 ty4 ry4 zc64 d3 u6", run_v<float, 1, 4, 4, 3, 6>, 4, 4, 64, false, 1},
+    {"vx1 ty16 ry2 zc64 d2 u2", run_v<float, 1, 16, 2, 2, 2>, 16, 2, 64, false, 1},
+    {"vx1 ty8 ry4 zc128 d3 u6", run_v<float, 1, 8, 4, 3, 6>, 8, 4, 128, false, 1},
+    {"vx1 ty16 ry2 zc256 d2 u2", run_v<float, 1, 16, 2, 2, 2>, 16, 2, 256, false, 1},
+    {"vx1 ty8 ry4 zc256 d4 u4", run_v<float, 1, 8, 4, 4, 4>, 8, 4, 256, false, 1},
+    {"vx1 ty8 ry4 zc256 d6 u6", run_v<float, 1, 8, 4, 6, 6>, 8, 4, 256, false, 1},
+    {"vx1 ty8 ry2 zc256 d4 u4", run_v<float, 1, 8, 2, 4, 4>, 8, 2, 256, false, 1},
+    {"vx2 ty8 ry2 zc256 d4 u4", run_v<float, 2, 8, 2, 4, 4>, 8, 2, 256, false, 2},
+    {"vx2 ty16 ry1 zc256 d4 u4", run_v<float, 2, 16, 1, 4, 4>, 16, 1, 256, false, 2},
+    {"vx2 ty16 ry1 zc256 d6 u6", run_v<float, 2, 16, 1, 6, 6>, 16, 1, 256, false, 2},
     // tiles loaded straight into LDS (k_fdtd3d_dma): "dma ty.. ry.. zc.. d.."
-    {"dma ty16 ry2 zc256 d2", run_dma_v<float, 16, 2, 256, 2>, false, 1, 4, true},
-    {"dma ty16 ry2 zc256 d3", run_dma_v<float, 16, 2, 256, 3>, false, 1, 4},
-    {"dma ty8 ry4 zc256 d2", run_dma_v<float, 8, 4, 256, 2>, false, 1, 4},
-    {"dma ty16 ry2 zc128 d2", run_dma_v<float, 16, 2, 128, 2>, false, 1, 4},
+    {"dma ty16 ry2 zc256 d2", run_dma_v<float, 16, 2, 2>, 16, 2, 256, false, 1, 4},
+    {"dma ty16 ry2 zc256 d3", run_dma_v<float, 16, 2, 3>, 16, 2, 256, false, 1, 4},
+    {"dma ty8 ry4 zc256 d2", run_dma_v<float, 8, 4, 2>, 8, 4, 256, false, 1, 4},
+    {"dma ty16 ry2 zc128 d2", run_dma_v<float, 16, 2, 2>, 16, 2, 128, false, 1, 4},
 };
 static const FdtdVariant kF64[] = {
-    {"vx1 ty8 ry2 zc256 d4 u4", run_v<double, 1, 8, 2, 256, 4, 4>, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u2", run_v<double, 1, 8, 2, 64, 2, 2>, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u2", run_v<double, 1, 4, 2, 64, 2, 2>, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<double, 1, 4, 4, 64, 2, 2>, false, 1},
-    {"vx1 ty4 ry2 zc128 d2 u2", run_v<double, 1, 4, 2, 128, 2, 2>, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<double, 1, 4, 2, 64, 2, 18>, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u18", run_v<double, 1, 8, 2, 64, 2, 18>, false, 1},
-    {"vx1 ty8 ry2 zc256 d2 u2", run_v<double, 1, 8, 2, 256, 2, 2>, false, 1},
-    {"vx1 ty4 ry4 zc256 d2 u2", run_v<double, 1, 4, 4, 256, 2, 2>, false, 1},
-    {"vx1 ty8 ry2 zc128 d2 u18", run_v<double, 1, 8, 2, 128, 2, 18>, false, 1},
-    {"vx1 ty4 ry4 zc256 d4 u4", run_v<double, 1, 4, 4, 256, 4, 4>, false, 1},
-    {"vx2 ty8 ry2 zc256 d2 u2", run_v<double, 2, 8, 2, 256, 2, 2>, false, 2},
-    {"vx2 ty16 ry1 zc256 d2 u2", run_v<double, 2, 16, 1, 256, 2, 2>, false, 2, 0, true},
-    {"vx1 ty16 ry1 zc256 d4 u4", run_v<double, 1, 16, 1, 256, 4, 4>, false, 1},
+    {"vx1 ty8 ry2 zc256 d4 u4", run_v<double, 1, 8, 2, 4, 4>, 8, 2, 256, false, 1},
+    {"vx1 ty8 ry2 zc64 d2 u2", run_v<double, 1, 8, 2, 2, 2>, 8, 2, 64, false, 1},
+    {"vx1 ty4 ry2 zc64 d2 u2", run_v<double, 1, 4, 2, 2, 2>, 4, 2, 64, false, 1},
+    {"vx1 ty4 ry4 zc64 d2 u2", run_v<double, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},
+    {"vx1 ty4 ry2 zc128 d2 u2", run_v<double, 1, 4, 2, 2, 2>, 4, 2, 128, false, 1},
+    {"vx1 ty4 ry2 zc64 d2 u18", run_v<double, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},
+    {"vx1 ty8 ry2 zc64 d2 u18", run_v<double, 1, 8, 2, 2, 18>, 8, 2, 64, false, 1},
+    {"vx1 ty8 ry2 zc256 d2 u2", run_v<double, 1, 8, 2, 2, 2>, 8, 2, 256, false, 1},
+    {"vx1 ty4 ry4 zc256 d2 u2", run_v<double, 1, 4, 4, 2, 2>, 4, 4, 256, false, 1},
+    {"vx1 ty8 ry2 zc128 d2 u18", run_v<double, 1, 8, 2, 2, 18>, 8, 2, 128, false, 1},
+    {"vx1 ty4 ry4 zc256 d4 u4", run_v<double, 1, 4, 4, 4, 4>, 4, 4, 256, false, 1},
+    {"vx2 ty8 ry2 zc256 d2 u2", run_v<double, 2, 8, 2, 2, 2>, 8, 2, 256, false, 2},
+    {"vx2 ty16 ry1 zc256 d2 u2", run_v<double, 2, 16, 1, 2, 2>, 16, 1, 256, false, 2},
+    {"vx1 ty16 ry1 zc256 d4 u4", run_v<double, 1, 16, 1, 4, 4>, 16, 1, 256, false, 1},
 };
 #define FDTD16_VARIANTS(S)                                                 \
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<S, 1, 4, 2, 64, 2, 18>, false, 1},      \
-    {"vx1 ty4 ry4 zc64 d2 u18", run_v<S, 1, 4, 4, 64, 2, 18>, false, 1},      \
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<S, 1, 4, 4, 64, 2, 2>, false, 1},        \
-    {"vx1 ty8 ry4 zc64 d2 u2", run_v<S, 1, 8, 4, 64, 2, 2>, false, 1},        \
-    {"vx2 ty4 ry4 zc64 d2 u18", run_v<S, 2, 4, 4, 64, 2, 18>, true, 2},       \
-    {"vx2 ty4 ry2 zc64 d2 u18", run_v<S, 2, 4, 2, 64, 2, 18>, true, 2},       \
-    {"vx2 ty8 ry2 zc64 d2 u18", run_v<S, 2, 8, 2, 64, 2, 18>, true, 2},       \
-    {"vx2 ty4 ry4 zc64 d2 u2", run_v<S, 2, 4, 4, 64, 2, 2>, true, 2},        \
-    {"vx2 ty8 ry2 zc128 d2 u18", run_v<S, 2, 8, 2, 128, 2, 18>, true, 2, 0, true}
+    {"vx1 ty4 ry2 zc64 d2 u18", run_v<S, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},      \
+    {"vx1 ty4 ry4 zc64 d2 u18", run_v<S, 1, 4, 4, 2, 18>, 4, 4, 64, false, 1},      \
+    {"vx1 ty4 ry4 zc64 d2 u2", run_v<S, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},        \
+    {"vx1 ty8 ry4 zc64 d2 u2", run_v<S, 1, 8, 4, 2, 2>, 8, 4, 64, false, 1},        \
+    {"vx2 ty4 ry4 zc64 d2 u18", run_v<S, 2, 4, 4, 2, 18>, 4, 4, 64, true, 2},       \
+    {"vx2 ty4 ry2 zc64 d2 u18", run_v<S, 2, 4, 2, 2, 18>, 4, 2, 64, true, 2},       \
+    {"vx2 ty8 ry2 zc64 d2 u18", run_v<S, 2, 8, 2, 2, 18>, 8, 2, 64, true, 2},       \
+    {"vx2 ty4 ry4 zc64 d2 u2", run_v<S, 2, 4, 4, 2, 2>, 4, 4, 64, true, 2},        \
+    {"vx2 ty8 ry2 zc128 d2 u18", run_v<S, 2, 8, 2, 2, 18>, 8, 2, 128, true, 2}
 static const FdtdVariant kF16[] = {FDTD16_VARIANTS(__half)};
 static const FdtdVariant kBF16[] = {FDTD16_VARIANTS(__hip_bfloat16)};
+
+// Planes per block of tiling v on an nx x ny x nz interior.  With m blocks to a CU (rounded up),
+// TY waves each, a sweep takes about
+//     max(m * TY * (zc + P), W0 * (zc + 9))
+// times a constant: the first where the CUs are busy, P the planes' worth of a block's prologue
+// (it reads 8 planes before its first and the direct-to-LDS form fills its ring), the second
+// where they are not: W0 waves keep a CU's loads in flight, fewer take as long, and the prologue
+// is then 9 planes' latency.  Fitted to sweeps with chunks of 2 to 256 planes (us):
+//     256^3 FP32, ty8 ry2 d2 u18:    zc256 115  128 61  64 34  32 28  16 29   8 30  4 34  2 46
+//     256^3 BF16, vx2 ty8 ry2 u18:   zc256 230  128 117 64 61  32 35  16 25   8 27  4 29  2 36
+//     512^3 FP32, dma ty16 ry2 d2:   zc256 213  128 243 64 253 32 269 16 303
+// A grid smaller than the chip wants chunks of a few planes; 256 planes each left a 256^3 box
+// with 32 to 64 blocks on 256 CUs.
+int planes_per_block(const FdtdVariant& v, int dtype, int num_cu, int nx, int ny, int nz)
+{
+    const double cus = num_cu > 0 ? num_cu : 256;
+    const double tiles = (double)ceil_div(nx, TXT * v.vx) * ceil_div(ny, v.ty * v.ry);
+    const double P = v.wmod ? 3.8 : 1.5;
+    const double W0 = dtype == APPFIS_F64 ? 9.0 : dtype == APPFIS_F32 ? 12.0 : 18.0;
+    int best = nz;
+    double least = 0.0;
+    for (int zc = nz; zc >= (nz < 2 ? nz : 2); zc--) {
+        const int chunks = (int)ceil_div(nz, zc);
+        if ((int)ceil_div(nz, chunks) != zc) continue;  // the same chunks in shorter blocks follow
+        const double m = std::ceil(tiles * chunks / cus);
+        const double cost = std::max(m * v.ty * (zc + P), W0 * (zc + 9.0));
+        if (least == 0.0 || cost < least) {
+            least = cost;
+            best = zc;
+        }
+    }
+    return best;
+}
+
+const FdtdVariant* find(const FdtdVariant* tab, int ntab, const char* name)
+{
+    for (int i = 0; i < ntab; i++)
+        if (strcmp(tab[i].name, name) == 0) return tab + i;
+    return tab;
+}
+
+// The name of v with zc planes per block, and v's name without its planes (what tells tilings
+// apart once the rule above sets them).
+std::string name_with(const FdtdVariant& v, int zc)
+{
+    const std::string n = v.name;
+    const size_t a = n.find("zc"), b = n.find(' ', a);
+    return n.substr(0, a) + (zc > 0 ? "zc" + std::to_string(zc) : "") + n.substr(b);
+}
 
 }  // namespace
 
@@ -680,29 +731,53 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
                            tab[i].name, tab[i].wmod);
         APPFIS_REQUIRE(fits(tab[i]), "fdtd3d: candidate %s needs nx %% %d == 0%s", tab[i].name, tab[i].vx,
                        tab[i].pairs ? " and 4-byte aligned buffers" : "");
-        return steps == 0 ? APPFIS_OK : tab[i].fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps);
+        return steps == 0 ? APPFIS_OK : tab[i].fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps, tab[i].zc);
     }
     if (steps == 0) return APPFIS_OK;
+    auto planes = [&](const FdtdVariant& v) { return planes_per_block(v, dtype, ctx->num_cu, nx, ny, nz); };
     if (variant == APPFIS_PLAIN) {
-        // a fixed tiling: the table's row marked plain where the shape and the buffers
-        // admit it, else row 0 -- one launch per sweep either way
-        int i0 = 0;
-        for (int i = 0; i < ntab; i++)
-            if (tab[i].plain && fits(tab[i])) {
-                i0 = i;
-                break;
-            }
-        return tab[i0].fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps);
+        // A fixed tiling by size and by what the shape and the buffers admit: low tiles of few
+        // rows per thread where the field is small (they make the most blocks), tall ones where
+        // it streams from memory and the tile's halo rows count.  Each with its planes by the
+        // rule above (us a sweep, this tiling / the other side of the line): FP32 256^3 ty4 27,
+        // dma 28, 320^3 76 / 61, 449^3 ty16 224, ty8 241; FP64 128^3 ty4 12.1, vx2 ty16 12.8,
+        // 200^3 30.5 / 29.2, 257^3 ty8 84, ty16 86, 321^3 165 / 148; BF16 65^3 ty4 ry2 5.2, ry4
+        // 5.6, 129^3 12.0 / 10.9, 320^3 vx2 ty4 47.8, ty8 49.5, 384^3 72.3 / 69.8.
+        const bool pair = nx % 2 == 0 && aligned4;
+        const double cells = (double)nx * ny * nz;
+        const double M = 1 << 20;
+        const char* name;
+        if (dtype == APPFIS_F32)
+            name = cells <= 16 * M                          ? "vx1 ty4 ry2 zc64 d2 u18"
+                   : (nx + 8) % 4 == 0 && aligned16         ? "dma ty16 ry2 zc256 d2"
+                   : cells <= 64 * M                        ? "vx1 ty8 ry2 zc64 d2 u18"
+                                                            : "vx1 ty16 ry2 zc256 d4 u4";
+        else if (dtype == APPFIS_F64)
+            name = cells <= (pair ? 2 : 4) * M ? "vx1 ty4 ry2 zc64 d2 u18"
+                   : pair                      ? "vx2 ty16 ry1 zc256 d2 u2"
+                   : cells <= 24 * M           ? "vx1 ty8 ry2 zc64 d2 u18"
+                                               : "vx1 ty16 ry1 zc256 d4 u4";
+        else if (pair && nx > 64)
+            name = cells <= 32 * M ? "vx2 ty4 ry2 zc64 d2 u18" : "vx2 ty8 ry2 zc128 d2 u18";
+        else
+            name = cells <= M ? "vx1 ty4 ry2 zc64 d2 u18" : "vx1 ty4 ry4 zc64 d2 u18";
+        const FdtdVariant& v = *find(tab, ntab, name);
+        return v.fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps, planes(v));
     }
-    // CHOSEN: the fastest tiling for this shape, timed once on scratch buffers.  Every
-    // candidate evaluates the same expression in the same order: results are identical.
+    // CHOSEN: the fastest tiling for this shape, each with its planes by the rule, timed once on
+    // scratch buffers.  Every candidate evaluates the same expression in the same order: results
+    // are identical.
     std::vector<int> cand;
+    std::vector<std::string> tilings, text;
+    for (int i = 0; i < ntab; i++) {
+        const std::string t = name_with(tab[i], 0);
+        if (!fits(tab[i]) || std::find(tilings.begin(), tilings.end(), t) != tilings.end()) continue;
+        cand.push_back(i);
+        tilings.push_back(t);
+        text.push_back(name_with(tab[i], planes(tab[i])));
+    }
     std::vector<const char*> names;
-    for (int i = 0; i < ntab; i++)
-        if (fits(tab[i])) {
-            cand.push_back(i);
-            names.push_back(tab[i].name);
-        }
+    for (const std::string& t : text) names.push_back(t.c_str());
     const int key[6] = {3, dtype, nx, ny, nz, aligned16 ? 2 : aligned4 ? 1 : 0};
     int pick = 0;
     const size_t bytes = (size_t)(nx + 8) * (ny + 8) * (nz + 8) * dtype_size(dtype);
@@ -722,7 +797,7 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
         APPFIS_HIP_CHECK(hipMemsetAsync(ctx->work, 0, 2 * half, ctx->stream));
     }
     st = tune_select(ctx, key, (int)cand.size(), names.data(),
-                     [&](int i) { return tab[cand[i]].fn(ctx, s0, s1, nx, ny, nz, coeff5, 2); }, 3, &pick);
+                     [&](int i) { return tab[cand[i]].fn(ctx, s0, s1, nx, ny, nz, coeff5, 2, planes(tab[cand[i]])); }, 3, &pick);
     if (st) return st;
-    return tab[cand[pick]].fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps);
+    return tab[cand[pick]].fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps, planes(tab[cand[pick]]));
 }

@@ -399,17 +399,14 @@ def _plan(iters, ts):
 
 
 
-# the PLAIN form's preferred fixed tilings (the library's rows marked plain), used where
-# the shape admits them: the bench's buffers are 256-byte aligned and n = 512
+# the PLAIN form's fixed tilings at 512^3 on 256-byte aligned buffers
 FDTD_PLAIN_PREFERRED = {"f32": "dma ty16 ry2 zc256 d2", "f64": "vx2 ty16 ry1 zc256 d2 u2",
                         "f16": "vx2 ty8 ry2 zc128 d2 u18", "bf16": "vx2 ty8 ry2 zc128 d2 u18"}
 
 
 def _fdtd_plain(hip, name, dt, n):
-    """The PLAIN form's fixed tiling at n^3: the preferred row where it fits (F32: n + 8
-    a multiple of 4; the others: n even), else the table's row 0."""
-    fits = (n + 8) % 4 == 0 if name == "f32" else n % 2 == 0
-    return FDTD_PLAIN_PREFERRED[name] if fits else hip.fdtd3d_candidates(dt)[0]
+    """The PLAIN form's fixed tiling at n^3 (a name of appfis_fdtd3d_candidates)."""
+    return FDTD_PLAIN_PREFERRED[name]
 
 
 FDTD_CTYPE = {"f32": "float", "f64": "double", "f16": "__half", "bf16": "__hip_bfloat16"}
@@ -432,11 +429,11 @@ def bench_fdtd(ctx, hip, n=512, steps=100):
             if tname.startswith("dma "):  # direct-to-LDS form: "dma ty16 ry2 zc256 d2"
                 ty, ry, zc, dd = (int(t[2:]) if t[:2] in ("ty", "ry", "zc") else int(t[1:])
                                   for t in tname.split()[1:])
-                kname = f"k_fdtd3d_dma<{FDTD_CTYPE[name]}, {ty}, {ry}, {zc}, {dd}>"
+                kname = f"k_fdtd3d_dma<{FDTD_CTYPE[name]}, {ty}, {ry}, {dd}>"
             else:
                 vx, ty, ry, zc, dd, uu = (int(t[2:]) if t[:2] in ("vx", "ty", "ry", "zc") else int(t[1:])
                                           for t in tname.split())
-                kname = f"k_fdtd3d<{FDTD_CTYPE[name]}, {vx}, {ty}, {ry}, {zc}, {dd}, {uu}>"
+                kname = f"k_fdtd3d<{FDTD_CTYPE[name]}, {vx}, {ty}, {ry}, {dd}, {uu}>"
             out[f"{name}_{form}"] = {"ms": round(ms, 3), "glups": round(n ** 3 * steps / (ms * 1e-3) / 1e9, 2),
                                      "tiling": tname, "roofline": roofline(float(bpl) * n ** 3, ms / steps, kname)}
             if form == "chosen":

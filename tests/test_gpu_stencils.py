@@ -372,6 +372,23 @@ def test_fdtd3d_every_candidate_bit_exact(ctx, dt, n):
     assert ran >= 2
 
 
+@pytest.mark.parametrize("dt", [hip.F32, hip.F64, hip.F16, hip.BF16])
+@pytest.mark.parametrize("n", [(5, 3, 1), (66, 9, 2), (100, 101, 103), (127, 131, 140), (162, 161, 163), (257, 257, 260),
+                               (256, 264, 260), (301, 330, 340), (321, 330, 640)])
+def test_fdtd3d_tilings_by_size(ctx, dt, n):
+    # the fixed tiling and the planes per block follow the grid: one plane, chunks of two, and
+    # sizes on either side of 1, 2, 4, 16, 24, 32 and 64 million points, even and odd widths
+    nx, ny, nz = n
+    if nx * ny * nz > 60e6 and dt == hip.F64:
+        pytest.skip("the FP64 lines all lie below")
+    coeff = FDTD_COEFF if dt != hip.F16 else [c / 2.0625 for c in FDTD_COEFF]
+    a, d0, d1 = _fdtd_pair(ctx, n, dt)
+    ref = oracle.fdtd3d(a.copy(), np.zeros_like(a), nx, ny, nz, coeff, 1, bf16=(dt == hip.BF16))
+    for variant in (hip.PLAIN, hip.CHOSEN):
+        ctx.fdtd3d(d0, d1, nx, ny, nz, coeff, 1, variant)
+        assert np.array_equal(d1.download(), ref)
+
+
 @pytest.mark.parametrize("dt,off", [(hip.F32, 4), (hip.F64, 8), (hip.F16, 2), (hip.BF16, 2)])
 def test_fdtd3d_on_unaligned_buffers(ctx, dt, off):
     # buffers that start `off` bytes into an allocation, so that the preferred tilings'
