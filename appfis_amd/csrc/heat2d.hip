@@ -2,18 +2,19 @@
 // HeatDiffusion/src/heat_appfis.hpp:166-174, driven like heat_appfis.hpp:86-91 on a
 // DUAL grid: sweep, then Grid::Swap).
 //
-//   u' = u + c*((((uN + uS) + uE) + uW) - 4u)      one rounding per operation, no FMA
+//   u' = u + c*((((uN + uS) + uE) + uW) - 4u)      each operation rounded
 //
 // PLAIN : one sweep per launch, one output per thread, x along the wave.
-// CHOSEN: temporal blocking.  A block loads a window of the field with a T-cell halo
-//         and advances it T sweeps on chip, then writes the window's centre; the valid
-//         region shrinks by one cell per sweep.  Two window forms are autotuned: in LDS
-//         (k_heat2d_tb) and in registers with DPP neighbours (k_heat2d_rt).  Dirichlet
-//         ghost cells are loaded and never updated, exactly as in the one-sweep form, so
-//         every interior value is bit-identical to PLAIN.  HBM/MALL traffic per sweep
-//         drops by ~T.
+// CHOSEN: temporal blocking.  A block loads a window of the field with a T-cell halo into
+//         registers and advances it T sweeps there, then writes the window's centre; the
+//         valid region shrinks by one cell per sweep (k_heat2d_rt; k_heat2d_whole is the
+//         window that holds a whole small grid and needs no halo).  Dirichlet ghost cells
+//         are loaded and never updated, exactly as in the one-sweep form, so every interior
+//         value is bit-identical to PLAIN.  HBM/MALL traffic per sweep drops by ~T.
 #include "common.hpp"
 
+#include <cmath>
+#include <type_traits>
 #include <vector>
 
 using namespace appfis;
@@ -57,78 +58,6 @@ __global__ __launch_bounds__(256) void k_heat2d_plain(const T* __restrict__ u, T
     }
 }
 
-// Temporal blocking: TX x TY output tile, TS sweeps per launch, NT threads.
-// One TX x TY output tile (tile coordinates tbx, tby) of one grid, `steps` <= TS sweeps.
-template <typename T, int TX, int TY, int TS, int NT>
-__device__ inline void tb_tile(const T* __restrict__ u, T* __restrict__ v, int nx, int ny, T c, int steps, int tbx,
-                               int tby)
-{
-    constexpr int RX = TX + 2 * TS, RY = TY + 2 * TS;
-    constexpr int NCELL = RX * RY;
-    constexpr int PER = (NCELL + NT - 1) / NT;
-    __shared__ T tile[RY][RX];
-    const int W = nx + 2, H = ny + 2;
-    // window origin in padded coordinates (may be negative / past the array)
-    const int gx0 = tbx * TX + 1 - TS;
-    const int gy0 = tby * TY + 1 - TS;
-    const int tid = threadIdx.x;
-    for (int p = tid; p < NCELL; p += NT) {
-        int ly = p / RX, lx = p - ly * RX;
-        int gx = gx0 + lx, gy = gy0 + ly;
-        T val = (T)0;
-        if (gx >= 0 && gx < W && gy >= 0 && gy < H) val = u[(size_t)gx + (size_t)W * (size_t)gy];
-        tile[ly][lx] = val;
-    }
-    __syncthreads();
-    T nv[PER];
-    for (int s = 0; s < steps; s++) {
-        // cells at distance >= s+1 from the window edge can be advanced to sweep s+1
-        const int lo = s + 1, hx = RX - s - 1, hy = RY - s - 1;
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            int p = tid + q * NT;
-            int ly = p / RX, lx = p - ly * RX;
-            int gx = gx0 + lx, gy = gy0 + ly;
-            bool active = p < NCELL && lx >= lo && lx < hx && ly >= lo && ly < hy && gx >= 1 && gx <= nx &&
-                          gy >= 1 && gy <= ny;
-            if (active) {
-                const T uc = tile[ly][lx];
-                T sum = tile[ly - 1][lx] + tile[ly + 1][lx];
-                sum = sum + tile[ly][lx + 1];
-                sum = sum + tile[ly][lx - 1];
-                sum = sum - (T)4 * uc;
-                nv[q] = uc + c * sum;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < PER; q++) {
-            int p = tid + q * NT;
-            int ly = p / RX, lx = p - ly * RX;
-            int gx = gx0 + lx, gy = gy0 + ly;
-            bool active = p < NCELL && lx >= lo && lx < hx && ly >= lo && ly < hy && gx >= 1 && gx <= nx &&
-                          gy >= 1 && gy <= ny;
-            if (active) tile[ly][lx] = nv[q];
-        }
-        __syncthreads();
-    }
-    // write the TX x TY centre (interior cells only)
-    for (int p = tid; p < TX * TY; p += NT) {
-        int ly = p / TX, lx = p - ly * TX;
-        int gx = tbx * TX + 1 + lx, gy = tby * TY + 1 + ly;
-        if (gx <= nx && gy <= ny) v[(size_t)gx + (size_t)W * (size_t)gy] = tile[ly + TS][lx + TS];
-    }
-}
-
-template <typename T, int TX, int TY, int TS, int NT>
-__global__ __launch_bounds__(NT) void k_heat2d_tb(const T* __restrict__ u, T* __restrict__ v, int nx, int ny, T c,
-                                                  int steps)
-{
-    const unsigned nbx = gridDim.x;
-    const unsigned t = xcd_tile(blockIdx.x + nbx * blockIdx.y, nbx * gridDim.y);
-    tb_tile<T, TX, TY, TS, NT>(u, v, nx, ny, c, steps, (int)(t % nbx), (int)(t / nbx));
-}
-
 // Ensemble: grid s owns tiles tile0 .. tile0 + tiles_x * tiles_y - 1 of one launch.
 template <typename T>
 struct HeatGrid {
@@ -161,34 +90,55 @@ __device__ inline int grid_of_tile(const HeatGrid<T>* __restrict__ tab, int ngri
 // last), which spoils one more ring per sweep; after TS sweeps the centre
 // (64*WPL-2TS) x (NW*K-2TS) is exact.  Ghost cells keep their loaded values, so every
 // interior value equals the one-sweep form's.
-template <typename T, int K, int NW, int TS, int WPL>
-__device__ inline void rt_tile(const T* __restrict__ u, T* __restrict__ v, int nx, int ny, T c, int steps, int tbx,
-                               int tby)
+//
+// The adds and multiplies bound it, so a cell does no more of anything than it needs: a block whose
+// window is all interior skips the selects, and rt_tile is forced inline (as a call, which two
+// callers made of it, the cells went through the calling convention's registers and scratch:
+// 120 registers for 7 x 1 cells, 53 inlined).  Further, 1024^2 on 256 CUs, us per sweep, the
+// 96 x 48 tile of 16 sweeps:
+//   FP64: sum - 4u as one FMA, 1.24 -> 1.20 (of these 0.02 are the check).  4u is exact where it
+//   does not overflow, so the FMA then rounds as the subtraction does.  `big` is the top word of a
+//   magnitude that the launch's sweeps cannot grow that far from; a block that loaded a larger one,
+//   an infinity or a NaN does its sweeps again with a multiply and a subtraction.
+//   FP32: a row's update starts when the row two above it is done (an empty asm that takes both),
+//   which keeps the schedule from stretching over the whole column of rows: 0.889 -> 0.868, and
+//   2048^2 2.035 -> 1.978.  In FP64 the same costs 1 %, and the FMA's check costs FP32 5 %.
+template <typename T, int K, int NW, int TS, int WPL, bool WHOLE>
+__device__ __forceinline__ void rt_tile(const T* __restrict__ u, T* __restrict__ v, int nx, int ny, T c, int steps,
+                               unsigned big, int tbx, int tby)
 {
     constexpr int TX = 64 * WPL - 2 * TS, TY = NW * K - 2 * TS;
-    static_assert(TX > 0 && TY > 0, "the window must be wider and taller than its halo");
+    static_assert(WHOLE || (TX > 0 && TY > 0), "the window must be wider and taller than its halo");
     __shared__ T edge[2][NW][2][WPL][64];
+    constexpr bool kFused = sizeof(T) == 8;
+    __shared__ int large[kFused ? NW : 1];
     const gmem<T>* ug = to_global(u);  // the ensemble reads u and v from its grid table
     gmem<T>* vg = to_global(v);
     const int W = nx + 2, H = ny + 2;
-    const int lane = (int)(threadIdx.x & 63), wv = (int)(threadIdx.x >> 6);
-    const int gx0 = tbx * TX + 1 - TS + WPL * lane;  // padded column of R[.][0]
-    const int gy0 = tby * TY + 1 - TS + wv * K;      // padded row of R[0][.]
+    const int lane = (int)(threadIdx.x & 63);
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int wx0 = WHOLE ? 0 : tbx * TX + 1 - TS;  // padded column and row of the window
+    const int wy0 = WHOLE ? 0 : tby * TY + 1 - TS;
+    const int gx0 = wx0 + WPL * lane;  // of R[.][0]
+    const int gy0 = wy0 + wv * K;      // of R[0][.]
     bool col_in[WPL];
 #pragma unroll
     for (int w = 0; w < WPL; w++) col_in[w] = gx0 + w >= 1 && gx0 + w <= nx;
     T R[K][WPL];
+    auto load = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int k = 0; k < K; k++) {
-        const int gy = gy0 + k;
+        for (int k = 0; k < K; k++) {
+            const int gy = gy0 + k;
 #pragma unroll
-        for (int w = 0; w < WPL; w++) {
-            const int gx = gx0 + w;
-            R[k][w] = (gx >= 0 && gx < W && gy >= 0 && gy < H) ? ug[(size_t)gx + (size_t)W * (size_t)gy] : (T)0;
+            for (int w = 0; w < WPL; w++) {
+                const int gx = gx0 + w;
+                R[k][w] = (gx >= 0 && gx < W && gy >= 0 && gy < H) ? ug[(size_t)gx + (size_t)W * (size_t)gy] : (T)0;
+            }
         }
-    }
+    };
+    load();
     // one sweep; its edge rows use LDS slot b (sweeps alternate slots)
-    auto sweep = [&](const int b) {
+    auto sweep = [&](auto masked, auto fused, const int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int w = 0; w < WPL; w++) {
             edge[b][wv][0][w][lane] = R[0][w];
@@ -218,56 +168,97 @@ __device__ inline void rt_tile(const T* __restrict__ u, T* __restrict__ v, int n
                 T sum = above[w] + (k == K - 1 ? dn[w] : R[k + 1][w]);
                 sum = sum + (w == WPL - 1 ? east : R[k][w + 1]);
                 sum = sum + (w == 0 ? west : R[k][w - 1]);
-                sum = sum - (T)4 * uc;
-                nv[w] = (col_in[w] && row_in) ? uc + c * sum : uc;
+                if constexpr (decltype(fused)::value) sum = __builtin_elementwise_fma((T)-4, uc, sum);
+                else sum = sum - (T)4 * uc;
+                const T next = uc + c * sum;
+                nv[w] = !decltype(masked)::value || (col_in[w] && row_in) ? next : uc;
             }
 #pragma unroll
             for (int w = 0; w < WPL; w++) {
                 above[w] = R[k][w];
                 R[k][w] = nv[w];
             }
+            // FP32 only (see above): row k + 2 waits for row k
+            if constexpr (!kFused)
+                if (k + 2 < K)
+#pragma unroll
+                    for (int w = 0; w < WPL; w++) asm volatile("" : "+v"(R[k + 2][w]) : "v"(nv[w]));
         }
     };
     // two sweeps per trip, so that the registers of consecutive sweeps are renamed
     // rather than copied
-    for (int s = 0; s + 1 < steps; s += 2) {
-        sweep(0);
-        sweep(1);
+    auto sweeps = [&](auto masked, auto fused) __attribute__((always_inline)) {
+        for (int s = 0; s + 1 < steps; s += 2) {
+            sweep(masked, fused, 0);
+            sweep(masked, fused, 1);
+        }
+        if (steps & 1) sweep(masked, fused, 0);
+    };
+    if constexpr (kFused) {
+        unsigned top = 0;
+#pragma unroll
+        for (int k = 0; k < K; k++)
+#pragma unroll
+            for (int w = 0; w < WPL; w++) top = max(top, (unsigned)__double2hiint(R[k][w]) & 0x7fffffffu);
+        const bool wave_large = __any(top >= big);
+        if (lane == 0) large[wv] = wave_large;  // read after the sweeps: their barriers order it
     }
-    if (steps & 1) sweep(0);
-    // the centre: window columns TS .. TS+TX-1, rows TS .. TS+TY-1 (interior cells only)
+    const bool inner = wx0 >= 1 && wx0 + 64 * WPL - 1 <= nx && wy0 >= 1 && wy0 + NW * K - 1 <= ny;
+    if (inner) sweeps(std::false_type{}, std::bool_constant<kFused>{});
+    else sweeps(std::true_type{}, std::bool_constant<kFused>{});
+    if constexpr (kFused)
+        if (__any(large[lane % NW])) {
+            __syncthreads();  // the last sweep's edge rows have been read
+            load();
+            sweeps(std::true_type{}, std::false_type{});
+        }
+    // the centre: window columns TS .. TS+TX-1, rows TS .. TS+TY-1 (interior cells only).  The
+    // column is made opaque: the loads' addresses would be kept in registers for the stores.
+    int sx0 = gx0;
+    asm volatile("" : "+v"(sx0));
 #pragma unroll
     for (int k = 0; k < K; k++) {
         const int r = wv * K + k, gy = gy0 + k;
-        if (r < TS || r >= TS + TY || gy < 1 || gy > ny) continue;
+        if ((!WHOLE && (r < TS || r >= TS + TY)) || gy < 1 || gy > ny) continue;
 #pragma unroll
         for (int w = 0; w < WPL; w++) {
             const int lx = WPL * lane + w;
-            if (lx >= TS && lx < TS + TX && col_in[w]) vg[(size_t)(gx0 + w) + (size_t)W * (size_t)gy] = R[k][w];
+            if ((WHOLE || (lx >= TS && lx < TS + TX)) && sx0 + w >= 1 && sx0 + w <= nx)
+                vg[(size_t)(sx0 + w) + (size_t)W * (size_t)gy] = R[k][w];
         }
     }
 }
 
 template <typename T, int K, int NW, int TS, int WPL>
 __global__ __launch_bounds__(64 * NW) void k_heat2d_rt(const T* __restrict__ u, T* __restrict__ v, int nx, int ny,
-                                                       T c, int steps)
+                                                       T c, int steps, unsigned big)
 {
     constexpr int TX = 64 * WPL - 2 * TS;
     const int tiles_x = (nx + TX - 1) / TX;
     const int t = (int)xcd_tile(blockIdx.x, gridDim.x);
     const int tby = t / tiles_x;
-    rt_tile<T, K, NW, TS, WPL>(u, v, nx, ny, c, steps, t - tby * tiles_x, tby);
+    rt_tile<T, K, NW, TS, WPL, false>(u, v, nx, ny, c, steps, big, t - tby * tiles_x, tby);
+}
+
+// A grid that fits one block's window, ghost ring included, needs no halo: its cells at the
+// window's edge are ghost cells, which keep their values, so any number of sweeps runs in one
+// launch of one block.
+template <typename T, int K, int NW, int WPL>
+__global__ __launch_bounds__(64 * NW) void k_heat2d_whole(const T* __restrict__ u, T* __restrict__ v, int nx, int ny,
+                                                          T c, int steps, unsigned big)
+{
+    rt_tile<T, K, NW, 0, WPL, true>(u, v, nx, ny, c, steps, big, 0, 0);
 }
 
 template <typename T, int K, int NW, int TS, int WPL>
 __global__ __launch_bounds__(64 * NW) void k_heat2d_rt_ens(const HeatGrid<T>* __restrict__ tab, int ngrid, int par,
-                                                           T c, int steps)
+                                                           T c, int steps, unsigned big)
 {
     const int tile = (int)xcd_tile(blockIdx.x, gridDim.x);
     const HeatGrid<T>& G = tab[grid_of_tile(tab, ngrid, tile)];
     const int t = tile - G.tile0;
     const int tby = t / G.tiles_x;
-    rt_tile<T, K, NW, TS, WPL>(G.b[par], G.b[par ^ 1], G.nx, G.ny, c, steps, t - tby * G.tiles_x, tby);
+    rt_tile<T, K, NW, TS, WPL, false>(G.b[par], G.b[par ^ 1], G.nx, G.ny, c, steps, big, t - tby * G.tiles_x, tby);
 }
 
 constexpr int PLAIN_RY = 4;
@@ -299,29 +290,16 @@ inline int plan_launches(int iters, int ts, int* counts, int max_launches)
     return n;
 }
 
-template <typename T, int TX, int TY, int TS, int NT>
-int run_tb(appfis_ctx* ctx, T* b0, T* b1, int nx, int ny, T c, int iters, int depth)
+// The top word of an FP64 magnitude below which all stay under a quarter of the largest double
+// through `steps` sweeps: a sweep multiplies the largest magnitude by at most |1 - 4c| + 4|c|
+// and its roundings.  0 (no magnitude is below it) where there is none.
+inline unsigned fused_limit(double c, int steps)
 {
-    T* buf[2] = {b0, b1};
-    dim3 grid(ceil_div(nx, TX), ceil_div(ny, TY));
-    std::vector<int> counts((size_t)iters);
-    int n = plan_launches(iters, depth < TS ? depth : TS, counts.data(), iters);
-    if (n <= 0) return invalid("heat2d: cannot split %d sweeps", iters);
-    for (int l = 0; l < n; l++) {
-        hipLaunchKernelGGL((k_heat2d_tb<T, TX, TY, TS, NT>), grid, dim3(NT), 0, ctx->stream, buf[l & 1],
-                           buf[(l + 1) & 1], nx, ny, c, counts[l]);
-        APPFIS_LAUNCH_CHECK();
-    }
-    return APPFIS_OK;
+    const double e = 1020.0 - steps * (std::log2(std::fabs(1.0 - 4.0 * c) + 4.0 * std::fabs(c)) + 1e-9);
+    return e > -1000.0 ? (unsigned)(1023 + (int)std::floor(e)) << 20 : 0;
 }
 
-template <typename T, int TX, int TY, int TS, int NT = 256>
-int run_tb_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, double c, int iters, int depth)
-{
-    return run_tb<T, TX, TY, TS, NT>(ctx, (T*)b0, (T*)b1, nx, ny, (T)c, iters, depth);
-}
-
-template <typename T, int K, int NW, int TS, int WPL = 1>
+template <typename T, int K, int NW, int TS, int WPL>
 int run_rt(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, double c, int iters, int depth)
 {
     constexpr int TX = 64 * WPL - 2 * TS, TY = NW * K - 2 * TS;
@@ -333,7 +311,31 @@ int run_rt(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, double c, int it
     if (n <= 0) return invalid("heat2d: cannot split %d sweeps", iters);
     for (int l = 0; l < n; l++) {
         hipLaunchKernelGGL((k_heat2d_rt<T, K, NW, TS, WPL>), dim3((unsigned)tiles), dim3(64 * NW), 0, ctx->stream,
-                           buf[l & 1], buf[(l + 1) & 1], nx, ny, (T)c, counts[l]);
+                           buf[l & 1], buf[(l + 1) & 1], nx, ny, (T)c, counts[l],
+                           fused_limit(c, counts[l]));
+        APPFIS_LAUNCH_CHECK();
+    }
+    return APPFIS_OK;
+}
+
+// Grids that fit the window of one block with K rows in each of NW waves.
+template <int K, int NW, int WPL>
+constexpr bool whole_fits(int nx, int ny)
+{
+    return nx <= 64 * WPL - 2 && ny <= NW * K - 2;
+}
+
+// The whole grid in one block where it fits; else the first tiles of the tables below.
+template <typename T, int K, int NW, int WPL>
+int run_whole(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, double c, int iters, int)
+{
+    if (!whole_fits<K, NW, WPL>(nx, ny)) return run_rt<T, 8, 8, 8, 1>(ctx, b0, b1, nx, ny, c, iters, 8);
+    T* buf[2] = {(T*)b0, (T*)b1};
+    const int n = iters & 1 ? 1 : 2;  // launches: their number has the parity of `iters`
+    for (int l = 0; l < n; l++) {
+        const int steps = n == 1 ? iters : iters / 2;
+        hipLaunchKernelGGL((k_heat2d_whole<T, K, NW, WPL>), dim3(1), dim3(64 * NW), 0, ctx->stream, buf[l & 1],
+                           buf[(l + 1) & 1], nx, ny, (T)c, steps, fused_limit(c, steps));
         APPFIS_LAUNCH_CHECK();
     }
     return APPFIS_OK;
@@ -345,48 +347,29 @@ struct HeatVariant {
     int ts;  // sweeps per launch at most
 };
 
-// temporal-blocking candidates (output tile TX x TY, TS sweeps per launch, NT threads).
-// A launch costs a fixed load of its (TX+2TS) x (TY+2TS) windows plus a per-sweep part;
-// larger tiles load less redundant window per output cell, and enough threads keep the
-// per-sweep part short.
-static const HeatVariant kHeatF64[] = {
-    {"tb 32x32 ts8 nt256", run_tb_v<double, 32, 32, 8>, 8},
-    {"tb 32x32 ts4 nt256", run_tb_v<double, 32, 32, 4>, 4},
-    {"tb 64x32 ts8 nt256", run_tb_v<double, 64, 32, 8>, 8},
-    {"tb 64x32 ts12 nt256", run_tb_v<double, 64, 32, 12>, 12},
-    {"tb 64x64 ts8 nt1024", run_tb_v<double, 64, 64, 8, 1024>, 8},
-    {"tb 64x64 ts12 nt1024", run_tb_v<double, 64, 64, 12, 1024>, 12},
-    {"tb 64x32 ts8 nt512", run_tb_v<double, 64, 32, 8, 512>, 8},
-    {"tb 64x32 ts16 nt256", run_tb_v<double, 64, 32, 16>, 16},
-    // register tiles, named by output tile: 64 - 2TS columns x NW*K - 2TS rows (at 1024^2
-    // each fills at most 256 blocks, one per CU)
-    {"rt 48x96 ts8 k7 w16", run_rt<double, 7, 16, 8>, 8},
-    {"rt 48x96 ts8 k14 w8", run_rt<double, 14, 8, 8>, 8},
-    {"rt 56x88 ts4 k6 w16", run_rt<double, 6, 16, 4>, 4},
-    {"rt 40x120 ts12 k9 w16", run_rt<double, 9, 16, 12>, 12},
-    {"rt 32x128 ts16 k10 w16", run_rt<double, 10, 16, 16>, 16},
-    // two blocks per CU at 1024^2 (one computes while the other waits at its barrier)
-    {"rt 48x48 ts8 k4 w16", run_rt<double, 4, 16, 8>, 8},
-    // two columns per lane: one horizontal neighbour of each cell is in the lane's
-    // registers (at 1024^2 it loses to one column per lane: 0.064 against 0.060 ms)
-    {"rt2 112x48 ts8 k4 w16", run_rt<double, 4, 16, 8, 2>, 8},
+// Temporal-blocking candidates (output tile TX x TY, TS sweeps per launch, K rows in each of NW
+// waves; "rt2": two columns per lane).  A launch costs about 5 us before its first sweep's worth of
+// work, and tiles load and compute a halo of TS cells around their output, so small grids take
+// small tiles of 8 sweeps (512^2 FP64: 48x24 0.89 us per sweep, 96x48 1.19), and grids of about one
+// block per CU deep ones (1024^2: 96x48 1.20, 48x48 1.32).  Beyond that the adds decide
+// (4096^2 FP64: 48x96 k14 10.3, k7 14.5, 96x48 over 12.2).  "whole" needs no halo: 62^2
+// takes 0.82 in one block, 1.04 in 48x24 tiles.  A fixed depth takes the first entry that
+// holds it.
+template <typename T>
+static const HeatVariant kHeat[] = {
+    {"rt 48x48 ts8 k8 w8", run_rt<T, 8, 8, 8, 1>, 8},
+    {"rt 48x96 ts8 k7 w16", run_rt<T, 7, 16, 8, 1>, 8},
+    {"rt 48x96 ts8 k14 w8", run_rt<T, 14, 8, 8, 1>, 8},
+    {"rt 48x24 ts8 k5 w8", run_rt<T, 5, 8, 8, 1>, 8},
+    {"rt 48x32 ts8 k6 w8", run_rt<T, 6, 8, 8, 1>, 8},
+    {"rt 48x48 ts8 k4 w16", run_rt<T, 4, 16, 8, 1>, 8},
+    {"rt2 112x48 ts8 k8 w8", run_rt<T, 8, 8, 8, 2>, 8},
+    {"rt 40x72 ts12 k12 w8", run_rt<T, 12, 8, 12, 1>, 12},
+    {"rt2 104x56 ts12 k5 w16", run_rt<T, 5, 16, 12, 2>, 12},
+    {"rt2 96x48 ts16 k5 w16", run_rt<T, 5, 16, 16, 2>, 16},
+    {"whole 64x80 k5 w16", run_whole<T, 5, 16, 1>, 0},
 };
-static const HeatVariant kHeatF32[] = {
-    {"tb 64x32 ts8 nt256", run_tb_v<float, 64, 32, 8>, 8},
-    {"tb 32x32 ts4 nt256", run_tb_v<float, 32, 32, 4>, 4},
-    {"tb 64x64 ts8 nt256", run_tb_v<float, 64, 64, 8>, 8},
-    {"tb 64x64 ts16 nt256", run_tb_v<float, 64, 64, 16>, 16},
-    {"tb 64x64 ts8 nt1024", run_tb_v<float, 64, 64, 8, 1024>, 8},
-    {"tb 64x64 ts16 nt1024", run_tb_v<float, 64, 64, 16, 1024>, 16},
-    {"tb 128x64 ts16 nt1024", run_tb_v<float, 128, 64, 16, 1024>, 16},
-    {"rt 48x96 ts8 k7 w16", run_rt<float, 7, 16, 8>, 8},
-    {"rt 48x96 ts8 k14 w8", run_rt<float, 14, 8, 8>, 8},
-    {"rt 56x88 ts4 k6 w16", run_rt<float, 6, 16, 4>, 4},
-    {"rt 40x120 ts12 k9 w16", run_rt<float, 9, 16, 12>, 12},
-    {"rt 32x128 ts16 k10 w16", run_rt<float, 10, 16, 16>, 16},
-    {"rt 48x48 ts8 k4 w16", run_rt<float, 4, 16, 8>, 8},
-    {"rt2 112x48 ts8 k4 w16", run_rt<float, 4, 16, 8, 2>, 8},
-};
+constexpr int kHeatCount = (int)(sizeof(kHeat<double>) / sizeof(kHeat<double>[0]));
 
 }  // namespace
 
@@ -406,16 +389,15 @@ extern "C" int appfis_heat2d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
     }
     if (variant == APPFIS_CHOSEN) {
         if (dtype != APPFIS_F64 && dtype != APPFIS_F32) return invalid("heat2d: dtype must be F64 or F32");
-        const HeatVariant* tab = dtype == APPFIS_F64 ? kHeatF64 : kHeatF32;
-        const int ntab = dtype == APPFIS_F64 ? (int)(sizeof(kHeatF64) / sizeof(kHeatF64[0]))
-                                             : (int)(sizeof(kHeatF32) / sizeof(kHeatF32[0]));
+        const HeatVariant* tab = dtype == APPFIS_F64 ? kHeat<double> : kHeat<float>;
         if (tsteps > 0) {
             // caller-fixed depth: the first candidate that holds that many sweeps per launch
-            for (int i = 0; i < ntab; i++)
+            for (int i = 0; i < kHeatCount; i++)
                 if (tab[i].ts >= tsteps) return tab[i].fn(ctx, buf0, buf1, nx, ny, c, iters, tsteps);
             return invalid("heat2d: tsteps %d exceeds the deepest temporal blocking (16)", tsteps);
         }
-        // autotuned tile shape and depth, timed once per shape on scratch buffers; every
+        // autotuned tile shape and depth, timed once per shape on scratch buffers over 96 sweeps
+        // (an even number of full launches at depths 8, 12 and 16 alike); every
         // candidate computes the same values in the same order
         const int key[6] = {1, dtype, nx, ny, 0, 0};
         bool cached = false;
@@ -432,34 +414,33 @@ extern "C" int appfis_heat2d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
             s1 = (char*)ctx->work + half;
             APPFIS_HIP_CHECK(hipMemsetAsync(ctx->work, 0, 2 * half, ctx->stream));
         }
+        // every candidate that differs here: "whole", the last, only where the grid fits it
+        const int ntab = whole_fits<5, 16, 1>(nx, ny) ? kHeatCount : kHeatCount - 1;
         std::vector<const char*> names;
         for (int i = 0; i < ntab; i++) names.push_back(tab[i].name);
         int pick = 0;
         int st = tune_select(ctx, key, ntab, names.data(),
-                             [&](int i) { return tab[i].fn(ctx, s0, s1, nx, ny, c, 48, tab[i].ts); }, 3, &pick);
+                             [&](int i) { return tab[i].fn(ctx, s0, s1, nx, ny, c, 96, tab[i].ts); }, 3, &pick);
         if (st) return st;
         return tab[pick].fn(ctx, buf0, buf1, nx, ny, c, iters, tab[pick].ts);
     }
     if (variant >= APPFIS_CANDIDATE0) {
         if (dtype != APPFIS_F64 && dtype != APPFIS_F32) return invalid("heat2d: dtype must be F64 or F32");
-        const HeatVariant* tab = dtype == APPFIS_F64 ? kHeatF64 : kHeatF32;
-        const int ntab = dtype == APPFIS_F64 ? (int)(sizeof(kHeatF64) / sizeof(kHeatF64[0]))
-                                             : (int)(sizeof(kHeatF32) / sizeof(kHeatF32[0]));
+        const HeatVariant* tab = dtype == APPFIS_F64 ? kHeat<double> : kHeat<float>;
         const int i = variant - APPFIS_CANDIDATE0;
-        APPFIS_REQUIRE(i < ntab, "heat2d: candidate %d out of range (%d candidates)", i, ntab);
+        APPFIS_REQUIRE(i < kHeatCount, "heat2d: candidate %d out of range (%d candidates)", i, kHeatCount);
         return tab[i].fn(ctx, buf0, buf1, nx, ny, c, iters, tab[i].ts);
     }
     return invalid("heat2d: unknown variant %d", variant);
 }
 
-template <typename T>
-using ens_kernel_t = void (*)(const HeatGrid<T>*, int, int, T, int);
-
-// Ensemble launches with output tiles TX x TY, at most TS sweeps per launch, NT threads.
-template <typename T, int TX, int TY, int TS, int NT>
-int run_ensemble(appfis_ctx* ctx, ens_kernel_t<T> kern, int ngrid, const int* nx, const int* ny, void* const* buf0,
+// Ensemble launches of the register tiles, at most TS sweeps each.
+template <typename T, int K, int NW, int TS, int WPL>
+int run_ensemble(appfis_ctx* ctx, int ngrid, const int* nx, const int* ny, void* const* buf0,
                  void* const* buf1, double c, int iters)
 {
+    constexpr int TX = 64 * WPL - 2 * TS, TY = NW * K - 2 * TS;
+    const auto kern = k_heat2d_rt_ens<T, K, NW, TS, WPL>;
     std::vector<HeatGrid<T>> hg((size_t)ngrid);
     long long tiles = 0;
     for (int g = 0; g < ngrid; g++) {
@@ -492,8 +473,8 @@ int run_ensemble(appfis_ctx* ctx, ens_kernel_t<T> kern, int ngrid, const int* nx
     st = cached_graph(ctx, key,
                       [&]() {
                           for (int l = 0; l < n; l++) {
-                              hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(NT), 0, ctx->stream, tab, ngrid,
-                                                 l & 1, (T)c, counts[l]);
+                              hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(64 * NW), 0, ctx->stream, tab, ngrid,
+                                                 l & 1, (T)c, counts[l], fused_limit(c, counts[l]));
                               APPFIS_LAUNCH_CHECK();
                           }
                           return APPFIS_OK;
@@ -514,24 +495,21 @@ extern "C" int appfis_heat2d_ensemble(appfis_ctx* ctx, int dtype, int ngrid, con
     APPFIS_REQUIRE(ngrid >= 1, "heat2d ensemble: need at least one grid");
     APPFIS_REQUIRE(iters >= 0, "iters must be >= 0");
     if (iters == 0) return APPFIS_OK;
-    // register tiles, 48 x 96 output cells, 8 sweeps per launch, 16 waves
+    // 64 grids of 128 to 1024 cells a side, 200 sweeps: FP64 3.28 ms with two columns per lane,
+    // 3.45 with one; FP32 1.77 and 1.58.
     if (dtype == APPFIS_F64)
-        return run_ensemble<double, 48, 96, 8, 1024>(ctx, k_heat2d_rt_ens<double, 7, 16, 8, 1>, ngrid, nx, ny, buf0, buf1,
-                                                     c, iters);
+        return run_ensemble<double, 8, 8, 8, 2>(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
     if (dtype == APPFIS_F32)
-        return run_ensemble<float, 48, 96, 8, 1024>(ctx, k_heat2d_rt_ens<float, 7, 16, 8, 1>, ngrid, nx, ny, buf0, buf1, c,
-                                                    iters);
+        return run_ensemble<float, 14, 8, 8, 1>(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
     return invalid("heat2d ensemble: dtype must be F64 or F32");
 }
 
 extern "C" int appfis_heat2d_candidates(int dtype, char* names, int len)
 {
     if (dtype != APPFIS_F64 && dtype != APPFIS_F32) return -invalid("heat2d: dtype must be F64 or F32");
-    const HeatVariant* tab = dtype == APPFIS_F64 ? kHeatF64 : kHeatF32;
-    const int ntab = dtype == APPFIS_F64 ? (int)(sizeof(kHeatF64) / sizeof(kHeatF64[0]))
-                                         : (int)(sizeof(kHeatF32) / sizeof(kHeatF32[0]));
+    const HeatVariant* tab = dtype == APPFIS_F64 ? kHeat<double> : kHeat<float>;
     std::string all;
-    for (int i = 0; i < ntab; i++) all += std::string(tab[i].name) + "\n";
+    for (int i = 0; i < kHeatCount; i++) all += std::string(tab[i].name) + "\n";
     if (names && len > 0) snprintf(names, (size_t)len, "%s", all.c_str());
-    return ntab;
+    return kHeatCount;
 }

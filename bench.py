@@ -270,7 +270,7 @@ def bench_heat(ctx, hip, n=1024, iters=500):
         if variant == hip.PLAIN:
             launches = iters
         else:
-            tname = _tuned(ctx, 1, hip.F64)  # e.g. "tb 64x64 ts8 nt1024", "rt 48x96 ts8 k7 w16"
+            tname = _tuned(ctx, 1, hip.F64)  # e.g. "rt 48x96 ts8 k7 w16"
             ts = int(tname.split()[2][2:])
             launches = len(_plan(iters, ts))
         per_launch_sweeps = iters / launches
@@ -371,7 +371,7 @@ def bench_heat_ensemble(ctx, hip, ngrid=64, iters=500):
         if name == "ensemble":
             # the FP64 ensemble runs 48 x 96 register tiles (7 rows x 16 waves), 8 sweeps per launch
             launches = len(_plan(iters, 8))
-            r["roofline"] = roofline(16.0 * cells * iters / launches, ms / launches, "k_heat2d_rt_ens<double, 7, 16, 8, 1>")
+            r["roofline"] = roofline(16.0 * cells * iters / launches, ms / launches, "k_heat2d_rt_ens<double, 8, 8, 8, 2>")
         out[name] = r
     assert res["ensemble"] == res["plain_one_at_a_time"] == res["chosen_one_at_a_time"]
     out["ensemble"]["speedup_vs_plain"] = round(out["plain_one_at_a_time"]["ms"] / out["ensemble"]["ms"], 3)

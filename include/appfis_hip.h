@@ -193,8 +193,8 @@ int appfis_reduce_device_noalloc(appfis_ctx* ctx, const void* data, int dtype, i
  * u' = u + c*(uN + uS + uE + uW - 4u) over the nx*ny interior, ghost 1, double
  * buffered.  bufs[0] holds the field at entry; after `iters` sweeps the field is in
  * bufs[iters % 2] (the Grid::Swap parity).  dtype F64 or F32.
- * variant PLAIN: one sweep per launch.  CHOSEN: `tsteps` sweeps per launch with an
- * LDS-resident tile (temporal blocking); tsteps <= 0 picks the tuned depth. */
+ * variant PLAIN: one sweep per launch.  CHOSEN: `tsteps` sweeps per launch with a
+ * register-resident tile (temporal blocking); tsteps <= 0 picks the tuned depth. */
 int appfis_heat2d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1, int nx, int ny, double c,
                   int iters, int variant, int tsteps);
 

@@ -61,6 +61,49 @@ def test_heat2d_every_candidate_bit_exact(ctx, dt, nx, ny, iters):
         assert np.array_equal((d0, d1)[iters % 2].download(), ref), name
 
 
+# 62 x 78 fills the window of the one-block form, 63 x 78 and 62 x 79 are the first that do not;
+# at 400 x 420 every tiling has blocks with and without a side of the grid
+@pytest.mark.parametrize("dt", [hip.F64, hip.F32])
+@pytest.mark.parametrize("nx,ny", [(62, 78), (63, 78), (62, 79), (1, 1), (400, 420)])
+@pytest.mark.parametrize("iters", [1, 2, 37])
+def test_heat2d_windows(ctx, dt, nx, ny, iters):
+    a, d0, d1 = _heat_pair(ctx, nx, ny, dt, seed=nx + ny)
+    ref = oracle.heat2d(a.copy(), np.zeros_like(a), nx, ny, 0.1, iters)
+    for variant in (hip.CHOSEN, *(hip.CANDIDATE0 + i for i in range(len(hip.heat2d_candidates(dt))))):
+        d0.upload(a)
+        d1.upload(np.zeros_like(a))
+        ctx.heat2d(d0, d1, nx, ny, 0.1, iters, variant)
+        assert np.array_equal((d0, d1)[iters % 2].download(), ref), variant
+
+
+# infinities, NaN and magnitudes of which four are (or grow to be) past the type's largest: every
+# form has to give what the one-sweep form does, near them and in the tiles that hold none
+@pytest.mark.parametrize("dt", [hip.F64, hip.F32])
+@pytest.mark.parametrize("c", [0.1, 0.4, -3.0])
+def test_heat2d_extreme_values(ctx, dt, c):
+    nx, ny, iters = 150, 140, 19
+    a, d0, d1 = _heat_pair(ctx, nx, ny, dt, seed=77)
+    top = np.finfo(a.dtype).max
+    a[30, 40], a[31, 90], a[100, 20], a[120, 130] = top / 2, top / 5, -top / 3, top / 1e5
+    for special in (None, np.inf, np.nan):
+        if special is not None:
+            a[60, 145] = special
+        d0.upload(a)
+        d1.upload(np.zeros_like(a))
+        ctx.heat2d(d0, d1, nx, ny, c, iters, hip.PLAIN)
+        ref = d1.download()
+        for variant in (hip.CHOSEN, *(hip.CANDIDATE0 + i for i in range(len(hip.heat2d_candidates(dt))))):
+            d0.upload(a)
+            d1.upload(np.zeros_like(a))
+            ctx.heat2d(d0, d1, nx, ny, c, iters, variant)
+            got = d1.download()
+            assert np.array_equal(got[1:-1, 1:-1], ref[1:-1, 1:-1], equal_nan=True), (special, variant)
+        d0.upload(a)
+        d1.upload(np.zeros_like(a))
+        ctx.heat2d_ensemble([(d0, d1, nx, ny)], c, iters)
+        assert np.array_equal(d1.download()[1:-1, 1:-1], ref[1:-1, 1:-1], equal_nan=True), special
+
+
 @pytest.mark.parametrize("dt", [hip.F64, hip.F32])
 @pytest.mark.parametrize("iters", [1, 8, 23, 64])
 def test_heat2d_ensemble_matches_oracle(ctx, dt, iters):
