@@ -86,6 +86,27 @@ def test_flood_strip_heights_bit_exact(ctx, n):
     assert np.allclose(vg, vc, rtol=1e-13, atol=0)
 
 
+# dx on both sides of the range in which dt * d / dx is taken by the reciprocal and its remainder,
+# some with inexact reciprocals; a dam breaks onto shallow and onto dry ground, so edges with the
+# entropy fix and with a dry side meet edges without in one wave
+@pytest.mark.parametrize("dx", [0.75, 1.0, 3.0000000000000004, 7.7, 2.0 ** 61])
+def test_flood_f64_cell_sizes_bit_exact(ctx, dx):
+    n, steps = 90, 12
+    h = np.full((n + 2, n + 2), 0.05)
+    h[:, :30] = 10.0
+    h[40:60, 50:] = 0.0
+    zero = np.zeros_like(h)
+    arrs = [h, zero, zero.copy(), np.linspace(0.0, 3.0, n + 2) * np.ones_like(h), zero.copy()]
+    d = [ctx.from_numpy(x, hip.F64) for x in arrs]
+    t, v = ctx.flood_run(*d, n, n, hip.FloodParams(dx, CN, HEXTRA, DT_FALLBACK, 0.0, RAIN, 0.0), steps)
+    c = [x.copy() for x in arrs]
+    tc, vc, _ = oracle.flood_run(*c, n, n, dx, CN, HEXTRA, DT_FALLBACK, 0.0, RAIN, 0.0, steps)
+    for a, b in zip(d[:3], c[:3]):
+        assert np.array_equal(a.download(), b)
+    assert np.array_equal(t, tc)
+    assert np.allclose(v, vc, rtol=1e-13, atol=0)
+
+
 @pytest.mark.parametrize("n,wet,steps", [(64, 0.0, 80), (90, 0.3, 50)])
 def test_flood_f64_with_friction(ctx, n, wet, steps):
     arrs = scenario(n, 3100 + n, wet=wet)
