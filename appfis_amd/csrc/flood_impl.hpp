@@ -413,13 +413,13 @@ constexpr int MWAVES = BT / 64;   // strips per block
 // Rows of a strip.  A strip solves its top edge row twice over (once per neighbour), so long
 // strips waste least, but a wave marches its rows one after the other: a grid cut into
 // fewer strips than the chip has SIMDs runs at the latency of one strip however small it is
-// (785 x 785 in FP64: 325 strips of 32 rows, 130 us a step, against 47 with 5 rows).  The
+// (785 x 785 in FP64: 325 strips of 32 rows, 119 us a step, against 42 with 5 rows).  The
 // blocks of a launch share the CUs, so a step takes about
 //     max(blocks per CU, rounded up, L) * (rows + E)
 // rows' time of a busy SIMD: E is the repeated work of a strip in rows (0.9 FP64, 1.2 FP32:
-// 4096 x 4096 in strips of 4, 8, 16 rows: 861, 776, 744 us; an FP32 ensemble of 8, 16, 32:
-// 813, 749, 734), and a wave alone on its SIMD takes L times a busy one's share of time per
-// row (FP64 3.9 against 2.7 us, FP32 2.4 against 1.0, both kernels of a step).  The choice is
+// 4096 x 4096 in strips of 4, 8, 16 rows: 715, 661, 642 us; an FP32 ensemble of 12, 16, 32:
+// 702, 692, 687), and a wave alone on its SIMD takes L times a busy one's share of time per
+// row (FP64 3.2 against 2.2 us, FP32 1.8 against 0.8, both kernels of a step).  The choice is
 // the minimum over the lengths below; every value of the fields is the same for all of them.
 template <typename R>
 int strip_rows(int num_cu, int nscen, const int* nx, const int* ny)
@@ -650,7 +650,10 @@ __device__ inline void wave_min_sum(R& m, double& s, double& c)
 // reads only h and z, which nothing here writes).  Each lane folds its cells into its
 // own CFL minimum and compensated volume sum, and the wave's DPP reduction leaves one
 // partial per strip, partials[3t .. 3t+2] = (min, sum, compensation).  No LDS and no
-// barriers.  MODE 0: initial CFL only (no fix); MODE 1: end of a step.
+// barriers.  MODE 0: initial CFL only (no fix); MODE 1: end of a step.  Memory bounds it
+// (16 bytes per FP32 cell at 4.4 TB/s in a 47 M cell ensemble, 170 us), so every row is
+// loaded one ahead of its use: without that 182 us, and 9.2 against
+// 8.3 for 785^2 in FP64.
 template <typename R, int MODE>
 __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc, int nscen, int nstrips, int mr,
                                                   int par, Params P)
@@ -676,20 +679,24 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
     const gmem<R>* z = to_global(S.z);
     const R G = (R)9.81, EPS12 = (R)1e-12;
     const R hextra = (R)P.hextra, dx = (R)P.dx, cn = (R)P.cn;
-    auto ld = [&](const gmem<R>* a, int row) { return colmem ? a[(size_t)col + W * (size_t)row] : (R)0.0; };
+    // Rows ahead of their use, unconditionally: lanes past the array load its last column, and
+    // rows past the strip a row inside the array; neither value is used (the next strip may be
+    // writing such a qx or qy).
+    const size_t colc = (size_t)(colmem ? col : nx + 1);
+    auto ld = [&](const gmem<R>* a, int row) { return a[colc + W * (size_t)min(row, ny + 1)]; };
     R cfl = RealLim<R>::max();
     double vs = 0.0, vc = 0.0;
-    R hm = ld(h, j0 - 1), hc = ld(h, j0), zm = (R)0.0, zc = (R)0.0;
+    R hm = ld(h, j0 - 1), hc = ld(h, j0), hp = ld(h, j0 + 1), qxv = ld(qx, j0), qyv = ld(qy, j0);
+    R zm = (R)0.0, zc = (R)0.0, zp = (R)0.0;
     if (MODE == 1) {
         zm = ld(z, j0 - 1);
         zc = ld(z, j0);
+        zp = ld(z, j0 + 1);
     }
     for (int r = 0; r < nr; r++) {
         const int j = j0 + r;
-        const R hp = ld(h, j + 1);  // j + 1 <= ny + 1
-        const R zp = MODE == 1 ? ld(z, j + 1) : (R)0.0;
-        R qxv = cell ? qx[(size_t)col + W * (size_t)j] : (R)0.0;
-        R qyv = cell ? qy[(size_t)col + W * (size_t)j] : (R)0.0;
+        const R hn = ld(h, j + 2), qxn = ld(qx, j + 1), qyn = ld(qy, j + 1);
+        const R zn = MODE == 1 ? ld(z, j + 2) : (R)0.0;
         R hl = (R)0.0, hr = (R)0.0, zl = (R)0.0, zr = (R)0.0;
         if (MODE == 1) {
             hl = lane_shift<true>(hc);
@@ -721,8 +728,12 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
         }
         hm = hc;
         hc = hp;
+        hp = hn;
         zm = zc;
         zc = zp;
+        zp = zn;
+        qxv = qxn;
+        qyv = qyn;
     }
     wave_min_sum(cfl, vs, vc);
     if (lane == WAVE_TOTAL_LANE) {
@@ -736,20 +747,39 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
 // Finalise: one block per scenario combines its tile partials in a fixed order (the
 // reference's Execute2DReduce(MIN) plus the config's FP64 Kahan volume), then does the
 // host-side bookkeeping of triton_appfis.hpp:322-335, 381-385 on the device.
+//
+// One block with a long list to read is bound by the latency of its loads: 16 waves with
+// four partials each in flight take 7.8 us for an FP32 ensemble of 28000 strips, where 4
+// waves with one took 18.7.
+constexpr int FT = 1024;
 template <typename R, int MODE>
-__global__ __launch_bounds__(BT) void k_finalize(const Scen<R>* __restrict__ sc, Params P)
+__global__ __launch_bounds__(FT) void k_finalize(const Scen<R>* __restrict__ sc, Params P)
 {
-    __shared__ double smin[BT / 64];
-    __shared__ double ssum[BT / 64][2];
+    __shared__ double smin[FT / 64];
+    __shared__ double ssum[FT / 64][2];
     const Scen<R>& S = sc[blockIdx.x];
-    if (MODE == 1 && finished(S.st, P)) return;  // before thread 0 updates simtime below
+    if (MODE == 1 && finished(S.st, P)) return;  // before one thread updates simtime below
     double m = (double)RealLim<R>::max();
     double as = 0.0, ac = 0.0;
-    for (int p = threadIdx.x; p < S.nstrips; p += BT) {
-        const double* pp = S.partials + 3 * (size_t)p;
-        m = pp[0] < m ? pp[0] : m;
-        two_sum(as, ac, pp[1]);
-        ac = __dadd_rn(ac, pp[2]);
+    // four partials' loads in flight per thread; 0 past the end changes no sum
+    constexpr int U = 4;
+    const gmem<double>* part = to_global((const double*)S.partials);
+    const int last = S.nstrips - 1;
+    for (int p0 = threadIdx.x; p0 < S.nstrips; p0 += FT * U) {
+        double x[U][3];
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const gmem<double>* pp = part + 3 * (size_t)min(p0 + k * FT, last);
+#pragma unroll
+            for (int c = 0; c < 3; c++) x[k][c] = pp[c];
+        }
+#pragma unroll
+        for (int k = 0; k < U; k++) {
+            const bool in = p0 + k * FT <= last;
+            m = in && x[k][0] < m ? x[k][0] : m;
+            two_sum(as, ac, in ? x[k][1] : 0.0);
+            ac = __dadd_rn(ac, in ? x[k][2] : 0.0);
+        }
     }
     wave_min_sum(m, as, ac);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -759,14 +789,11 @@ __global__ __launch_bounds__(BT) void k_finalize(const Scen<R>* __restrict__ sc,
         ssum[wid][1] = ac;
     }
     __syncthreads();
-    if (threadIdx.x != 0) return;
-    double bs = ssum[0][0], bc = ssum[0][1];
-    for (int w = 1; w < BT / 64; w++) {
-        m = smin[w] < m ? smin[w] : m;
-        two_sum(bs, bc, ssum[w][0]);
-        bc = __dadd_rn(bc, ssum[w][1]);
-    }
-    m = smin[0] < m ? smin[0] : m;
+    if (wid != 0) return;
+    m = lane < FT / 64 ? smin[lane] : (double)RealLim<R>::max();
+    double bs = lane < FT / 64 ? ssum[lane][0] : 0.0, bc = lane < FT / 64 ? ssum[lane][1] : 0.0;
+    wave_min_sum(m, bs, bc);
+    if (lane != WAVE_TOTAL_LANE) return;
     ScenState* st = S.st;
     const double PI = P.print_interval;
     double simtime = st->simtime;
@@ -945,7 +972,7 @@ int run_flood(appfis_ctx* ctx, int nscen, const int* nx, const int* ny, void* co
     // dt of the first step from the initial state
     hipLaunchKernelGGL((k_fix_march<R, 0>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, 0, P);
     APPFIS_LAUNCH_CHECK();
-    hipLaunchKernelGGL((k_finalize<R, 0>), dim3(nscen), dim3(BT), 0, ctx->stream, tab, P);
+    hipLaunchKernelGGL((k_finalize<R, 0>), dim3(nscen), dim3(FT), 0, ctx->stream, tab, P);
     APPFIS_LAUNCH_CHECK();
     auto step_pair = [&](int par) -> int {
         hipLaunchKernelGGL((k_flux_march<R>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, par, P);
@@ -956,7 +983,7 @@ int run_flood(appfis_ctx* ctx, int nscen, const int* nx, const int* ny, void* co
         }
         hipLaunchKernelGGL((k_fix_march<R, 1>), grid, dim3(BT), 0, ctx->stream, tab, nscen, nstrips, mr, par ^ 1, P);
         APPFIS_LAUNCH_CHECK();
-        hipLaunchKernelGGL((k_finalize<R, 1>), dim3(nscen), dim3(BT), 0, ctx->stream, tab, P);
+        hipLaunchKernelGGL((k_finalize<R, 1>), dim3(nscen), dim3(FT), 0, ctx->stream, tab, P);
         APPFIS_LAUNCH_CHECK();
         return APPFIS_OK;
     };
