@@ -11,9 +11,14 @@
 //   compile-time byte offset W mod 16 (one kernel instance per residue).  Neighbour
 //   counts are SWAR byte sums (column sums, then +/-1 byte shifts with v_alignbyte),
 //   the B3/S23 rule is a zero-byte test, and the chunk is stored with 16-byte stores.
-//   Ghost cells in a chunk (x = 0 or W-1, and the two ghost rows) take the wrapped
-//   value new(xw, yw), recomputed from the current buffer whose ring is valid, so the
-//   written buffer leaves with its ring already exchanged: no second launch.
+//   Ghost cells take the wrapped value new(xw, yw), recomputed from the current buffer
+//   whose ring is valid, so the written buffer leaves with its ring already exchanged:
+//   no second launch.  A generation of a small board is a few latencies long, so a wave
+//   issues all its loads before it uses any: a chunk's ghost columns (at most one pair, for
+//   W >= 17) take six words loaded with everything else, and chunks of the ghost rows are
+//   computed whole, like the others, from the rows they wrap to.  Per generation, against
+//   recomputing ghost cells one by one: 100 x 100 5.1 us for 12.7, 1000 x 777 5.0 for 7.9,
+//   4096^2 9.9 for 15.7; 8192^2 25.8 for 32.7 (5.2 TB/s: the rate of a copy).
 //
 // CHOSEN: gol_bits.hip (bit-packed copy of the field, 32 cells per word) from 32 cells a row on,
 //   this byte kernel below.
@@ -75,7 +80,7 @@ __device__ __forceinline__ uint8_t rule(int n, uint8_t alive) { return (uint8_t)
 
 // New value of cell (x, y) of the padded buffer, ghost cells mapped to the wrapped
 // interior cell; neighbours read from the current buffer (valid ring).
-__device__ __noinline__ uint8_t cell_new(const uint8_t* __restrict__ u, int W, int H, int x, int y)
+__device__ inline uint8_t cell_new(const uint8_t* __restrict__ u, int W, int H, int x, int y)
 {
     const int nx = W - 2, ny = H - 2;
     int xw = x == 0 ? nx : (x == W - 1 ? 1 : x);
@@ -85,6 +90,72 @@ __device__ __noinline__ uint8_t cell_new(const uint8_t* __restrict__ u, int W, i
     const uint8_t* r2 = r1 + W;
     int n = r0[xw - 1] + r0[xw] + r0[xw + 1] + r1[xw - 1] + r1[xw + 1] + r2[xw - 1] + r2[xw] + r2[xw + 1];
     return rule(n, r1[xw]);
+}
+
+// CB cells by SWAR: the rows above, at and below them and the sums of the columns on their
+// left and right.  alive' = (n == 3) | (alive & n == 2) = ((n | alive) == 3) for n <= 8.
+template <int ND>
+__device__ __forceinline__ void next_cells(const uint32_t (&up)[ND], const uint32_t (&m)[ND], const uint32_t (&dn)[ND],
+                                           uint32_t sl, uint32_t sr, uint32_t (&out)[ND])
+{
+    uint32_t s[ND];  // column sums (bytes <= 3), then x-1 / x+1 shifted copies
+#pragma unroll
+    for (int d = 0; d < ND; d++) s[d] = up[d] + m[d] + dn[d];
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        const uint32_t lo = d == 0 ? (sl << 24) : s[d - 1];
+        const uint32_t hi = d == ND - 1 ? sr : s[d + 1];
+        const uint32_t n = abyte(s[d], lo, 3) + s[d] + abyte(hi, s[d], 1) - m[d];
+        out[d] = zero_bytes((n | m[d]) ^ 0x03030303u);
+    }
+}
+
+// The 3 x 3 cells around one cell: a word from any address of each of three rows W apart, that
+// ends with the row's three cells (HIGH) or starts with them.
+struct Around {
+    uint32_t above, at, below;
+};
+template <bool HIGH>
+__device__ __forceinline__ Around load_around(const uint8_t* __restrict__ u, int first, int W)
+{
+    const uint8_t* p = u + first - (HIGH ? 1 : 0);
+    Around a;
+    __builtin_memcpy(&a.above, p, 4);
+    __builtin_memcpy(&a.at, p + W, 4);
+    __builtin_memcpy(&a.below, p + 2 * W, 4);
+    return a;
+}
+template <bool HIGH>
+__device__ __forceinline__ uint32_t next_cell(const Around& a)
+{
+    constexpr int S = HIGH ? 8 : 0;
+    const uint32_t s = (a.above + a.at + a.below) >> S, alive = (a.at >> (8 + S)) & 1u;  // bytes <= 3
+    const uint32_t n = (s & 0xFFu) + ((s >> 8) & 0xFFu) + ((s >> 16) & 0xFFu) - alive;
+    return (n | alive) == 3u ? 1u : 0u;
+}
+
+// Four bytes from any offset, those outside the buffer undefined: the load, from the nearest
+// offset inside, and, once it is there, the move of its bytes to their places.
+__device__ __forceinline__ uint32_t load_word(const uint8_t* __restrict__ u, int off, int nbytes)
+{
+    uint32_t x;
+    __builtin_memcpy(&x, u + min(max(off, 0), nbytes - 4), 4);
+    return x;
+}
+__device__ __forceinline__ uint32_t place_word(uint32_t x, int off, int nbytes)
+{
+    const int sh = (off - min(max(off, 0), nbytes - 4)) * 8;
+    return sh < 0 ? x << (-sh & 31) : x >> (sh & 31);
+}
+
+template <int ND>
+__device__ __forceinline__ void set_byte(uint32_t (&w)[ND], int b, uint32_t x)  // b < 0 or >= 4*ND: none
+{
+#pragma unroll
+    for (int d = 0; d < ND; d++) {
+        const uint32_t mask = (unsigned)(b - 4 * d) < 4u ? 0xFFu << (((unsigned)b & 3u) * 8) : 0u;
+        w[d] = (w[d] & ~mask) | (mask & (x * 0x01010101u));
+    }
 }
 
 template <int DB, int CB>
@@ -104,6 +175,15 @@ __global__ __launch_bounds__(256) void k_gol_plain(const uint8_t* __restrict__ u
     const bool valid = c < nchunks;
     const bool full = valid && p0 + CB <= nbytes;
 
+    if (W <= CB) {  // several boundaries of rows in a chunk: cell by cell
+        if (!valid) return;
+#pragma unroll 1
+        for (int b = 0; b < CB && p0 + b < nbytes; b++) {
+            const int y = rd.row(p0 + b);
+            v[p0 + b] = cell_new(u, W, H, p0 + b - y * W, y);
+        }
+        return;
+    }
     // rows of the first and last cell of the chunk, and whether the fast path applies
     // (all CB cells in interior rows and every load in bounds) -- before any load, so
     // that all loads of the lane are in flight together
@@ -137,6 +217,34 @@ __global__ __launch_bounds__(256) void k_gol_plain(const uint8_t* __restrict__ u
         if (lane == 0 || c == 0) mlb = u[p0 - 1];
         if (lane == 63 || c + 1 >= nchunks || p0 + 2 * CB > nbytes) mrb = u[p0 + CB];
     }
+    // the chunk's ghost columns: byte br is the right one of row y0, byte bl the left one of the
+    // row after it, or of row y0 where the chunk starts with it
+    const int nx = W - 2, ny = H - 2;
+    auto wrap = [&](int y) { return y == 0 ? ny : (y == H - 1 ? 1 : y); };
+    const int x0 = p0 - y0 * W;
+    const int br = W - 1 - x0, bl = x0 == 0 ? 0 : br + 1;
+    const bool has_r = valid && br < CB && p0 + br < nbytes, has_l = valid && bl < CB && p0 + bl < nbytes;
+    // a chunk of a ghost row, at the buffer's ends, or whose aligned spans leave it: the CB
+    // cells of row y0, and those of row y0 + 1 if the chunk reaches into it, from the rows
+    // they wrap to
+    const bool two = br + 1 < CB && p0 + br + 1 < nbytes;
+    uint32_t a[2][3][ND + 1];  // from the byte before the chunk's on, three rows of each part
+    auto part_at = [&](int part, int k, int d) {
+        return p0 - 1 + (wrap(y0 + part) - (y0 + part) + k - 1) * W + 4 * d;
+    };
+    auto load_part = [&](int part) {
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int d = 0; d <= ND; d++) a[part][k][d] = load_word(u, part_at(part, k, d), nbytes);
+    };
+    if (valid && !fast) {
+        load_part(0);
+        if (two) load_part(1);
+    }
+    Around gr = {}, gl = {};
+    if (has_r) gr = load_around<false>(u, (wrap(y0) - 1) * W, W);
+    if (has_l) gl = load_around<true>(u, (wrap(x0 == 0 ? y0 : y0 + 1) - 1) * W + nx - 1, W);
     // left / right neighbour bytes of the centre row from the adjacent lanes
     const uint32_t prevl = __shfl_up(m[ND - 1], 1, 64);
     const uint32_t next0 = __shfl_down(m[0], 1, 64);
@@ -158,35 +266,10 @@ __global__ __launch_bounds__(256) void k_gol_plain(const uint8_t* __restrict__ u
             window<DA, CB>(a8, up, ul, ur);
             window<DB, CB>(b8, dn, dl, dr);
         }
-        // column sums (bytes <= 3), then x-1 / x+1 shifted copies
-        uint32_t s[ND];
-#pragma unroll
-        for (int d = 0; d < ND; d++) s[d] = up[d] + m[d] + dn[d];
-        const uint32_t sl = ul + ml + dl, sr = ur + mr + dr;
         uint32_t out[ND];
-#pragma unroll
-        for (int d = 0; d < ND; d++) {
-            const uint32_t lo = d == 0 ? (sl << 24) : s[d - 1];
-            const uint32_t hi = d == ND - 1 ? sr : s[d + 1];
-            const uint32_t left = abyte(s[d], lo, 3);
-            const uint32_t right = abyte(hi, s[d], 1);
-            const uint32_t n = left + s[d] + right - m[d];
-            // alive' = (n == 3) | (alive & n == 2) = ((n | alive) == 3) for n <= 8, alive <= 1
-            out[d] = zero_bytes((n | m[d]) ^ 0x03030303u);
-        }
-        // patch ghost cells (x == 0 or x == W-1) inside the chunk
-        const int x0 = p0 - y0 * W;
-        if (x0 + CB - 1 >= W - 1 || x0 == 0) {
-#pragma unroll
-            for (int b = 0; b < CB; b++) {
-                const int p = p0 + b;
-                const int y = (unsigned)p / (unsigned)W, x = p - y * W;
-                if (x == 0 || x == W - 1) {
-                    const uint32_t nvv = cell_new(u, W, H, x, y);
-                    out[b >> 2] = (out[b >> 2] & ~(0xFFu << ((b & 3) * 8))) | (nvv << ((b & 3) * 8));
-                }
-            }
-        }
+        next_cells(up, m, dn, ul + ml + dl, ur + mr + dr, out);
+        if (has_r) set_byte(out, br, next_cell<false>(gr));
+        if (has_l) set_byte(out, bl, next_cell<true>(gl));
 #pragma unroll
         for (int q = 0; q < ND / 4; q++) {
             uint4 o;
@@ -194,12 +277,45 @@ __global__ __launch_bounds__(256) void k_gol_plain(const uint8_t* __restrict__ u
             *(uint4*)(v + p0 + 16 * q) = o;
         }
     } else if (valid) {
-        // slow path: chunk touches a ghost row, the buffer end, or an edge window
-        for (int b = 0; b < CB; b++) {
-            const int p = p0 + b;
-            if (p >= nbytes) break;
-            const int y = (unsigned)p / (unsigned)W, x = p - y * W;
-            v[p] = cell_new(u, W, H, x, y);
+        auto part_cells = [&](int part, uint32_t (&o)[ND]) {
+            uint32_t w[3][ND], sl = 0, sr = 0;
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                uint32_t x[ND + 1];
+#pragma unroll
+                for (int d = 0; d <= ND; d++) x[d] = place_word(a[part][k][d], part_at(part, k, d), nbytes);
+#pragma unroll
+                for (int d = 0; d < ND; d++) w[k][d] = abyte(x[d + 1], x[d], 1);
+                sl += x[0] & 0xFFu;
+                sr += (x[ND] >> 8) & 0xFFu;
+            }
+            next_cells(w[0], w[1], w[2], sl, sr, o);
+        };
+        uint32_t out[ND];
+        part_cells(0, out);
+        if (two) {
+            uint32_t o[ND];
+            part_cells(1, o);
+#pragma unroll
+            for (int d = 0; d < ND; d++) {
+                const int keep = min(max(br + 1 - 4 * d, 0), 4);  // bytes up to br are row y0's
+                const uint32_t mask = keep == 0 ? 0u : 0xFFFFFFFFu >> (32 - 8 * keep);
+                out[d] = (out[d] & mask) | (o[d] & ~mask);
+            }
+        }
+        if (has_r) set_byte(out, br, next_cell<false>(gr));
+        if (has_l) set_byte(out, bl, next_cell<true>(gl));
+        if (full) {
+#pragma unroll
+            for (int q = 0; q < ND / 4; q++) {
+                uint4 o;
+                o.x = out[4 * q]; o.y = out[4 * q + 1]; o.z = out[4 * q + 2]; o.w = out[4 * q + 3];
+                *(uint4*)(v + p0 + 16 * q) = o;
+            }
+        } else {
+#pragma unroll
+            for (int b = 0; b < CB; b++)
+                if (p0 + b < nbytes) v[p0 + b] = (uint8_t)(out[b >> 2] >> ((b & 3) * 8));
         }
     }
 }

@@ -225,6 +225,17 @@ def test_gol_plain_all_residues(ctx, nx):
     assert np.array_equal((d0, d1)[(gens + 1) % 2].download(), prev)
 
 
+# rows of 16 bytes and less (cell by cell), the narrowest that are computed by chunks, boards of
+# two rows (every chunk touches a ghost row), and chunks that end a ghost row and start the next
+@pytest.mark.parametrize("nx,ny", [(2, 2), (14, 2), (15, 2), (15, 40), (16, 3), (17, 2), (30, 2), (45, 4), (1021, 2)])
+def test_gol_plain_ghost_chunks(ctx, nx, ny):
+    gens = 12
+    a, d0, d1 = _gol_pair(ctx, nx, ny, seed=nx + ny, p=0.4)
+    ctx.gol(d0, d1, nx, ny, gens, hip.PLAIN)
+    assert np.array_equal(d0.download(), oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens))
+    assert np.array_equal(d1.download(), oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens - 1))
+
+
 def test_gol_full_config_prefix(ctx):
     # 8192^2 config: the first 12 generations against the oracle bit for bit
     nx = ny = 8192
