@@ -349,12 +349,12 @@ struct HeatVariant {
 
 // Temporal-blocking candidates (output tile TX x TY, TS sweeps per launch, K rows in each of NW
 // waves; "rt2": two columns per lane).  A launch costs about 5 us before its first sweep's worth of
-// work, and tiles load and compute a halo of TS cells around their output, so small grids take
-// small tiles of 8 sweeps (512^2 FP64: 48x24 0.89 us per sweep, 96x48 1.19), and grids of about one
-// block per CU deep ones (1024^2: 96x48 1.20, 48x48 1.32).  Beyond that the adds decide
-// (4096^2 FP64: 48x96 k14 10.3, k7 14.5, 96x48 over 12.2).  "whole" needs no halo: 62^2
-// takes 0.82 in one block, 1.04 in 48x24 tiles.  A fixed depth takes the first entry that
-// holds it.
+// work, and tiles load and compute a halo of TS cells around their output: the deepest are best
+// while the tiles fit the CUs about once, in the smallest window that makes it so (FP64, us per
+// sweep: 96 x 80 32x16 0.84, 48x24 1.03; 512^2 32x32 0.78, 48x24 0.87, 96x48 1.19; 1024^2 96x48
+// 1.20, 48x48 1.32).  Beyond that the adds decide (4096^2: 48x96 k14 10.3, k7 14.5, 96x48 over
+// 12.2).  "whole" needs no halo, but one CU does all the work: 62^2 takes 0.82, 48 x 48 the
+// same and in 32x16 tiles 0.83.  A fixed depth takes the first entry that holds it.
 template <typename T>
 static const HeatVariant kHeat[] = {
     {"rt 48x48 ts8 k8 w8", run_rt<T, 8, 8, 8, 1>, 8},
@@ -367,6 +367,8 @@ static const HeatVariant kHeat[] = {
     {"rt 40x72 ts12 k12 w8", run_rt<T, 12, 8, 12, 1>, 12},
     {"rt2 104x56 ts12 k5 w16", run_rt<T, 5, 16, 12, 2>, 12},
     {"rt2 96x48 ts16 k5 w16", run_rt<T, 5, 16, 16, 2>, 16},
+    {"rt 32x16 ts16 k6 w8", run_rt<T, 6, 8, 16, 1>, 16},
+    {"rt 32x32 ts16 k4 w16", run_rt<T, 4, 16, 16, 1>, 16},
     {"whole 64x80 k5 w16", run_whole<T, 5, 16, 1>, 0},
 };
 constexpr int kHeatCount = (int)(sizeof(kHeat<double>) / sizeof(kHeat<double>[0]));
