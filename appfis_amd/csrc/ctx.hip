@@ -383,7 +383,9 @@ int appfis_malloc(appfis_ctx* ctx, size_t bytes, void** out)
     if (bytes == 0) bytes = 1;
     APPFIS_HIP_CHECK(hipSetDevice(ctx->device));
     APPFIS_HIP_CHECK(hipMalloc(out, bytes));
+    // zeroed before the caller has the pointer: it may write there from another stream
     APPFIS_HIP_CHECK(hipMemsetAsync(*out, 0, bytes, ctx->stream));
+    APPFIS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
     return APPFIS_OK;
 }
 

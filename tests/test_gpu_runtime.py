@@ -24,6 +24,20 @@ def test_abi_version_and_roundtrip(ctx):
     assert np.array_equal(d.download(), a)
 
 
+def test_malloc_zeroed_before_use_on_another_stream(ctx):
+    # the context's stream is busy when the array is made; another context's stream writes it at once
+    n = 2048
+    u, v = ctx.array((n + 2, n + 2), hip.F64), ctx.array((n + 2, n + 2), hip.F64)
+    a = np.arange(1, 100001, dtype=np.float64)
+    with hip.Context(0) as other:
+        ctx.heat2d(u, v, n, n, 0.1, 400, hip.PLAIN)
+        d = ctx.array(a.shape, hip.F64)
+        hip.check(hip.lib().appfis_memcpy_h2d(other.handle, d.ptr, a.ctypes.data, a.nbytes), "h2d")
+        other.sync()
+    ctx.sync()
+    assert np.array_equal(d.download(), a)
+
+
 @pytest.mark.parametrize("nbytes,src_off,dst_off", [(4096, 0, 0), (1000003, 0, 0), (77, 16, 32), (5000, 3, 0),
                                                      (16, 0, 16), (100000, 16, 5)])
 def test_memcpy_d2d(ctx, nbytes, src_off, dst_off):
