@@ -252,17 +252,20 @@ __device__ inline bool roe(R h1, R h2, R qx1, R qy1, R z1, R qx2, R qy2, R z2, R
     eigen[2] = un + c12;
 #pragma unroll
     for (int i = 0; i < 3; i++) eigenE[i] = (R)0.0;
-    R e1 = N::dot(u1, v1) - SQRTG * sqh1;
-    R e2 = N::dot(u2, v2) - SQRTG * sqh2;
-    if (e1 < (R)0.0 && e2 > (R)0.0) {
-        eigenE[0] = eigen[0] - fdiv(e1 * (e2 - eigen[0]), e2 - e1);
-        eigen[0] = fdiv(e1 * (e2 - eigen[0]), e2 - e1);
-    }
-    e1 = N::dot(u1, v1) + SQRTG * sqh1;
-    e2 = N::dot(u2, v2) + SQRTG * sqh2;
-    if (e1 < (R)0.0 && e2 > (R)0.0) {
-        eigenE[2] = eigen[2] - fdiv(e2 * (eigen[2] - e1), e2 - e1);
-        eigen[2] = fdiv(e2 * (eigen[2] - e1), e2 - e1);
+    // the entropy fix: transcritical edges only, so the wave computes it where any of its edges is one
+    const R a1 = N::dot(u1, v1) - SQRTG * sqh1, a2 = N::dot(u2, v2) - SQRTG * sqh2;
+    const R b1 = N::dot(u1, v1) + SQRTG * sqh1, b2 = N::dot(u2, v2) + SQRTG * sqh2;
+    const bool fix0 = a1 < (R)0.0 && a2 > (R)0.0, fix2 = b1 < (R)0.0 && b2 > (R)0.0;
+    const bool any_fix = __any(fix0 || fix2);
+    if (any_fix) {
+        if (fix0) {
+            eigenE[0] = eigen[0] - fdiv(a1 * (a2 - eigen[0]), a2 - a1);
+            eigen[0] = fdiv(a1 * (a2 - eigen[0]), a2 - a1);
+        }
+        if (fix2) {
+            eigenE[2] = eigen[2] - fdiv(b2 * (eigen[2] - b1), b2 - b1);
+            eigen[2] = fdiv(b2 * (eigen[2] - b1), b2 - b1);
+        }
     }
     eigev[0][0] = (R)1.0;
     eigev[0][1] = N::subx(u12, c12);
@@ -324,10 +327,9 @@ __device__ inline bool roe(R h1, R h2, R qx1, R qy1, R z1, R qx2, R qy2, R z2, R
             }
         }
     }
-    // Without an entropy fix (transcritical edges only) these terms are zeros, which change no
-    // sum but of infinities and NaN: the wave takes them where any of its edges has one.
+    // Without an entropy fix these terms are zeros, which change no sum but of infinities and NaN.
     const R size = (fabs(alpha[0]) + fabs(alpha[1])) + (fabs(alpha[2]) + c12) + (fabs(u12) + fabs(v12));
-    if (__any(eigenE[0] != (R)0.0 || eigenE[2] != (R)0.0 || !(size <= RealLim<R>::max()))) {
+    if (any_fix || __any(!(size <= RealLim<R>::max()))) {
 #pragma unroll
         for (int i = 0; i < 3; i++) {
             if (eigenE[i] > (R)0.0) {
@@ -364,6 +366,20 @@ __device__ inline int find_scen(const Scen<R>* sc, int nscen, int strip)
     return lo;
 }
 
+// The wave's number in its block, as a scalar: all that follows from it (the strip, its scenario's
+// fields, the rows' addresses) then lives in scalar registers and is computed by the scalar unit.
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); }
+
+// A row of a field as a scalar base address, opaque so that it is added by the load or store itself
+// and not, 64 bits wide, by the vector unit.
+template <typename R>
+__device__ __forceinline__ R* row_base(R* field, size_t first)
+{
+    R* p = field + first;
+    asm("" : "+s"(p));
+    return p;
+}
+
 // One cell's state and the per-cell values every edge solve of it uses.
 template <typename R>
 struct CellV {
@@ -374,7 +390,7 @@ struct CellV {
 // offset into the array, and the values of lanes or rows outside it are never used.
 template <typename R>
 __device__ inline void cell_load(CellV<R>& c, const gmem<R>* h, const gmem<R>* qx, const gmem<R>* qy, const gmem<R>* z,
-                                 const gmem<R>* n2, size_t off)
+                                 const gmem<R>* n2, unsigned off)
 {
     c.h = h[off];
     c.qx = qx[off];
@@ -402,11 +418,13 @@ __device__ inline void cell_derive(CellV<R>& c, R hextra)
 // Every edge is solved once; each cell's velocities and sqrt(h) once; the arguments of
 // every solve and the order of the rhs accumulation are those of the functors, so the
 // results are those of the per-cell form.  No LDS and no barriers.
-// The vector instructions bound it (they fill about 70 % of the time; memory would take
-// 60 % of it in FP32): in FP64 a third of them are divisions, so those by dx share one
-// reciprocal, and terms that only some edges have are left out of waves without any such
-// edge (the dry-side test and the entropy fix in roe).  785^2 FP64 33.0 -> 29.9 us,
-// an FP32 ensemble of 47 M cells 519 -> 504.
+// The vector instructions bound it (1.6 GB in 455 us in a 47 M cell FP32 ensemble, where memory would
+// take 300; one instruction takes a SIMD 4 clocks).  In FP64 a third of them were divisions, so
+// those by dx share one reciprocal; terms that only some edges have are left out of waves
+// without any such edge (the dry-side test and the entropy fix in roe: 519 -> 485 us, 785^2
+// FP64 33.0 -> 29.9); and a strip's rows are addressed by the scalar unit, which takes the vector
+// work and the registers of ten 64-bit pointers out (FP32 82 -> 57 registers, 485 -> 455;
+// FP64 142 -> 122, 2048^2 182 -> 177 us a step).
 constexpr int MW = 62;            // strip columns (lanes 1..62)
 constexpr int MWAVES = BT / 64;   // strips per block
 
@@ -445,7 +463,7 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
                                                    int par, Params P)
 {
     const int lane = threadIdx.x & 63;
-    const int strip = blockIdx.x * MWAVES + (threadIdx.x >> 6);  // uniform per wave
+    const int strip = blockIdx.x * MWAVES + wave_index();
     if (strip >= nstrips) return;
     const int s = find_scen(sc, nscen, strip);
     const Scen<R>& S = sc[s];
@@ -475,9 +493,14 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
     const RhsScale<R> scale(dt, dx);
 
     CellV<R> prev, cur, nxt;
-    const size_t colc = (size_t)(colmem ? col : nx + 1);  // lanes past the array load column nx+1
-    cell_load(prev, h, qx, qy, z, n2, colc + W * (size_t)(j0 - 1));
-    cell_load(cur, h, qx, qy, z, n2, colc + W * (size_t)j0);
+    // lane l's column of a row from the strip's first; lanes past the array load column nx+1
+    const unsigned at = (unsigned)min(lane, nx + 1 - tx * MW);
+    auto load_row = [&](CellV<R>& c, int row) {
+        const size_t o = (size_t)(tx * MW) + W * (size_t)row;
+        cell_load(c, row_base(h, o), row_base(qx, o), row_base(qy, o), row_base(z, o), row_base(n2, o), at);
+    };
+    load_row(prev, j0 - 1);
+    load_row(cur, j0);
     cell_derive(prev, hextra);
     // rhs*0 / rhs*1 of the previous row's cell (h, qx, qy)
     R p0[3] = {(R)0, (R)0, (R)0}, p1[3] = {(R)0, (R)0, (R)0};
@@ -488,7 +511,7 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
     for (int r = 0; r <= rend; r++) {
         const int j = j0 + r;
         // prefetch row j+1 while row j is solved
-        cell_load(nxt, h, qx, qy, z, n2, colc + W * (size_t)min(j + 1, ny + 1));  // unused at r == rend
+        load_row(nxt, min(j + 1, ny + 1));  // unused at r == rend
         cell_derive(cur, hextra);
         R c0[3] = {(R)0, (R)0, (R)0}, c1[3] = {(R)0, (R)0, (R)0};
         if (r < mr) {  // uniform: row j is a strip row
@@ -535,7 +558,7 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
         }
         // row j-1 is complete: update with implicit Manning friction (1046-1092) and rain
         if (r >= 1 && cell && j - 1 <= ny) {
-            const size_t c = (size_t)col + W * (size_t)(j - 1);
+            const size_t c = (size_t)(tx * MW) + W * (size_t)(j - 1);
             const R hn = prev.h, qxc = prev.qx, qyc = prev.qy;
             R hij, qxij, qyij;
             hij = hn - p0[0] - p1[0];
@@ -557,9 +580,9 @@ __global__ __launch_bounds__(BT) void k_flux_march(const Scen<R>* __restrict__ s
                     qyij = my;
                 }
             }
-            hout[c] = hij + rain * dt;
-            qxout[c] = qxij;
-            qyout[c] = qyij;
+            row_base(hout, c)[at] = hij + rain * dt;
+            row_base(qxout, c)[at] = qxij;
+            row_base(qyout, c)[at] = qyij;
         }
         prev = cur;
         cur = nxt;
@@ -659,7 +682,7 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
                                                   int par, Params P)
 {
     const int lane = threadIdx.x & 63;
-    const int strip = blockIdx.x * MWAVES + (threadIdx.x >> 6);  // uniform per wave
+    const int strip = blockIdx.x * MWAVES + wave_index();
     if (strip >= nstrips) return;
     const int s = find_scen(sc, nscen, strip);
     const Scen<R>& S = sc[s];
@@ -670,7 +693,6 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
     const size_t W = (size_t)nx + 2;
     const int col = tx * MW + lane;  // padded column of this lane
     const int j0 = ty * mr + 1;
-    const bool colmem = col <= nx + 1;
     const bool cell = lane >= 1 && lane <= MW && col <= nx;
     const int nr = min(mr, ny + 1 - j0);  // cell rows of the strip (j0 <= ny)
     const gmem<R>* h = to_global((const R*)S.h[par]);
@@ -682,8 +704,10 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
     // Rows ahead of their use, unconditionally: lanes past the array load its last column, and
     // rows past the strip a row inside the array; neither value is used (the next strip may be
     // writing such a qx or qy).
-    const size_t colc = (size_t)(colmem ? col : nx + 1);
-    auto ld = [&](const gmem<R>* a, int row) { return a[colc + W * (size_t)min(row, ny + 1)]; };
+    const unsigned at = (unsigned)min(lane, nx + 1 - tx * MW);
+    auto ld = [&](auto* a, int row) {
+        return row_base(a, (size_t)(tx * MW) + W * (size_t)min(row, ny + 1))[at];
+    };
     R cfl = RealLim<R>::max();
     double vs = 0.0, vc = 0.0;
     R hm = ld(h, j0 - 1), hc = ld(h, j0), hp = ld(h, j0 + 1), qxv = ld(qx, j0), qyv = ld(qy, j0);
@@ -705,17 +729,17 @@ __global__ __launch_bounds__(BT) void k_fix_march(const Scen<R>* __restrict__ sc
             zr = lane_shift<false>(zc);
         }
         if (cell) {
-            const size_t c = (size_t)col + W * (size_t)j;
+            const size_t c = (size_t)(tx * MW) + W * (size_t)j;
             const R hij = hc;
             if (MODE == 1 && hij > hextra) {  // triton_appfis.hpp:1095-1112
                 const R zij = zc;
                 if (((hij + zij < zr) && (hr < EPS12)) || ((hij + zij < zl) && (hl < EPS12))) {
                     qxv = (R)0.0;
-                    qx[c] = qxv;
+                    row_base(qx, c)[at] = qxv;
                 }
                 if (((hij + zij < zm) && (hm < EPS12)) || ((hij + zij < zp) && (hp < EPS12))) {
                     qyv = (R)0.0;
-                    qy[c] = qyv;
+                    row_base(qy, c)[at] = qyv;
                 }
             }
             if (hij > hextra) {  // triton_appfis.hpp:567-586
