@@ -431,18 +431,20 @@ constexpr int MWAVES = BT / 64;   // strips per block
 // Rows of a strip.  A strip solves its top edge row twice over (once per neighbour), so long
 // strips waste least, but a wave marches its rows one after the other: a grid cut into
 // fewer strips than the chip has SIMDs runs at the latency of one strip however small it is
-// (785 x 785 in FP64: 325 strips of 32 rows, 119 us a step, against 42 with 5 rows).  The
+// (785 x 785 in FP64: 325 strips of 32 rows, 120 us a step, against 42 with 5 rows).  The
 // blocks of a launch share the CUs, so a step takes about
 //     max(blocks per CU, rounded up, L) * (rows + E)
-// rows' time of a busy SIMD: E is the repeated work of a strip in rows (0.9 FP64, 1.2 FP32:
-// 4096 x 4096 in strips of 4, 8, 16 rows: 715, 661, 642 us; an FP32 ensemble of 12, 16, 32:
-// 702, 692, 687), and a wave alone on its SIMD takes L times a busy one's share of time per
-// row (FP64 3.2 against 2.2 us, FP32 1.8 against 0.8, both kernels of a step).  The choice is
-// the minimum over the lengths below; every value of the fields is the same for all of them.
+// rows' time of a busy SIMD: E is the repeated work of a strip in rows, and up to L blocks a CU
+// is as slow as with one, its waves waiting for their own results.  The choice is the minimum
+// over the lengths below; every value of the fields is the same for all of them.  L and E are
+// those whose choices come nearest the best measured length for 9 grids of 333^2 to 4096^2 and an
+// ensemble (FP64 within 0.5 % of it, FP32 4 %); us a step in strips of 4, 8, 16, 32 rows: FP64
+// 785^2 46, 55, 68, 120, 2048^2 177, 174, 186, 228, 4096^2 667, 620, 606, 635; FP32 2048^2 74, 73,
+// 76, 101, ensemble of 12 (from 8) 626, 609, 623.
 template <typename R>
 int strip_rows(int num_cu, int nscen, const int* nx, const int* ny)
 {
-    const double L = sizeof(R) == 8 ? 1.46 : 2.4, E = sizeof(R) == 8 ? 0.9 : 1.2;
+    const double L = sizeof(R) == 8 ? 2.1 : 2.2, E = sizeof(R) == 8 ? 0.4 : 0.2;
     int best = 32;
     double least = 0.0;
     for (int mr : {32, 28, 24, 20, 16, 14, 12, 10, 8, 7, 6, 5, 4, 3, 2, 1}) {
