@@ -13,6 +13,7 @@
 //         value is bit-identical to PLAIN.  HBM/MALL traffic per sweep drops by ~T.
 #include "common.hpp"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 #include <vector>
@@ -99,7 +100,9 @@ __device__ inline int grid_of_tile(const HeatGrid<T>* __restrict__ tab, int ngri
 //   FP64: sum - 4u as one FMA, 1.24 -> 1.20 (of these 0.02 are the check).  4u is exact where it
 //   does not overflow, so the FMA then rounds as the subtraction does.  `big` is the top word of a
 //   magnitude that the launch's sweeps cannot grow that far from; a block that loaded a larger one,
-//   an infinity or a NaN does its sweeps again with a multiply and a subtraction.
+//   an infinity or a NaN does its sweeps again with a multiply and a subtraction.  That loop is
+//   short and out of the way: a launch fetches its code anew (0.7 us a launch less than with
+//   two sweeps a trip in line).
 //   FP32: a row's update starts when the row two above it is done (an empty asm that takes both),
 //   which keeps the schedule from stretching over the whole column of rows: 0.889 -> 0.868, and
 //   2048^2 2.035 -> 1.978.  In FP64 the same costs 1 %, and the FMA's check costs FP32 5 %.
@@ -207,10 +210,11 @@ __device__ __forceinline__ void rt_tile(const T* __restrict__ u, T* __restrict__
     if (inner) sweeps(std::false_type{}, std::bool_constant<kFused>{});
     else sweeps(std::true_type{}, std::bool_constant<kFused>{});
     if constexpr (kFused)
-        if (__any(large[lane % NW])) {
+        if (__builtin_expect(__any(large[lane % NW]), 0)) {
             __syncthreads();  // the last sweep's edge rows have been read
             load();
-            sweeps(std::true_type{}, std::false_type{});
+#pragma clang loop unroll(disable)
+            for (int s = 0; s < steps; s++) sweep(std::true_type{}, std::false_type{}, s & 1);
         }
     // the centre: window columns TS .. TS+TX-1, rows TS .. TS+TY-1 (interior cells only).  The
     // column is made opaque: the loads' addresses would be kept in registers for the stores.
@@ -279,11 +283,16 @@ int run_plain(appfis_ctx* ctx, T* b0, T* b1, int nx, int ny, T c, int iters)
 // Split `iters` sweeps into launches of at most TS sweeps such that the number of
 // launches has the parity of `iters`: the field then ends in bufs[iters % 2], as
 // with one sweep per launch.
-inline int plan_launches(int iters, int ts, int* counts, int max_launches)
+inline int launch_count(int iters, int ts)
 {
     int n = (iters + ts - 1) / ts;
     if ((n & 1) != (iters & 1)) n++;
-    if (n > iters) n = iters;
+    return n > iters ? iters : n;
+}
+
+inline int plan_launches(int iters, int ts, int* counts, int max_launches)
+{
+    const int n = launch_count(iters, ts);
     if (n > max_launches) return -1;
     int base = iters / n, extra = iters % n;
     for (int l = 0; l < n; l++) counts[l] = base + (l < extra ? 1 : 0);
@@ -489,6 +498,58 @@ int run_ensemble(appfis_ctx* ctx, int ngrid, const int* nx, const int* ny, void*
     return APPFIS_OK;
 }
 
+// Tiles an ensemble may take.  Its launches take about
+//     launches * launch + sweeps * sweep * blocks per CU
+// us, blocks per CU being the mean of their number and of it rounded up, and at least a quarter:
+// the tiles are those of the least sum.  The constants are fitted to 26 ensembles of 4 to 64 grids
+// of 64 to 1024 cells a side and 20 to 200 sweeps; the choice is within 1 % of the best of ten
+// tilings on average, 9 % at most.  (FP64, us for all sweeps, in the order below: 8 grids up to 256,
+// 96 sweeps 158, 112, 101, 135; 30 up to 256, 96 sweeps 172, 173, 209, 150; 30 up to 512, 48
+// sweeps 185, 172, 260, 206; 64 up to 1024, 96 sweeps 1262, 1482, 2646, 1801.)
+struct HeatEnsemble {
+    int (*fn)(appfis_ctx*, int, const int*, const int*, void* const*, void* const*, double, int);
+    int tx, ty, ts;
+    double launch, sweep;
+};
+template <typename T, int K, int NW, int TS, int WPL>
+constexpr HeatEnsemble ensemble_tiles(double launch, double sweep)
+{
+    return {run_ensemble<T, K, NW, TS, WPL>, 64 * WPL - 2 * TS, NW * K - 2 * TS, TS, launch, sweep};
+}
+static const HeatEnsemble kEnsembleF64[] = {
+    ensemble_tiles<double, 8, 8, 8, 2>(5.95, 0.77),
+    ensemble_tiles<double, 6, 8, 8, 1>(4.65, 0.28),
+    ensemble_tiles<double, 4, 16, 16, 1>(5.98, 0.36),
+    ensemble_tiles<double, 5, 16, 16, 2>(5.3, 1.01),
+};
+static const HeatEnsemble kEnsembleF32[] = {
+    ensemble_tiles<float, 8, 8, 8, 2>(5.81, 0.45),
+    ensemble_tiles<float, 6, 8, 8, 1>(4.24, 0.19),
+    ensemble_tiles<float, 4, 16, 16, 1>(4.74, 0.25),
+    ensemble_tiles<float, 5, 16, 16, 2>(6.86, 0.5),
+};
+
+const HeatEnsemble& pick_ensemble(const HeatEnsemble (&tab)[4], int num_cu, int ngrid, const int* nx, const int* ny,
+                                  int iters)
+{
+    int best = 0;
+    double least = 0.0;
+    for (int i = 0; i < 4; i++) {
+        const HeatEnsemble& e = tab[i];
+        double blocks = 0.0;
+        for (int g = 0; g < ngrid; g++)
+            if (nx[g] > 0 && ny[g] > 0) blocks += (double)ceil_div(nx[g], e.tx) * ceil_div(ny[g], e.ty);
+        const double per_cu = blocks / (num_cu > 0 ? num_cu : 256);
+        const double cost = launch_count(iters, e.ts) * e.launch +
+                            iters * e.sweep * std::max(0.5 * (per_cu + std::ceil(per_cu)), 0.25);
+        if (i == 0 || cost < least) {
+            least = cost;
+            best = i;
+        }
+    }
+    return tab[best];
+}
+
 extern "C" int appfis_heat2d_ensemble(appfis_ctx* ctx, int dtype, int ngrid, const int* nx, const int* ny,
                                       void* const* buf0, void* const* buf1, double c, int iters)
 {
@@ -497,12 +558,10 @@ extern "C" int appfis_heat2d_ensemble(appfis_ctx* ctx, int dtype, int ngrid, con
     APPFIS_REQUIRE(ngrid >= 1, "heat2d ensemble: need at least one grid");
     APPFIS_REQUIRE(iters >= 0, "iters must be >= 0");
     if (iters == 0) return APPFIS_OK;
-    // 64 grids of 128 to 1024 cells a side, 200 sweeps: FP64 3.28 ms with two columns per lane,
-    // 3.45 with one; FP32 1.77 and 1.58.
     if (dtype == APPFIS_F64)
-        return run_ensemble<double, 8, 8, 8, 2>(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
+        return pick_ensemble(kEnsembleF64, ctx->num_cu, ngrid, nx, ny, iters).fn(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
     if (dtype == APPFIS_F32)
-        return run_ensemble<float, 14, 8, 8, 1>(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
+        return pick_ensemble(kEnsembleF32, ctx->num_cu, ngrid, nx, ny, iters).fn(ctx, ngrid, nx, ny, buf0, buf1, c, iters);
     return invalid("heat2d ensemble: dtype must be F64 or F32");
 }
 

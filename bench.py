@@ -369,7 +369,8 @@ def bench_heat_ensemble(ctx, hip, ngrid=64, iters=500):
         res[name] = [(a, b)[iters % 2].download().sum() for a, b, _, _ in grids[:2]]
         r = {"ms": round(ms, 3), "glups": round(cells * iters / (ms * 1e-3) / 1e9, 2)}
         if name == "ensemble":
-            # the FP64 ensemble runs 48 x 96 register tiles (7 rows x 16 waves), 8 sweeps per launch
+            # an FP64 ensemble of this size runs 112 x 48 register tiles (8 rows x 8 waves, two columns
+            # per lane), 8 sweeps per launch
             launches = len(_plan(iters, 8))
             r["roofline"] = roofline(16.0 * cells * iters / launches, ms / launches, "k_heat2d_rt_ens<double, 8, 8, 8, 2>")
         out[name] = r

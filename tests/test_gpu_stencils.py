@@ -119,6 +119,22 @@ def test_heat2d_ensemble_matches_oracle(ctx, dt, iters):
         assert np.array_equal((d0, d1)[iters % 2].download(), ref), (nx, ny)
 
 
+# ensembles for which the cost rule takes each of its tilings (most grids of the larger ones are
+# uneven by a cell, so all have partial tiles)
+@pytest.mark.parametrize("dt", [hip.F64, hip.F32])
+@pytest.mark.parametrize("ngrid,side,iters", [(3, 70, 15), (3, 70, 16), (24, 143, 15), (24, 200, 16)])
+def test_heat2d_ensemble_tilings(ctx, dt, ngrid, side, iters):
+    grids, refs = [], []
+    for k in range(ngrid):
+        nx, ny = side + k % 3, side - k % 5
+        a, d0, d1 = _heat_pair(ctx, nx, ny, dt, seed=2500 + k)
+        grids.append((d0, d1, nx, ny))
+        refs.append(oracle.heat2d(a.copy(), np.zeros_like(a), nx, ny, 0.1, iters))
+    ctx.heat2d_ensemble(grids, 0.1, iters)
+    for (d0, d1, nx, ny), ref in zip(grids, refs):
+        assert np.array_equal((d0, d1)[iters % 2].download(), ref), (nx, ny)
+
+
 def test_heat2d_ensemble_repeated_calls(ctx):
     # each call captures and replays its launch chain as a graph; three calls in a row on
     # the same grids (eager reductions between them) continue the same trajectory
