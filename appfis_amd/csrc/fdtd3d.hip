@@ -642,6 +642,8 @@ static const FdtdVariant kBF16[] = {FDTD16_VARIANTS(__hip_bfloat16)};
 //     256^3 FP32, ty8 ry2 d2 u18:    zc256 115  128 61  64 34  32 28  16 29   8 30  4 34  2 46
 //     256^3 BF16, vx2 ty8 ry2 u18:   zc256 230  128 117 64 61  32 35  16 25   8 27  4 29  2 36
 //     512^3 FP32, dma ty16 ry2 d2:   zc256 213  128 243 64 253 32 269 16 303
+// 16-bit fields past the 256 MB of last-level cache take W0 = 15, so longer chunks, of which fewer
+// stream at once (512^3 BF16 196 us against 201, 480^3 178 / 184; 300^3 54 / 48, so not below).
 // A grid smaller than the chip wants chunks of a few planes; 256 planes each left a 256^3 box
 // with 32 to 64 blocks on 256 CUs.
 int planes_per_block(const FdtdVariant& v, int dtype, int num_cu, int nx, int ny, int nz)
@@ -649,7 +651,8 @@ int planes_per_block(const FdtdVariant& v, int dtype, int num_cu, int nx, int ny
     const double cus = num_cu > 0 ? num_cu : 256;
     const double tiles = (double)ceil_div(nx, TXT * v.vx) * ceil_div(ny, v.ty * v.ry);
     const double P = v.wmod ? 3.8 : 1.5;
-    const double W0 = dtype == APPFIS_F64 ? 9.0 : dtype == APPFIS_F32 ? 12.0 : 18.0;
+    const bool streams = 2.0 * nx * ny * nz * (double)dtype_size(dtype) > 256.0 * (1 << 20);
+    const double W0 = dtype == APPFIS_F64 ? 9.0 : dtype == APPFIS_F32 ? 12.0 : streams ? 15.0 : 18.0;
     int best = nz;
     double least = 0.0;
     for (int zc = nz; zc >= (nz < 2 ? nz : 2); zc--) {
