@@ -192,7 +192,11 @@ __global__ __launch_bounds__(TXT* TY) void k_fdtd3d(const S* __restrict__ u, S* 
     const int W = nx + 2 * R, H = ny + 2 * R;
     const long long szl = (long long)W * H;
     const int plane_bytes = (int)(szl * (long long)sizeof(S));
-    const int tx = threadIdx.x, ty = threadIdx.y;
+    // A wave is a thread row.  With its number as a scalar the 16-bit tilings of 4 rows a thread, bound
+    // by their vector instructions, go from 173 to 151 registers and are the best of the large
+    // boxes (512^3 BF16 196 -> 188 us, 400^3 102 -> 95); the others gain nothing by it, or lose.
+    const int tx = threadIdx.x;
+    const int ty = sizeof(S) == 2 && RY == 4 ? __builtin_amdgcn_readfirstlane((int)threadIdx.y) : (int)threadIdx.y;
     const int tid = ty * TXT + tx;
     const int bx = tbx * PX + R, by = tby * PY + R;  // padded origin of the tile
     const int z0 = tbz * zc + R;
