@@ -340,9 +340,9 @@ int run_whole(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, double c, int
 {
     if (!whole_fits<K, NW, WPL>(nx, ny)) return run_rt<T, 8, 8, 8, 1>(ctx, b0, b1, nx, ny, c, iters, 8);
     T* buf[2] = {(T*)b0, (T*)b1};
-    const int n = iters & 1 ? 1 : 2;  // launches: their number has the parity of `iters`
+    const int n = launch_count(iters, 1024);  // a launch ends within a millisecond or so
     for (int l = 0; l < n; l++) {
-        const int steps = n == 1 ? iters : iters / 2;
+        const int steps = iters / n + (l < iters % n ? 1 : 0);
         hipLaunchKernelGGL((k_heat2d_whole<T, K, NW, WPL>), dim3(1), dim3(64 * NW), 0, ctx->stream, buf[l & 1],
                            buf[(l + 1) & 1], nx, ny, (T)c, steps, fused_limit(c, steps));
         APPFIS_LAUNCH_CHECK();

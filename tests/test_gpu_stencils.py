@@ -76,6 +76,14 @@ def test_heat2d_windows(ctx, dt, nx, ny, iters):
         assert np.array_equal((d0, d1)[iters % 2].download(), ref), variant
 
 
+def test_heat2d_whole_grid_launch_split(ctx):
+    # more sweeps than one launch of the one-block form takes
+    nx, ny, iters = 30, 41, 2311
+    a, d0, d1 = _heat_pair(ctx, nx, ny, hip.F64)
+    ctx.heat2d(d0, d1, nx, ny, 0.1, iters, hip.CANDIDATE0 + len(hip.heat2d_candidates(hip.F64)) - 1)
+    assert np.array_equal(d1.download(), oracle.heat2d(a.copy(), np.zeros_like(a), nx, ny, 0.1, iters))
+
+
 # infinities, NaN and magnitudes of which four are (or grow to be) past the type's largest: every
 # form has to give what the one-sweep form does, near them and in the tiles that hold none
 @pytest.mark.parametrize("dt", [hip.F64, hip.F32])
