@@ -245,8 +245,8 @@ __global__ __launch_bounds__(64 * NW) void k_heat2d_rt(const T* __restrict__ u, 
 }
 
 // A grid that fits one block's window, ghost ring included, needs no halo: its cells at the
-// window's edge are ghost cells, which keep their values, so any number of sweeps runs in one
-// launch of one block.
+// window's edge are ghost cells, which keep their values, so one launch of one block runs as many
+// sweeps as it is given.
 template <typename T, int K, int NW, int WPL>
 __global__ __launch_bounds__(64 * NW) void k_heat2d_whole(const T* __restrict__ u, T* __restrict__ v, int nx, int ny,
                                                           T c, int steps, unsigned big)
