@@ -33,6 +33,11 @@ struct appfis_ctx {
     // intermediates); grown on demand, kept until the context is destroyed
     void* work = nullptr;
     size_t work_bytes = 0;
+    // whether a call under graph capture has used the scratch or the workspace: the caller's
+    // graph holds its address from then on, so where it is replaced by a larger one the old
+    // one moves to `retired`, freed with the context, instead of being freed at once
+    bool scratch_lent = false, work_lent = false;
+    std::vector<void*> retired;
     // pinned host staging for small results
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
@@ -65,7 +70,8 @@ int invalid(const char* fmt, ...);
 // capture of their own, none of which a capture allows.
 int refuse_if_capturing(appfis_ctx* ctx, const char* what);
 
-// Ensure ctx->scratch holds at least `bytes`; returns status.
+// Ensure ctx->scratch (ctx->work) holds at least `bytes` for the launches that follow; returns
+// status.  A call under graph capture keeps the block for the context's life (see `retired`).
 int ensure_scratch(appfis_ctx* ctx, size_t bytes);
 int ensure_work(appfis_ctx* ctx, size_t bytes);
 int ensure_pinned(appfis_ctx* ctx, size_t bytes);

@@ -47,15 +47,35 @@ int refuse_if_capturing(appfis_ctx* ctx, const char* what)
     return APPFIS_ERR_UNSUPPORTED;
 }
 
+static bool capturing(appfis_ctx* ctx)
+{
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// Gives up a block of the context that a larger one replaces: freed, or kept until the context
+// is destroyed where a graph of the caller holds its address.  The stream must have drained.
+static int drop_block(appfis_ctx* ctx, void** block, size_t* bytes, bool* lent)
+{
+    if (*lent) ctx->retired.push_back(*block);
+    else APPFIS_HIP_CHECK(hipFree(*block));
+    *block = nullptr;
+    *bytes = 0;
+    *lent = false;
+    return APPFIS_OK;
+}
+
 int ensure_scratch(appfis_ctx* ctx, size_t bytes)
 {
-    if (ctx->scratch_bytes >= bytes) return APPFIS_OK;
+    if (ctx->scratch_bytes >= bytes) {
+        if (!ctx->scratch_lent) ctx->scratch_lent = capturing(ctx);
+        return APPFIS_OK;
+    }
     APPFIS_NOT_CAPTURING(ctx, "growing the context scratch");
     if (ctx->scratch) {
         APPFIS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
-        APPFIS_HIP_CHECK(hipFree(ctx->scratch));
-        ctx->scratch = nullptr;
-        ctx->scratch_bytes = 0;
+        int st = drop_block(ctx, &ctx->scratch, &ctx->scratch_bytes, &ctx->scratch_lent);
+        if (st) return st;
     }
     size_t want = bytes < 4096 ? 4096 : bytes;
     APPFIS_HIP_CHECK(hipMalloc(&ctx->scratch, want));
@@ -66,16 +86,18 @@ int ensure_scratch(appfis_ctx* ctx, size_t bytes)
 
 int ensure_work(appfis_ctx* ctx, size_t bytes)
 {
-    if (ctx->work_bytes >= bytes) return APPFIS_OK;
+    if (ctx->work_bytes >= bytes) {
+        if (!ctx->work_lent) ctx->work_lent = capturing(ctx);
+        return APPFIS_OK;
+    }
     APPFIS_NOT_CAPTURING(ctx, "growing the context workspace");
     if (ctx->work) {
         APPFIS_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         // the cached graphs hold pointers into the old workspace
         int st = clear_graphs(ctx);
         if (st) return st;
-        APPFIS_HIP_CHECK(hipFree(ctx->work));
-        ctx->work = nullptr;
-        ctx->work_bytes = 0;
+        st = drop_block(ctx, &ctx->work, &ctx->work_bytes, &ctx->work_lent);
+        if (st) return st;
     }
     APPFIS_HIP_CHECK(hipMalloc(&ctx->work, bytes));
     ctx->work_bytes = bytes;
@@ -96,12 +118,6 @@ int ensure_pinned(appfis_ctx* ctx, size_t bytes)
     APPFIS_HIP_CHECK(hipHostMalloc(&ctx->pinned, want, hipHostMallocDefault));
     ctx->pinned_bytes = want;
     return APPFIS_OK;
-}
-
-static bool capturing(appfis_ctx* ctx)
-{
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(ctx->stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
 }
 
 int ktime_begin(appfis_ctx* ctx)
@@ -338,6 +354,7 @@ int appfis_ctx_destroy(appfis_ctx* ctx)
     ctx->graphs.clear();
     if (ctx->scratch) note(hipFree(ctx->scratch));
     if (ctx->work) note(hipFree(ctx->work));
+    for (void* p : ctx->retired) note(hipFree(p));
     if (ctx->pinned) note(hipHostFree(ctx->pinned));
     if (ctx->ev_start) note(hipEventDestroy(ctx->ev_start));
     if (ctx->ev_stop) note(hipEventDestroy(ctx->ev_stop));

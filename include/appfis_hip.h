@@ -31,6 +31,10 @@
  *     appfis_kernel_timing's first enabling call, appfis_reduce, appfis_reduce_sum_wide,
  *     appfis_himeno, appfis_heat2d_ensemble, the flood entry points, a first CHOSEN
  *     call) returns APPFIS_ERR_UNSUPPORTED under capture and enqueues nothing.
+ *     Captured appfis_reduce_device and appfis_gol CHOSEN calls use the context's scratch and
+ *     workspace: replay their graphs on the context's stream, and not after the context is
+ *     destroyed.  A later call that needs more leaves the memory such graphs use in place
+ *     until then.
  */
 #ifndef APPFIS_HIP_H
 #define APPFIS_HIP_H

@@ -14,6 +14,7 @@ from appfis_amd import hip
 
 pytestmark = pytest.mark.gpu
 
+FDTD_COEFF = [0.5, 0.125, 0.125 / 2, 0.125 / 3, 0.125 / 4]
 NPDT = {hip.U8: np.uint8, hip.I32: np.int32, hip.F32: np.float32, hip.F64: np.float64, hip.F16: np.float16}
 
 
@@ -216,6 +217,50 @@ def test_graph_capture_of_plain_heat2d_and_device_reduction(ctx):
             assert abs(out.download()[0] - exp) <= 1e-14 * float(np.abs(ref).sum())
     finally:
         ctx.graph_destroy(g)
+
+
+def test_captured_calls_outlive_a_larger_workspace_and_scratch():
+    """A graph that holds addresses of the context's workspace (Life CHOSEN at a ragged width) and
+    scratch (the device reduction), replayed after later calls replaced both by larger ones and new
+    arrays may lie where the old ones were: every replay equals the oracle, and the arrays keep
+    their values."""
+    import ctypes as C
+
+    nx, ny, gens = 100, 90, 7
+    a = np.zeros((ny + 2, nx + 2), dtype=np.uint8)
+    oracle.fill_bernoulli(a, 1, 91, 0.3)
+    with hip.Context(0) as c:
+        L = hip.lib()
+        d0, d1, out = c.from_numpy(a), c.array(a.shape, hip.U8), c.array((1,), hip.I64)
+        dims = (C.c_int * 2)(nx + 2, ny + 2)
+        box = (C.c_int * 4)(1, nx + 1, 1, ny + 1)
+
+        def chain():
+            c.gol(d0, d1, nx, ny, gens, hip.CHOSEN)
+            hip.check(L.appfis_reduce_device(c.handle, d1.ptr, hip.U8, 2, dims, box, hip.SUM, out.ptr), "reduce")
+
+        chain()  # sizes both
+        c.graph_begin()
+        chain()
+        g = c.graph_end()
+        f0, f1 = c.array((24, 24, 24), hip.F64), c.array((24, 24, 24), hip.F64)
+        c.fdtd3d(f0, f1, 16, 16, 16, FDTD_COEFF, 2, hip.CHOSEN)  # a larger workspace
+        h = [c.array((5, 5, 5), hip.F32) for _ in range(14)]
+        c.himeno(h, 5, 5, 5, 0.8, 6000)  # a larger scratch
+        held = [c.array((1 << k,), hip.U8) for k in (11, 12, 12, 13, 14, 15, 15, 16, 17)]
+        for x in held:
+            c.fill_value(x, 173)
+        for rep in range(3):
+            b = np.roll(a, 5 * rep, axis=0)
+            b[[0, -1]] = 0
+            d0.upload(b)
+            c.graph_launch(g, 1)
+            c.sync()
+            ref = oracle.gol_u8(b.copy(), np.zeros_like(b), nx, ny, gens)
+            assert np.array_equal(d1.download(), ref)
+            assert out.download()[0] == int(ref[1:-1, 1:-1].sum())
+            assert all((x.download() == 173).all() for x in held)
+        c.graph_destroy(g)
 
 
 def test_kernel_timing_of_gol_calls(ctx):
