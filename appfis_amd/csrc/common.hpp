@@ -18,6 +18,7 @@
 struct appfis_tune_entry {
     int key[6];
     int choice;
+    int param = 0;  // what the variant runs with, where a rule sets it (FDTD3d: planes per block)
     std::string report;
 };
 
@@ -117,6 +118,7 @@ inline size_t dtype_size(int dtype)
 // run_variant(i) must enqueue the timed work of candidate i on ctx->stream (on scratch
 // buffers, never on the caller's data) and return a status; each candidate is run once
 // untimed, then `reps` times under hipEvents; the fastest mean wins.
+const appfis_tune_entry* tuned_entry(const appfis_ctx* ctx, const int key[6]);  // null: not tuned yet
 int tune_select(appfis_ctx* ctx, const int key[6], int ncand, const char* const* names,
                 const std::function<int(int)>& run_variant, int reps, int* choice);
 

@@ -193,14 +193,20 @@ int cached_graph(appfis_ctx* ctx, std::vector<uint64_t> key, const std::function
     return APPFIS_OK;
 }
 
+const appfis_tune_entry* tuned_entry(const appfis_ctx* ctx, const int key[6])
+{
+    for (const appfis_tune_entry& e : ctx->tuned)
+        if (memcmp(e.key, key, sizeof(e.key)) == 0) return &e;
+    return nullptr;
+}
+
 int tune_select(appfis_ctx* ctx, const int key[6], int ncand, const char* const* names,
                 const std::function<int(int)>& run_variant, int reps, int* choice)
 {
-    for (const appfis_tune_entry& e : ctx->tuned)
-        if (memcmp(e.key, key, sizeof(e.key)) == 0) {
-            *choice = e.choice;
-            return APPFIS_OK;
-        }
+    if (const appfis_tune_entry* e = tuned_entry(ctx, key)) {
+        *choice = e->choice;
+        return APPFIS_OK;
+    }
     APPFIS_NOT_CAPTURING(ctx, "autotuning (the first CHOSEN call for a shape)");
     std::string rep = "autotune kernel " + std::to_string(key[0]) + " dtype " + std::to_string(key[1]) + " shape " +
                       std::to_string(key[2]) + "x" + std::to_string(key[3]) + "x" + std::to_string(key[4]) + ":";

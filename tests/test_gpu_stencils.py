@@ -8,6 +8,7 @@ for a few sweeps plus size-independent properties for the full sweep count.
 import hashlib
 import json
 import os
+import time
 
 import numpy as np
 import pytest
@@ -465,6 +466,23 @@ def test_fdtd3d_tilings_by_size(ctx, dt, n):
     for variant in (hip.PLAIN, hip.CHOSEN):
         ctx.fdtd3d(d0, d1, nx, ny, nz, coeff, 1, variant)
         assert np.array_equal(d1.download(), ref)
+
+
+def test_fdtd3d_chosen_call_costs_the_host_no_tuning(ctx):
+    # a call on a tuned shape launches its kernel and no more, whatever the number of planes:
+    # preparing the tuning took this column 100 ms and more of the host's time, a launch takes
+    # some 10 us
+    n = (1, 1, 1000000)
+    _, d0, d1 = _fdtd_pair(ctx, n, hip.F32)
+    ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 1, hip.CHOSEN)
+    ctx.sync()
+    t = []
+    for _ in range(3):
+        t0 = time.perf_counter()
+        ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 1, hip.CHOSEN)
+        t.append(time.perf_counter() - t0)
+        ctx.sync()
+    assert min(t) < 5e-3, t
 
 
 @pytest.mark.parametrize("dt,off", [(hip.F32, 4), (hip.F64, 8), (hip.F16, 2), (hip.BF16, 2)])
