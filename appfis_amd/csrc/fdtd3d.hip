@@ -555,10 +555,18 @@ int run(appfis_ctx* ctx, S* b0, S* b1, int nx, int ny, int nz, const double* cf,
     return APPFIS_OK;
 }
 
+// Blocks of `kernel` that a CU holds at once (registers and LDS).
+int resident_blocks(const void* kernel, int threads)
+{
+    int n = 0;
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, 0) == hipSuccess && n > 0 ? n : 1;
+}
+
 typedef int (*fdtd_fn)(appfis_ctx*, void*, void*, int, int, int, const double*, int, int);
 struct FdtdVariant {
     const char* name;
     fdtd_fn fn;
+    int (*resident)();  // resident_blocks of its kernel, asked once
     int ty, ry;    // thread rows (one wave each), rows per thread: a tile is 64*vx x ty*ry points
     int zc;        // planes per block where the candidate is forced
     bool pairs;    // 16-bit storage moved in 32-bit pairs: needs 4-byte aligned buffers
@@ -573,101 +581,143 @@ int run_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const dou
     return run<S, VX, TY, RY, D, U>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps, zc);
 }
 
+template <typename S, int VX, int TY, int RY, int D, int U>
+int res_v()
+{
+    static const int n = resident_blocks((const void*)k_fdtd3d<S, VX, TY, RY, D, U>, TXT * TY);
+    return n;
+}
+
 template <typename S, int TY, int RY, int D>
 int run_dma_v(appfis_ctx* ctx, void* b0, void* b1, int nx, int ny, int nz, const double* cf, int steps, int zc)
 {
     return run_dma<S, TY, RY, D>(ctx, (S*)b0, (S*)b1, nx, ny, nz, cf, steps, zc);
 }
 
+template <typename S, int TY, int RY, int D>
+int res_dma_v()
+{
+    static const int n = resident_blocks((const void*)k_fdtd3d_dma<S, TY, RY, D>, TXT * TY);
+    return n;
+}
+
+// a 16-bit tiling of two points a lane moves pairs
+template <typename S, int VX, int TY, int RY, int D, int U>
+constexpr FdtdVariant tiling(const char* name, int zc)
+{
+    return {name, run_v<S, VX, TY, RY, D, U>, res_v<S, VX, TY, RY, D, U>, TY, RY, zc, sizeof(S) == 2 && VX == 2, VX};
+}
+template <typename S, int TY, int RY, int D>
+constexpr FdtdVariant dma_tiling(const char* name, int zc)
+{
+    return {name, run_dma_v<S, TY, RY, D>, res_dma_v<S, TY, RY, D>, TY, RY, zc, false, 1, 4};
+}
+
 // Candidate tilings (VX x-points per thread, TY thread rows, RY rows per thread, zc
 // planes per block, D-deep prefetch, U-step unroll: 18 rotates the queue).
 static const FdtdVariant kF32[] = {
-    {"vx1 ty16 ry2 zc256 d4 u4", run_v<float, 1, 16, 2, 4, 4>, 16, 2, 256, false, 1},
-    {"vx1 ty8 ry4 zc256 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 256, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<float, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},
-    {"vx1 ty8 ry4 zc64 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 64, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u18", run_v<float, 1, 4, 4, 2, 18>, 4, 4, 64, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<float, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u18", run_v<float, 1, 8, 2, 2, 18>, 8, 2, 64, false, 1},
-    {"vx1 ty4 ry4 zc32 d2 u2", run_v<float, 1, 4, 4, 2, 2>, 4, 4, 32, false, 1},
-    {"vx1 ty8 ry4 zc128 d2 u2", run_v<float, 1, 8, 4, 2, 2>, 8, 4, 128, false, 1},
-    {"vx1 ty4 ry4 zc64 d3 u6", run_v<float, 1, 4, 4, 3, 6>, 4, 4, 64, false, 1},
-    {"vx1 ty16 ry2 zc64 d2 u2", run_v<float, 1, 16, 2, 2, 2>, 16, 2, 64, false, 1},
-    {"vx1 ty8 ry4 zc128 d3 u6", run_v<float, 1, 8, 4, 3, 6>, 8, 4, 128, false, 1},
-    {"vx1 ty16 ry2 zc256 d2 u2", run_v<float, 1, 16, 2, 2, 2>, 16, 2, 256, false, 1},
-    {"vx1 ty8 ry4 zc256 d4 u4", run_v<float, 1, 8, 4, 4, 4>, 8, 4, 256, false, 1},
-    {"vx1 ty8 ry4 zc256 d6 u6", run_v<float, 1, 8, 4, 6, 6>, 8, 4, 256, false, 1},
-    {"vx1 ty8 ry2 zc256 d4 u4", run_v<float, 1, 8, 2, 4, 4>, 8, 2, 256, false, 1},
-    {"vx2 ty8 ry2 zc256 d4 u4", run_v<float, 2, 8, 2, 4, 4>, 8, 2, 256, false, 2},
-    {"vx2 ty16 ry1 zc256 d4 u4", run_v<float, 2, 16, 1, 4, 4>, 16, 1, 256, false, 2},
-    {"vx2 ty16 ry1 zc256 d6 u6", run_v<float, 2, 16, 1, 6, 6>, 16, 1, 256, false, 2},
+    tiling<float, 1, 16, 2, 4, 4>("vx1 ty16 ry2 zc256 d4 u4", 256),
+    tiling<float, 1, 8, 4, 2, 2>("vx1 ty8 ry4 zc256 d2 u2", 256),
+    tiling<float, 1, 4, 4, 2, 2>("vx1 ty4 ry4 zc64 d2 u2", 64),
+    tiling<float, 1, 8, 4, 2, 2>("vx1 ty8 ry4 zc64 d2 u2", 64),
+    tiling<float, 1, 4, 4, 2, 18>("vx1 ty4 ry4 zc64 d2 u18", 64),
+    tiling<float, 1, 4, 2, 2, 18>("vx1 ty4 ry2 zc64 d2 u18", 64),
+    tiling<float, 1, 8, 2, 2, 18>("vx1 ty8 ry2 zc64 d2 u18", 64),
+    tiling<float, 1, 4, 4, 2, 2>("vx1 ty4 ry4 zc32 d2 u2", 32),
+    tiling<float, 1, 8, 4, 2, 2>("vx1 ty8 ry4 zc128 d2 u2", 128),
+    tiling<float, 1, 4, 4, 3, 6>("vx1 ty4 ry4 zc64 d3 u6", 64),
+    tiling<float, 1, 16, 2, 2, 2>("vx1 ty16 ry2 zc64 d2 u2", 64),
+    tiling<float, 1, 8, 4, 3, 6>("vx1 ty8 ry4 zc128 d3 u6", 128),
+    tiling<float, 1, 16, 2, 2, 2>("vx1 ty16 ry2 zc256 d2 u2", 256),
+    tiling<float, 1, 8, 4, 4, 4>("vx1 ty8 ry4 zc256 d4 u4", 256),
+    tiling<float, 1, 8, 4, 6, 6>("vx1 ty8 ry4 zc256 d6 u6", 256),
+    tiling<float, 1, 8, 2, 4, 4>("vx1 ty8 ry2 zc256 d4 u4", 256),
+    tiling<float, 2, 8, 2, 4, 4>("vx2 ty8 ry2 zc256 d4 u4", 256),
+    tiling<float, 2, 16, 1, 4, 4>("vx2 ty16 ry1 zc256 d4 u4", 256),
+    tiling<float, 2, 16, 1, 6, 6>("vx2 ty16 ry1 zc256 d6 u6", 256),
     // tiles loaded straight into LDS (k_fdtd3d_dma): "dma ty.. ry.. zc.. d.."
-    {"dma ty16 ry2 zc256 d2", run_dma_v<float, 16, 2, 2>, 16, 2, 256, false, 1, 4},
-    {"dma ty16 ry2 zc256 d3", run_dma_v<float, 16, 2, 3>, 16, 2, 256, false, 1, 4},
-    {"dma ty8 ry4 zc256 d2", run_dma_v<float, 8, 4, 2>, 8, 4, 256, false, 1, 4},
-    {"dma ty16 ry2 zc128 d2", run_dma_v<float, 16, 2, 2>, 16, 2, 128, false, 1, 4},
+    dma_tiling<float, 16, 2, 2>("dma ty16 ry2 zc256 d2", 256),
+    dma_tiling<float, 16, 2, 3>("dma ty16 ry2 zc256 d3", 256),
+    dma_tiling<float, 8, 4, 2>("dma ty8 ry4 zc256 d2", 256),
+    dma_tiling<float, 16, 2, 2>("dma ty16 ry2 zc128 d2", 128),
 };
 static const FdtdVariant kF64[] = {
-    {"vx1 ty8 ry2 zc256 d4 u4", run_v<double, 1, 8, 2, 4, 4>, 8, 2, 256, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u2", run_v<double, 1, 8, 2, 2, 2>, 8, 2, 64, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u2", run_v<double, 1, 4, 2, 2, 2>, 4, 2, 64, false, 1},
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<double, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},
-    {"vx1 ty4 ry2 zc128 d2 u2", run_v<double, 1, 4, 2, 2, 2>, 4, 2, 128, false, 1},
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<double, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},
-    {"vx1 ty8 ry2 zc64 d2 u18", run_v<double, 1, 8, 2, 2, 18>, 8, 2, 64, false, 1},
-    {"vx1 ty8 ry2 zc256 d2 u2", run_v<double, 1, 8, 2, 2, 2>, 8, 2, 256, false, 1},
-    {"vx1 ty4 ry4 zc256 d2 u2", run_v<double, 1, 4, 4, 2, 2>, 4, 4, 256, false, 1},
-    {"vx1 ty8 ry2 zc128 d2 u18", run_v<double, 1, 8, 2, 2, 18>, 8, 2, 128, false, 1},
-    {"vx1 ty4 ry4 zc256 d4 u4", run_v<double, 1, 4, 4, 4, 4>, 4, 4, 256, false, 1},
-    {"vx2 ty8 ry2 zc256 d2 u2", run_v<double, 2, 8, 2, 2, 2>, 8, 2, 256, false, 2},
-    {"vx2 ty16 ry1 zc256 d2 u2", run_v<double, 2, 16, 1, 2, 2>, 16, 1, 256, false, 2},
-    {"vx1 ty16 ry1 zc256 d4 u4", run_v<double, 1, 16, 1, 4, 4>, 16, 1, 256, false, 1},
+    tiling<double, 1, 8, 2, 4, 4>("vx1 ty8 ry2 zc256 d4 u4", 256),
+    tiling<double, 1, 8, 2, 2, 2>("vx1 ty8 ry2 zc64 d2 u2", 64),
+    tiling<double, 1, 4, 2, 2, 2>("vx1 ty4 ry2 zc64 d2 u2", 64),
+    tiling<double, 1, 4, 4, 2, 2>("vx1 ty4 ry4 zc64 d2 u2", 64),
+    tiling<double, 1, 4, 2, 2, 2>("vx1 ty4 ry2 zc128 d2 u2", 128),
+    tiling<double, 1, 4, 2, 2, 18>("vx1 ty4 ry2 zc64 d2 u18", 64),
+    tiling<double, 1, 8, 2, 2, 18>("vx1 ty8 ry2 zc64 d2 u18", 64),
+    tiling<double, 1, 8, 2, 2, 2>("vx1 ty8 ry2 zc256 d2 u2", 256),
+    tiling<double, 1, 4, 4, 2, 2>("vx1 ty4 ry4 zc256 d2 u2", 256),
+    tiling<double, 1, 8, 2, 2, 18>("vx1 ty8 ry2 zc128 d2 u18", 128),
+    tiling<double, 1, 4, 4, 4, 4>("vx1 ty4 ry4 zc256 d4 u4", 256),
+    tiling<double, 2, 8, 2, 2, 2>("vx2 ty8 ry2 zc256 d2 u2", 256),
+    tiling<double, 2, 16, 1, 2, 2>("vx2 ty16 ry1 zc256 d2 u2", 256),
+    tiling<double, 1, 16, 1, 4, 4>("vx1 ty16 ry1 zc256 d4 u4", 256),
 };
 #define FDTD16_VARIANTS(S)                                                 \
-    {"vx1 ty4 ry2 zc64 d2 u18", run_v<S, 1, 4, 2, 2, 18>, 4, 2, 64, false, 1},      \
-    {"vx1 ty4 ry4 zc64 d2 u18", run_v<S, 1, 4, 4, 2, 18>, 4, 4, 64, false, 1},      \
-    {"vx1 ty4 ry4 zc64 d2 u2", run_v<S, 1, 4, 4, 2, 2>, 4, 4, 64, false, 1},        \
-    {"vx1 ty8 ry4 zc64 d2 u2", run_v<S, 1, 8, 4, 2, 2>, 8, 4, 64, false, 1},        \
-    {"vx2 ty4 ry4 zc64 d2 u18", run_v<S, 2, 4, 4, 2, 18>, 4, 4, 64, true, 2},       \
-    {"vx2 ty4 ry2 zc64 d2 u18", run_v<S, 2, 4, 2, 2, 18>, 4, 2, 64, true, 2},       \
-    {"vx2 ty8 ry2 zc64 d2 u18", run_v<S, 2, 8, 2, 2, 18>, 8, 2, 64, true, 2},       \
-    {"vx2 ty4 ry4 zc64 d2 u2", run_v<S, 2, 4, 4, 2, 2>, 4, 4, 64, true, 2},        \
-    {"vx2 ty8 ry2 zc128 d2 u18", run_v<S, 2, 8, 2, 2, 18>, 8, 2, 128, true, 2}
+    tiling<S, 1, 4, 2, 2, 18>("vx1 ty4 ry2 zc64 d2 u18", 64), \
+    tiling<S, 1, 4, 4, 2, 18>("vx1 ty4 ry4 zc64 d2 u18", 64), \
+    tiling<S, 1, 4, 4, 2, 2>("vx1 ty4 ry4 zc64 d2 u2", 64), \
+    tiling<S, 1, 8, 4, 2, 2>("vx1 ty8 ry4 zc64 d2 u2", 64), \
+    tiling<S, 2, 4, 4, 2, 18>("vx2 ty4 ry4 zc64 d2 u18", 64), \
+    tiling<S, 2, 4, 2, 2, 18>("vx2 ty4 ry2 zc64 d2 u18", 64), \
+    tiling<S, 2, 8, 2, 2, 18>("vx2 ty8 ry2 zc64 d2 u18", 64), \
+    tiling<S, 2, 4, 4, 2, 2>("vx2 ty4 ry4 zc64 d2 u2", 64), \
+    tiling<S, 2, 8, 2, 2, 18>("vx2 ty8 ry2 zc128 d2 u18", 128)
 static const FdtdVariant kF16[] = {FDTD16_VARIANTS(__half)};
 static const FdtdVariant kBF16[] = {FDTD16_VARIANTS(__hip_bfloat16)};
 
-// Planes per block of tiling v on an nx x ny x nz interior.  With m blocks to a CU (rounded up),
-// TY waves each, a sweep takes about
-//     max(m * TY * (zc + P), W0 * (zc + 9))
+// Planes per block of tiling v on an nx x ny x nz interior.  With m blocks to a CU (rounded up), of
+// which `res` run at once, TY waves each, a sweep takes about
+//     max(m * TY * (zc + P), ceil(m / res) * W * (zc + 8))
 // times a constant: the first where the CUs are busy, P the planes' worth of a block's prologue
 // (it reads 8 planes before its first and the direct-to-LDS form fills its ring), the second
-// where they are not: W0 waves keep a CU's loads in flight, fewer take as long, and the prologue
-// is then 9 planes' latency.  Fitted to sweeps with chunks of 2 to 256 planes (us):
-//     256^3 FP32, ty8 ry2 d2 u18:    zc256 115  128 61  64 34  32 28  16 29   8 30  4 34  2 46
-//     256^3 BF16, vx2 ty8 ry2 u18:   zc256 230  128 117 64 61  32 35  16 25   8 27  4 29  2 36
-//     512^3 FP32, dma ty16 ry2 d2:   zc256 213  128 243 64 253 32 269 16 303
-// 16-bit fields past the 256 MB of last-level cache take W0 = 15, so longer chunks, of which fewer
-// stream at once (512^3 BF16 196 us against 201, 480^3 178 / 184; 300^3 54 / 48, so not below).
-// A grid smaller than the chip wants chunks of a few planes; 256 planes each left a 256^3 box
-// with 32 to 64 blocks on 256 CUs.
+// where they are not: W waves keep a CU's loads in flight, fewer take as long, more where a row
+// leaves lanes without a point.  In fields of FP32 and FP64 past the 256 MB of last-level cache
+// blocks that start in a second round no longer march beside their neighbours in y, and their
+// halo rows come from memory again: 15 % more.  Fitted to the sweeps of every tiling with chunks of
+// 2 planes to all on 28 grids of 16^3 to 640^3 points: the fastest tiling with the rule's planes is 1 %
+// over the best of all planes on average, 9 % at most.  us a sweep:
+//     256^3 FP32, ty8 ry2 d2 u18:    zc128 61  64 34  32 28  16 29   8 30  4 34  2 46
+//     512^3 FP32, dma ty16 ry2 d2:   zc512 350  256 212  128 241  64 254  32 269  16 302
+//     512^3 FP32, dma ty8 ry4 d2:    zc512 388  256 215  128 241  64 255  32 271  16 309
+//     384^3 FP32, dma ty16 ry2 d2:   zc384 255  192 141  128 106  55 115  28 122  16 134
+//     512^3 FP64, vx2 ty16 ry1 d2:   zc512 698  256 461  128 480  64 488  32 511  16 558
+//     1024 x 1024 x 16 BF16, vx2 ty8 ry2: zc16 24.2  8 26.6
+// The direct-to-LDS form holds 96 KB of a CU's 160, so its blocks never run together.
+// The chunk counts tried are those that fill the CUs m = 1, 2, .. blocks deep, to 8 rounds, and
+// the first four: a few dozen whatever nz is.
 int planes_per_block(const FdtdVariant& v, int dtype, int num_cu, int nx, int ny, int nz)
 {
     const double cus = num_cu > 0 ? num_cu : 256;
-    const double tiles = (double)ceil_div(nx, TXT * v.vx) * ceil_div(ny, v.ty * v.ry);
-    const double P = v.wmod ? 3.8 : 1.5;
-    const bool streams = 2.0 * nx * ny * nz * (double)dtype_size(dtype) > 256.0 * (1 << 20);
-    const double W0 = dtype == APPFIS_F64 ? 9.0 : dtype == APPFIS_F32 ? 12.0 : streams ? 15.0 : 18.0;
-    int best = nz;
+    const int tiles_x = (int)ceil_div(nx, TXT * v.vx), res = v.resident();
+    const double tiles = (double)tiles_x * ceil_div(ny, v.ty * v.ry);
+    const double P = v.wmod ? 5.0 : 0.5;
+    const bool streams = dtype_size(dtype) >= 4 && 2.0 * nx * ny * nz * (double)dtype_size(dtype) > 256.0 * (1 << 20);
+    const double lanes = (double)nx / ((double)tiles_x * TXT * v.vx);
+    const double W = (dtype == APPFIS_F32 ? 8.5 : dtype == APPFIS_F64 ? 14.0 : 16.0) / std::sqrt(lanes);
+    const int most = (nz + 1) / 2;  // chunks of two planes
+    int best = nz, last = 0;
     double least = 0.0;
-    for (int zc = nz; zc >= (nz < 2 ? nz : 2); zc--) {
-        const int chunks = (int)ceil_div(nz, zc);
-        if ((int)ceil_div(nz, chunks) != zc) continue;  // the same chunks in shorter blocks follow
-        const double m = std::ceil(tiles * chunks / cus);
-        const double cost = std::max(m * v.ty * (zc + P), W0 * (zc + 9.0));
+    auto consider = [&](int chunks) {
+        const int zc = (int)ceil_div(nz, std::max(1, std::min(chunks, most)));
+        if (zc == last) return;
+        last = zc;
+        const double m = std::ceil(tiles * ceil_div(nz, zc) / cus);
+        double cost = std::max(m * v.ty * (zc + P), std::ceil(m / res) * W * (zc + 8.0));
+        if (streams && m > res) cost *= 1.15;
         if (least == 0.0 || cost < least) {
             least = cost;
             best = zc;
         }
+    };
+    for (int c = 1; c <= 4; c++) consider(c);
+    for (int m = 1, c = 0; m <= 8 * res && c < most; m++) {
+        c = (int)(m * cus / tiles);
+        consider(c);
     }
     return best;
 }

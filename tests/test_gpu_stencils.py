@@ -485,6 +485,33 @@ def test_fdtd3d_chosen_call_costs_the_host_no_tuning(ctx):
     assert min(t) < 5e-3, t
 
 
+def test_fdtd3d_plain_call_costs_the_host_no_loop_over_planes(ctx):
+    # the planes of a block are chosen from a few dozen counts: trying every one took this column
+    # some 30 ms of the host's time in each call, a launch takes some 10 us
+    n = (1, 1, 4000000)
+    _, d0, d1 = _fdtd_pair(ctx, n, hip.F16)
+    ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 1, hip.PLAIN)
+    ctx.sync()
+    t = []
+    for _ in range(3):
+        t0 = time.perf_counter()
+        ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 1, hip.PLAIN)
+        t.append(time.perf_counter() - t0)
+        ctx.sync()
+    assert min(t) < 5e-3, t
+
+
+def test_fdtd3d_streaming_tilings_keep_long_blocks(ctx):
+    # 512^3 in FP32: the direct-to-LDS tilings, one block to a CU, march 256 planes each (128 in two
+    # rounds take 241 us a sweep for 212)
+    n = (512, 512, 512)
+    d0, d1 = (ctx.array(tuple(x + 8 for x in n), hip.F32) for _ in range(2))
+    ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 2, hip.CHOSEN)
+    report = [x for x in ctx.tune_report().splitlines() if "kernel 3 dtype 2 shape 512x512x512" in x][-1]
+    for tiling in ("dma ty16 ry2 zc256 d2", "dma ty16 ry2 zc256 d3", "dma ty8 ry4 zc256 d2"):
+        assert tiling in report, report
+
+
 @pytest.mark.parametrize("dt,off", [(hip.F32, 4), (hip.F64, 8), (hip.F16, 2), (hip.BF16, 2)])
 def test_fdtd3d_on_unaligned_buffers(ctx, dt, off):
     # buffers that start `off` bytes into an allocation, so that the preferred tilings'
