@@ -780,6 +780,8 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
     auto fits = [&](const FdtdVariant& v) {
         return nx % v.vx == 0 && (!v.pairs || aligned4) && (v.wmod == 0 || ((nx + 8) % v.wmod == 0 && aligned16));
     };
+    // a launch has at most 65536 tiles in y
+    auto rows_fit = [&](const FdtdVariant& v) { return ceil_div(ny, v.ty * v.ry) <= 65536; };
     if (variant >= APPFIS_CANDIDATE0) {
         const int i = variant - APPFIS_CANDIDATE0;
         APPFIS_REQUIRE(i < ntab, "fdtd3d: candidate %d out of range (%d candidates)", i, ntab);
@@ -818,6 +820,11 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
             name = cells <= 32 * M ? "vx2 ty4 ry2 zc64 d2 u18" : "vx2 ty8 ry2 zc128 d2 u18";
         else
             name = cells <= M ? "vx1 ty4 ry2 zc64 d2 u18" : "vx1 ty4 ry4 zc64 d2 u18";
+        // boxes of more rows than low tiles reach take the tallest that fits any width
+        if (!rows_fit(*find(tab, ntab, name)))
+            name = dtype == APPFIS_F32   ? "vx1 ty16 ry2 zc256 d4 u4"
+                   : dtype == APPFIS_F64 ? "vx1 ty8 ry2 zc256 d4 u4"
+                                         : "vx1 ty8 ry4 zc64 d2 u2";
         const FdtdVariant& v = *find(tab, ntab, name);
         return v.fn(ctx, buf0, buf1, nx, ny, nz, coeff5, steps, planes(v));
     }
@@ -832,9 +839,10 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
     APPFIS_NOT_CAPTURING(ctx, "appfis_fdtd3d CHOSEN's first call for a shape (autotuning)");
     std::vector<int> cand, zcs;
     std::vector<std::string> tilings, text;
+    const bool low = std::any_of(tab, tab + ntab, [&](const FdtdVariant& v) { return fits(v) && rows_fit(v); });
     for (int i = 0; i < ntab; i++) {
         const std::string t = name_with(tab[i], 0);
-        if (!fits(tab[i]) || std::find(tilings.begin(), tilings.end(), t) != tilings.end()) continue;
+        if (!fits(tab[i]) || (low && !rows_fit(tab[i])) || std::find(tilings.begin(), tilings.end(), t) != tilings.end()) continue;
         cand.push_back(i);
         zcs.push_back(planes(tab[i]));
         tilings.push_back(t);

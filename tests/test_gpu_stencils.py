@@ -501,6 +501,18 @@ def test_fdtd3d_plain_call_costs_the_host_no_loop_over_planes(ctx):
     assert min(t) < 5e-3, t
 
 
+@pytest.mark.parametrize("dt", [hip.F32, hip.F64, hip.BF16])
+def test_fdtd3d_more_rows_than_low_tiles_reach(ctx, dt):
+    # 540000 rows are 67500 tiles of 8 rows, over a launch's 65536: taller tiles take them
+    n = (1, 540000, 1)
+    a, d0, d1 = _fdtd_pair(ctx, n, dt)
+    ref = oracle.fdtd3d(a.copy(), np.zeros_like(a), *n, FDTD_COEFF, 1, bf16=(dt == hip.BF16))
+    for variant in (hip.PLAIN, hip.CHOSEN):
+        d1.upload(np.zeros_like(a))
+        ctx.fdtd3d(d0, d1, *n, FDTD_COEFF, 1, variant)
+        assert np.array_equal(d1.download(), ref), variant
+
+
 def test_fdtd3d_streaming_tilings_keep_long_blocks(ctx):
     # 512^3 in FP32: the direct-to-LDS tilings, one block to a CU, march 256 planes each (128 in two
     # rounds take 241 us a sweep for 212)
