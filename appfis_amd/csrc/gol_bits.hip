@@ -76,6 +76,47 @@ __global__ __launch_bounds__(256) void k_pack(const uint8_t* __restrict__ u, uin
     P[t] = word;
 }
 
+// One generation of a board whose rows are whole words, K rows of a word column a thread.  Where
+// it beats the blocked forms is step_cost's business (see gol_bits_run): calls of two generations,
+// and tall boards of few words, in whose windows most lanes hold nothing.
+template <int K>
+__global__ __launch_bounds__(256) void k_step(const uint32_t* __restrict__ P, uint32_t* __restrict__ Q, int NW, int ny,
+                                              unsigned nitems)
+{
+    // consecutive blocks share rows at their band edges: keep them on one XCD
+    const unsigned t = xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
+    if (t >= nitems) return;
+    const int band = (int)(t / (unsigned)NW), w = (int)(t - (unsigned)band * NW);
+    const int wl = w == 0 ? NW - 1 : w - 1;
+    const int wr = w == NW - 1 ? 0 : w + 1;
+    const int y0 = band * K;
+    uint32_t h0[K + 2], h1[K + 2], cen[K + 2];
+#pragma unroll
+    for (int r = 0; r < K + 2; r++) {
+        int y = y0 - 1 + r;  // periodic rows; y < ny + K, so the loop ends (once if K <= ny)
+        if (y < 0) y += ny;
+        while (y >= ny) y -= ny;
+        const uint32_t* row = P + (size_t)y * NW;
+        const uint32_t c = row[w], l = row[wl], rr = row[wr];
+        const uint32_t W = __builtin_amdgcn_alignbit(c, l, 31);  // cell x-1 at bit x
+        const uint32_t E = __builtin_amdgcn_alignbit(rr, c, 1);  // cell x+1 at bit x
+        h0[r] = xor3(W, c, E);
+        h1[r] = maj(W, c, E);
+        cen[r] = c;
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int y = y0 + k;
+        if (y >= ny) break;
+        // S = h[k] + h[k+1] + h[k+2] through the carry-save adders of the two bit-planes
+        const uint32_t s0 = xor3(h0[k], h0[k + 1], h0[k + 2]);
+        const uint32_t c0 = maj(h0[k], h0[k + 1], h0[k + 2]);
+        const uint32_t u1 = xor3(h1[k], h1[k + 1], h1[k + 2]);
+        const uint32_t c1 = maj(h1[k], h1[k + 1], h1[k + 2]);
+        Q[(size_t)y * NW + w] = life_rule(s0, c0, u1, c1, cen[k + 1]);
+    }
+}
+
 constexpr int KROWS = 8;
 
 // 32 cells from cell x on of one padded uint8 row (bit b of word = cell x + b), and the ring
@@ -648,21 +689,56 @@ int run_win(appfis_ctx* ctx, const golbits::WinVariant& v, uint32_t* const P[2],
 // states: blocks that share a CU take about 0.8 of their times' sum.  Measured (48 generations,
 // us; k4 g24, k6 g24, k6 g16, k8 g24, k8 g16, k12 g16): 1000 x 1000 23 30 34 37 43 56; 3000 x 3000
 // 34 30 34 37 42 57; 8191 x 8191 139 88 79 86 71 92; 16384 x 16384 457 247 199 201 196 171.
+double win_blocks(const golbits::WinVariant& v, int nx, int ny)
+{
+    return (double)ceil_div((nx + 31) / 32, golbits::WIN_WORDS) * ceil_div(ny, v.nwaves * v.k - 2 * v.g);
+}
+double win_cost(const appfis_ctx* ctx, const golbits::WinVariant& v, int nx, int ny, int gens)
+{
+    const double cus = ctx->num_cu > 0 ? ctx->num_cu : 256, blocks = win_blocks(v, nx, ny);
+    const double load = blocks <= cus ? 1.0 : 0.8 * std::ceil(blocks / cus);
+    return 4.5 * ceil_div(gens, v.g) + gens * (0.07 + 0.0775 * v.k) * load;
+}
 const golbits::WinVariant& win_for(const appfis_ctx* ctx, int nx, int ny, int gens)
 {
-    const double cus = ctx->num_cu > 0 ? ctx->num_cu : 256;
     const golbits::WinVariant* best = nullptr;
     double least = 0.0;
     for (const golbits::WinVariant& v : golbits::kWin) {
-        const double blocks = (double)ceil_div((nx + 31) / 32, golbits::WIN_WORDS) * ceil_div(ny, v.nwaves * v.k - 2 * v.g);
-        const double load = blocks <= cus ? 1.0 : 0.8 * std::ceil(blocks / cus);
-        const double cost = 4.5 * ceil_div(gens, v.g) + gens * (0.07 + 0.0775 * v.k) * load;
+        const double cost = win_cost(ctx, v, nx, ny, gens);
         if (!best || cost < least) {
             best = &v;
             least = cost;
         }
     }
     return *best;
+}
+
+// `gens` generations from P[*cur] one by one
+int run_step(appfis_ctx* ctx, uint32_t* const P[2], int* cur, int NW, int ny, int gens, int* launches)
+{
+    using namespace golbits;
+    const unsigned nitems = (unsigned)NW * ceil_div(ny, KROWS);
+    for (int g = 0; g < gens; g++) {
+        hipLaunchKernelGGL(k_step<KROWS>, dim3(ceil_div(nitems, 256)), dim3(256), 0, ctx->stream, P[*cur], P[*cur ^ 1],
+                           NW, ny, nitems);
+        APPFIS_LAUNCH_CHECK();
+        *cur ^= 1;
+    }
+    *launches = gens;
+    return APPFIS_OK;
+}
+
+// Whether `gens` generations of a board of whole words run faster one by one than in windows of v.
+// One takes 2.9 us and its words' traffic, up to ten times that where rows of few words leave a
+// wave's lanes far apart; a window launch of several blocks to a CU loads and stores 2.2 us longer
+// for each.  us a call, one by one / windows: 64 x 10^6 2 generations 90 / 146, 30 601 / 678; 512 x
+// 131072 2 46.5 / 56.7, 4 57.8 / 62.2, 6 69.1 / 67.9; 96 x 96 2 10.7 / 11.9, 4 16.6 / 12.9.
+bool step_faster(const appfis_ctx* ctx, const golbits::WinVariant& v, int nx, int ny, int gens)
+{
+    const double cus = ctx->num_cu > 0 ? ctx->num_cu : 256, NW = nx / 32;
+    const double step = 2.9 + 1.5e-6 * NW * ny * std::max(1.0, 10.0 / NW);
+    const double more = std::ceil(win_blocks(v, nx, ny) / cus) - 1.0;
+    return gens * step < win_cost(ctx, v, nx, ny, gens) + ceil_div(gens, v.g) * 2.2 * more;
 }
 
 // `gens` generations from P[*cur] with k_step_tb, rows spread over NW / 64 waves
@@ -726,8 +802,9 @@ bool gol_bits_workspace(appfis_ctx* ctx, int nx, int ny)
 // against the window (at 8192 x 8192 63 us for 48 generations against 69, at 2048 x 2048 31
 // against 24).  With full-row waves and two or more generations, all of them run in their
 // launches (at least two), the first reading the uint8 field and the last writing both uint8
-// buffers; otherwise k_pack packs the field, generations 1 .. gens-1 run blocked, and the last
-// one runs fused with the unpacking (k_step_unpack), so that generation gens-1 is still at hand.
+// buffers; otherwise k_pack packs the field, generations 1 .. gens-1 run blocked, or one by one
+// where step_faster says so, and the last one runs fused with the unpacking (k_step_unpack), so
+// that generation gens-1 is still at hand.
 int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int gens, int force)
 {
     const int NW = (nx + 31) / 32;
@@ -772,6 +849,12 @@ int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int 
                              4, &c);
             if (st) return st;
             if (c < (int)cand.size()) tw = cand[c];
+            // The tuner times the generations alone.  In a short call the two launches that the
+            // full-row form does without, its first packing the board and its last unpacking it,
+            // count for more than its longer generations, where a lane holds one word (2048 x
+            // 2048, us a call, full rows / windows: 2 generations 13.9 / 15.3, 16 18.3 / 20.3,
+            // 24 23.3 / 22.7; 4096 x 1000, two words: 20.2 / 15.3, 27.5 / 20.5, 33.8 / 22.9).
+            else if (cand[0]->wpl == 1 && gens < 20) tw = cand[0];
         }
     }
     uint8_t* buf[2] = {b0, b1};
@@ -810,8 +893,12 @@ int gol_bits_run(appfis_ctx* ctx, uint8_t* b0, uint8_t* b1, int nx, int ny, int 
     st = ktime_begin(ctx);
     if (st) return st;
     if (gens > 1) {
-        st = win ? run_win(ctx, *win, P, &cur, nx, ny, gens - 1, &launches)
-                 : run_tb(ctx, P, &cur, NW, ny, gens - 1, &launches);
+        if (!win)
+            st = run_tb(ctx, P, &cur, NW, ny, gens - 1, &launches);
+        else if (force < 0 && nx % 32 == 0 && step_faster(ctx, *win, nx, ny, gens - 1))
+            st = run_step(ctx, P, &cur, NW, ny, gens - 1, &launches);
+        else
+            st = run_win(ctx, *win, P, &cur, nx, ny, gens - 1, &launches);
         if (st) return st;
     }
     st = ktime_end(ctx, launches, gens - 1);

@@ -451,6 +451,32 @@ def test_fdtd3d_every_candidate_bit_exact(ctx, dt, n):
     assert ran >= 2
 
 
+# board, generations, launches of the packed generations: two generations and tall boards of few
+# words go one by one (all but the last, which unpacks), short calls of 2048 cells a row run in
+# full-row waves (8 generations a launch, conversions included), all others in windows
+@pytest.mark.parametrize("nx,ny,gens,launches", [
+    (32, 3, 2, 1), (32, 5, 3, 1), (96, 96, 2, 1), (96, 97, 3, 1), (64, 300001, 2, 1), (64, 300001, 5, 4),
+    (2048, 7, 2, 2), (2048, 65, 8, 2), (2048, 65, 9, 2), (2048, 300, 19, 3)])
+def test_gol_short_calls_and_tall_boards(ctx, nx, ny, gens, launches):
+    a = np.zeros((ny + 2, nx + 2), dtype=np.uint8)
+    oracle.fill_bernoulli(a, 1, 71, 0.3)
+    d0, d1 = ctx.from_numpy(a), ctx.from_numpy(np.full_like(a, 1))
+    ctx.gol(d0, d1, nx, ny, gens, hip.CHOSEN)  # tunes the shape
+    d0.upload(a)
+    d1.upload(np.full_like(a, 1))
+    ctx.kernel_timing(True)
+    ctx.gol(d0, d1, nx, ny, gens, hip.CHOSEN)
+    got = ctx.kernel_time()[1]
+    ctx.kernel_timing(False)
+    e = [ctx.from_numpy(a), ctx.from_numpy(np.full_like(a, 1))]
+    ctx.gol(e[0], e[1], nx, ny, gens, hip.PLAIN)
+    ref = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens)
+    assert np.array_equal((d0, d1)[gens % 2].download()[1:-1, 1:-1], ref[1:-1, 1:-1])
+    for x, y in zip((d0, d1), e):  # both buffers, rings included
+        assert np.array_equal(x.download(), y.download())
+    assert got == launches
+
+
 @pytest.mark.parametrize("dt", [hip.F32, hip.F64, hip.F16, hip.BF16])
 @pytest.mark.parametrize("n", [(5, 3, 1), (66, 9, 2), (100, 101, 103), (127, 131, 140), (162, 161, 163), (257, 257, 260),
                                (256, 264, 260), (301, 330, 340), (321, 330, 640)])
