@@ -451,6 +451,20 @@ def test_fdtd3d_every_candidate_bit_exact(ctx, dt, n):
     assert ran >= 2
 
 
+@pytest.mark.parametrize("nx", [2, 3, 5, 12, 13, 14, 15, 16, 17, 30])
+def test_gol_byte_kernel_on_narrow_boards(ctx, nx):
+    # padded rows shorter than the kernel's 16-byte chunk, equal to it and longer; both buffers with
+    # their rings: generation n and, in the other, n - 1
+    for ny in (2, 3, 21, 700):
+        a = np.zeros((ny + 2, nx + 2), dtype=np.uint8)
+        oracle.fill_bernoulli(a, 1, 73 + nx, 0.4)
+        d = [ctx.from_numpy(a), ctx.from_numpy(np.full_like(a, 1))]
+        ctx.gol(d[0], d[1], nx, ny, 3, hip.PLAIN)
+        for gens, got in ((3, d[1]), (2, d[0])):
+            ref = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens)[1:-1, 1:-1]
+            assert np.array_equal(got.download(), np.pad(ref, 1, mode="wrap")), (ny, gens)
+
+
 # board, generations, launches of the packed generations: two generations and tall boards of few
 # words go one by one (all but the last, which unpacks), short calls of 2048 cells a row run in
 # full-row waves (8 generations a launch, conversions included), all others in windows
