@@ -18,7 +18,8 @@
 struct appfis_tune_entry {
     int key[6];
     int choice;
-    int param = 0;  // what the variant runs with, where a rule sets it (FDTD3d: planes per block)
+    int param = 0;          // FDTD3d: planes per block; Heat2D: the variant of shallow launches
+    std::vector<float> ms;  // of every candidate
     std::string report;
 };
 

@@ -211,7 +211,7 @@ int tune_select(appfis_ctx* ctx, const int key[6], int ncand, const char* const*
     std::string rep = "autotune kernel " + std::to_string(key[0]) + " dtype " + std::to_string(key[1]) + " shape " +
                       std::to_string(key[2]) + "x" + std::to_string(key[3]) + "x" + std::to_string(key[4]) + ":";
     int best = 0;
-    float best_ms = 0.f;
+    std::vector<float> times;
     // events of its own: the caller's timer (ctx->ev_start/ev_stop) may be running
     hipEvent_t e0 = nullptr, e1 = nullptr;
     APPFIS_HIP_CHECK(hipEventCreate(&e0));
@@ -243,15 +243,14 @@ int tune_select(appfis_ctx* ctx, const int key[6], int ncand, const char* const*
         char line[160];
         snprintf(line, sizeof(line), " [%s %.4f ms]", names[i], ms);
         rep += line;
-        if (i == 0 || ms < best_ms) {
-            best = i;
-            best_ms = ms;
-        }
+        times.push_back(ms);
+        if (ms < times[best]) best = i;
     }
     rep += std::string(" -> ") + names[best];
     appfis_tune_entry e;
     memcpy(e.key, key, sizeof(e.key));
     e.choice = best;
+    e.ms = std::move(times);
     e.report = rep;
     ctx->tuned.push_back(e);
     ctx->tune_report = rep;

@@ -380,6 +380,7 @@ static const HeatVariant kHeat[] = {
     {"rt 32x32 ts16 k4 w16", run_rt<T, 4, 16, 16, 1>, 16},
     {"whole 64x80 k5 w16", run_whole<T, 5, 16, 1>, 0},
 };
+constexpr int SHALLOW = 8;
 constexpr int kHeatCount = (int)(sizeof(kHeat<double>) / sizeof(kHeat<double>[0]));
 
 }  // namespace
@@ -411,29 +412,39 @@ extern "C" int appfis_heat2d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
         // (an even number of full launches at depths 8, 12 and 16 alike); every
         // candidate computes the same values in the same order
         const int key[6] = {1, dtype, nx, ny, 0, 0};
-        bool cached = false;
-        for (const appfis_tune_entry& e : ctx->tuned)
-            if (memcmp(e.key, key, sizeof(key)) == 0) cached = true;
-        void* s0 = nullptr;
-        void* s1 = nullptr;
-        if (!cached) {
+        if (!tuned_entry(ctx, key)) {
             APPFIS_NOT_CAPTURING(ctx, "appfis_heat2d CHOSEN's first call for a shape (autotuning)");
             const size_t half = ((size_t)(nx + 2) * (ny + 2) * dtype_size(dtype) + 255) / 256 * 256;
             int st = ensure_work(ctx, 2 * half);
             if (st) return st;
-            s0 = ctx->work;
-            s1 = (char*)ctx->work + half;
+            void* const s0 = ctx->work;
+            void* const s1 = (char*)ctx->work + half;
             APPFIS_HIP_CHECK(hipMemsetAsync(ctx->work, 0, 2 * half, ctx->stream));
-        }
-        // every candidate that differs here: "whole", the last, only where the grid fits it
-        const int ntab = whole_fits<5, 16, 1>(nx, ny) ? kHeatCount : kHeatCount - 1;
-        std::vector<const char*> names;
-        for (int i = 0; i < ntab; i++) names.push_back(tab[i].name);
-        int pick = 0;
-        int st = tune_select(ctx, key, ntab, names.data(),
+            // every candidate that differs here: "whole", the last, only where the grid fits it
+            const int ntab = whole_fits<5, 16, 1>(nx, ny) ? kHeatCount : kHeatCount - 1;
+            std::vector<const char*> names;
+            for (int i = 0; i < ntab; i++) names.push_back(tab[i].name);
+            int pick = 0;
+            st = tune_select(ctx, key, ntab, names.data(),
                              [&](int i) { return tab[i].fn(ctx, s0, s1, nx, ny, c, 96, tab[i].ts); }, 3, &pick);
-        if (st) return st;
-        return tab[pick].fn(ctx, buf0, buf1, nx, ny, c, iters, tab[pick].ts);
+            if (st) return st;
+            appfis_tune_entry& e = ctx->tuned.back();
+            for (int i = 0; i < ntab; i++)
+                if (tab[i].ts == SHALLOW && (tab[e.param].ts != SHALLOW || e.ms[i] < e.ms[e.param])) e.param = i;
+        }
+        // The launches of a call have the parity of its sweeps, so calls of one and two take one
+        // launch a sweep in any form, and PLAIN's needs no halo (us, tiles / PLAIN: 2048^2 FP32
+        // 12.5 / 8.0, 1000^2 FP64 6.1 / 4.8, 8192^2 FP64 277 / 239).  Where the deep tiles' halo
+        // saves no launch the best shallow ones are faster (1000^2 FP64, 5 sweeps 9.5 / 8.3, 16
+        // sweeps 23.9 / 20.5, 20 sweeps 27.0 / 32.7; 96 x 80, 7 sweeps 5.6 / 5.0).
+        if (iters <= 2)
+            return dtype == APPFIS_F64 ? run_plain<double>(ctx, (double*)buf0, (double*)buf1, nx, ny, c, iters)
+                                       : run_plain<float>(ctx, (float*)buf0, (float*)buf1, nx, ny, (float)c, iters);
+        const appfis_tune_entry* e = tuned_entry(ctx, key);
+        const int ts = tab[e->choice].ts;
+        const bool shallow = ts > SHALLOW && launch_count(iters, SHALLOW) == launch_count(iters, ts);
+        const HeatVariant& v = tab[shallow ? e->param : e->choice];
+        return v.fn(ctx, buf0, buf1, nx, ny, c, iters, v.ts);
     }
     if (variant >= APPFIS_CANDIDATE0) {
         if (dtype != APPFIS_F64 && dtype != APPFIS_F32) return invalid("heat2d: dtype must be F64 or F32");

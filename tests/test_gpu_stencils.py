@@ -451,6 +451,31 @@ def test_fdtd3d_every_candidate_bit_exact(ctx, dt, n):
     assert ran >= 2
 
 
+@pytest.mark.parametrize("dt", [hip.F64, hip.F32])
+@pytest.mark.parametrize("nx,ny", [(40, 33), (96, 80), (333, 250)])
+def test_heat2d_chosen_calls_of_few_sweeps(ctx, dt, nx, ny):
+    # one and two sweeps one by one, up to 16 in shallow tiles where these need no more launches
+    for it in range(1, 20):
+        a, d0, d1 = _heat_pair(ctx, nx, ny, dt)
+        ctx.heat2d(d0, d1, nx, ny, 0.1, it, hip.CHOSEN)
+        ref = oracle.heat2d(a.copy(), np.zeros_like(a), nx, ny, 0.1, it)
+        assert np.array_equal((d0, d1)[it % 2].download(), ref), it
+
+
+def test_heat2d_call_of_one_sweep_loads_no_halo(ctx):
+    # one sweep of 2048 x 2048 in FP32 takes 8 us without a halo, 12 in tiles with one of 12 cells
+    n = 2048
+    d0, d1 = (ctx.array((n + 2, n + 2), hip.F32) for _ in range(2))
+    ms = {}
+    for v in (hip.PLAIN, hip.CHOSEN, hip.PLAIN, hip.CHOSEN):
+        for _ in range(8):
+            ctx.timer_start()
+            for _ in range(20):
+                ctx.heat2d(d0, d1, n, n, 0.1, 1, v)
+            ms[v] = min(ms.get(v, 1e9), ctx.timer_stop())
+    assert ms[hip.CHOSEN] < 1.25 * ms[hip.PLAIN], ms
+
+
 @pytest.mark.parametrize("nx", [2, 3, 5, 12, 13, 14, 15, 16, 17, 30])
 def test_gol_byte_kernel_on_narrow_boards(ctx, nx):
     # padded rows shorter than the kernel's 16-byte chunk, equal to it and longer; both buffers with
