@@ -510,34 +510,35 @@ int run_ensemble(appfis_ctx* ctx, int ngrid, const int* nx, const int* ny, void*
 }
 
 // Tiles an ensemble may take.  Its launches take about
-//     launches * launch + sweeps * sweep * blocks per CU
-// us, blocks per CU being the mean of their number and of it rounded up, and at least a quarter:
-// the tiles are those of the least sum.  The constants are fitted to 26 ensembles of 4 to 64 grids
-// of 64 to 1024 cells a side and 20 to 200 sweeps; the choice is within 1 % of the best of ten
-// tilings on average, 9 % at most.  (FP64, us for all sweeps, in the order below: 8 grids up to 256,
-// 96 sweeps 158, 112, 101, 135; 30 up to 256, 96 sweeps 172, 173, 209, 150; 30 up to 512, 48
-// sweeps 185, 172, 260, 206; 64 up to 1024, 96 sweeps 1262, 1482, 2646, 1801.)
+//     launches * (launch + load * blocks per CU) + sweeps * sweep * blocks per CU
+// us, `load` a block's window in and its tile out, blocks per CU being the mean of their number and
+// of it rounded up, and at least a quarter: the tiles are those of the least sum.  The constants are
+// fitted to 14 ensembles of 1 to 256 grids of 20 to 8192 cells a side and 1 to 200 sweeps; the choice
+// is within 1 % of the best of the four on average, 10 % at most.  (Us for all sweeps, in the order
+// below; FP64: two of 4000 x 4000 1 sweep 164, 146, 260, 182, 5 165, 161, 333, 251, 100 1878, 2356,
+// 4173, 2816; 30 up to 256 10 sweeps 58, 58, 70, 61, 100 183, 181, 223, 159.  FP32: 64 of 64 to 883 x 137
+// to 200 4 sweeps 78, 93, 140, 89, 100 343, 408, 613, 376.)
 struct HeatEnsemble {
     int (*fn)(appfis_ctx*, int, const int*, const int*, void* const*, void* const*, double, int);
     int tx, ty, ts;
-    double launch, sweep;
+    double launch, load, sweep;
 };
 template <typename T, int K, int NW, int TS, int WPL>
-constexpr HeatEnsemble ensemble_tiles(double launch, double sweep)
+constexpr HeatEnsemble ensemble_tiles(double launch, double load, double sweep)
 {
-    return {run_ensemble<T, K, NW, TS, WPL>, 64 * WPL - 2 * TS, NW * K - 2 * TS, TS, launch, sweep};
+    return {run_ensemble<T, K, NW, TS, WPL>, 64 * WPL - 2 * TS, NW * K - 2 * TS, TS, launch, load, sweep};
 }
 static const HeatEnsemble kEnsembleF64[] = {
-    ensemble_tiles<double, 8, 8, 8, 2>(5.95, 0.77),
-    ensemble_tiles<double, 6, 8, 8, 1>(4.65, 0.28),
-    ensemble_tiles<double, 4, 16, 16, 1>(5.98, 0.36),
-    ensemble_tiles<double, 5, 16, 16, 2>(5.3, 1.01),
+    ensemble_tiles<double, 8, 8, 8, 2>(4.58, 4.12, 0.21),
+    ensemble_tiles<double, 6, 8, 8, 1>(4.34, 1.05, 0.12),
+    ensemble_tiles<double, 4, 16, 16, 1>(5.26, 1.42, 0.23),
+    ensemble_tiles<double, 5, 16, 16, 2>(3.6, 3.97, 0.68),
 };
 static const HeatEnsemble kEnsembleF32[] = {
-    ensemble_tiles<float, 8, 8, 8, 2>(5.81, 0.45),
-    ensemble_tiles<float, 6, 8, 8, 1>(4.24, 0.19),
-    ensemble_tiles<float, 4, 16, 16, 1>(4.74, 0.25),
-    ensemble_tiles<float, 5, 16, 16, 2>(6.86, 0.5),
+    ensemble_tiles<float, 8, 8, 8, 2>(5.04, 1.64, 0.19),
+    ensemble_tiles<float, 6, 8, 8, 1>(4.09, 0.96, 0.05),
+    ensemble_tiles<float, 4, 16, 16, 1>(4.51, 1.42, 0.12),
+    ensemble_tiles<float, 5, 16, 16, 2>(5.69, 1.92, 0.3),
 };
 
 const HeatEnsemble& pick_ensemble(const HeatEnsemble (&tab)[4], int num_cu, int ngrid, const int* nx, const int* ny,
@@ -550,9 +551,8 @@ const HeatEnsemble& pick_ensemble(const HeatEnsemble (&tab)[4], int num_cu, int 
         double blocks = 0.0;
         for (int g = 0; g < ngrid; g++)
             if (nx[g] > 0 && ny[g] > 0) blocks += (double)ceil_div(nx[g], e.tx) * ceil_div(ny[g], e.ty);
-        const double per_cu = blocks / (num_cu > 0 ? num_cu : 256);
-        const double cost = launch_count(iters, e.ts) * e.launch +
-                            iters * e.sweep * std::max(0.5 * (per_cu + std::ceil(per_cu)), 0.25);
+        const double mean = blocks / (num_cu > 0 ? num_cu : 256), per_cu = std::max(0.5 * (mean + std::ceil(mean)), 0.25);
+        const double cost = launch_count(iters, e.ts) * (e.launch + e.load * per_cu) + iters * e.sweep * per_cu;
         if (i == 0 || cost < least) {
             least = cost;
             best = i;
