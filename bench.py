@@ -179,8 +179,10 @@ def heat_kernel_name(tname, dtype="double"):
     """Kernel symbol of a Heat2D temporal-blocking candidate: "tb 64x64 ts12 nt1024" ->
     k_heat2d_tb<double, 64, 64, 12, 1024> (output tile, sweeps, threads); "rt 48x96 ts8 k7
     w16" -> k_heat2d_rt<double, 7, 16, 8, 1> (rows per wave, waves, sweeps, columns per
-    lane: "rt2" holds two)."""
+    lane: "rt2" holds two); "whole 64x80 k5 w16" -> k_heat2d_whole<double, 5, 16, 1>."""
     form, tile, ts, a, *rest = tname.split()
+    if form == "whole":
+        return f"k_heat2d_whole<{dtype}, {int(ts[1:])}, {int(a[1:])}, 1>"
     if form.startswith("rt"):
         wpl = int(form[2:] or 1)
         return f"k_heat2d_rt<{dtype}, {int(a[1:])}, {int(rest[0][1:])}, {int(ts[2:])}, {wpl}>"
@@ -190,14 +192,16 @@ def heat_kernel_name(tname, dtype="double"):
 
 def gol_kernel_name(tname):
     """Kernel symbol of a bit-packed GoL candidate: "tb k12 g8 w16" -> k_step_tb<12, 8, 16>,
-    "tw4 k4 g8 w12" -> k_step_tw<4, 4, 8, 12> (words per lane first); no candidate (widths
-    the blocked kernels do not take) -> the one-generation k_step<8>."""
+    "tw4 k4 g8 w12" -> k_step_tw<4, 4, 8, 12> (words per lane first), "win k8 g16 w16" ->
+    k_step_win<1, 8, 16, 16>; no candidate -> the one-generation k_step<8>."""
     if not tname:
         return "k_step<8>"
     form, *rest = tname.split()
     k, g, w = (int(t[1:]) for t in rest[:3])
     if form.startswith("tw"):
         return f"k_step_tw<{int(form[2:])}, {k}, {g}, {w}>"
+    if form == "win":
+        return f"k_step_win<1, {k}, {g}, {w}>"
     return f"k_step_{form}<{k}, {g}, {w}>"
 
 

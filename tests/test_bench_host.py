@@ -101,3 +101,17 @@ def test_heat_kernel_names():
     assert bench.heat_kernel_name("rt2 112x48 ts8 k8 w8") == "k_heat2d_rt<double, 8, 8, 8, 2>"
     assert bench._short("void (anonymous namespace)::k_heat2d_rt<double, 7, 16, 8, 1>(double const*, double*, int, "
                         "int, double, int)") == "k_heat2d_rt<double, 7, 16, 8, 1>"
+
+
+def test_kernel_names_of_the_candidates_the_library_lists():
+    from appfis_amd import hip
+
+    src = "".join(open(os.path.join(ROOT, "appfis_amd", "csrc", f)).read() for f in ("gol_bits.hip", "heat2d.hip"))
+    for name in hip.gol_candidates():
+        assert bench.gol_kernel_name(name).split("<")[0] + "(" in src, name
+    for dt in (hip.F64, hip.F32):
+        for name in hip.heat2d_candidates(dt):
+            assert bench.heat_kernel_name(name).split("<")[0] + "(" in src, name
+    assert bench.gol_kernel_name("win k8 g16 w16") == "k_step_win<1, 8, 16, 16>"
+    assert "k_step_win<1, 8, 16, 16>" in json.load(open(os.path.join(ROOT, "profiles", "traffic.json")))
+    assert bench.heat_kernel_name("whole 64x80 k5 w16", "float") == "k_heat2d_whole<float, 5, 16, 1>"
