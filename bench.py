@@ -404,20 +404,17 @@ def _plan(iters, ts):
 
 
 
-# the PLAIN form's fixed tilings at 512^3 on 256-byte aligned buffers
-FDTD_PLAIN_PREFERRED = {"f32": "dma ty16 ry2 zc256 d2", "f64": "vx2 ty16 ry1 zc256 d2 u2",
-                        "f16": "vx2 ty8 ry2 zc128 d2 u18", "bf16": "vx2 ty8 ry2 zc128 d2 u18"}
-
-
-def _fdtd_plain(hip, name, dt, n):
-    """The PLAIN form's fixed tiling at n^3 (a name of appfis_fdtd3d_candidates)."""
-    return FDTD_PLAIN_PREFERRED[name]
+# the PLAIN form's tilings at 512^3 on 256-byte aligned buffers (it picks by size; the planes per
+# block, which follow the size too, are no part of a kernel's name)
+FDTD_PLAIN_512 = {"f32": "dma ty16 ry2 zc256 d2", "f64": "vx2 ty16 ry1 zc256 d2 u2",
+                  "f16": "vx2 ty8 ry2 zc128 d2 u18", "bf16": "vx2 ty8 ry2 zc128 d2 u18"}
 
 
 FDTD_CTYPE = {"f32": "float", "f64": "double", "f16": "__half", "bf16": "__hip_bfloat16"}
 
 
-def bench_fdtd(ctx, hip, n=512, steps=100):
+def bench_fdtd(ctx, hip, steps=100):
+    n = 512
     out = {"workload": f"FDTD3d r=4 {n}^3, {steps} steps (CHOSEN = autotuned tiling, same values as PLAIN)"}
     finals = {}  # each dtype's field after the timed CHOSEN run, as float64, normalised by 2.0625^steps
     for name, dt, bpl in (("f32", hip.F32, 8), ("f64", hip.F64, 16), ("f16", hip.F16, 4), ("bf16", hip.BF16, 4)):
@@ -430,7 +427,7 @@ def bench_fdtd(ctx, hip, n=512, steps=100):
             ctx.fdtd3d(a, b, n, n, n, coeff, 2, variant)  # warm-up (and the one-time autotuning)
             ctx.fill_uniform(a, 4, 1004)
             ms, _ = timed(ctx, lambda: ctx.fdtd3d(a, b, n, n, n, coeff, steps, variant))
-            tname = _fdtd_plain(hip, name, dt, n) if variant == hip.PLAIN else _tuned(ctx, 3, dt)
+            tname = FDTD_PLAIN_512[name] if variant == hip.PLAIN else _tuned(ctx, 3, dt)
             if tname.startswith("dma "):  # direct-to-LDS form: "dma ty16 ry2 zc256 d2"
                 ty, ry, zc, dd = (int(t[2:]) if t[:2] in ("ty", "ry", "zc") else int(t[1:])
                                   for t in tname.split()[1:])
