@@ -482,12 +482,31 @@ def _himeno_dev(ctx, hip, nx, ny, nz, dt):
     return arrs, p
 
 
+def himeno_pairs(iters):
+    """Launches of two sweeps in a PLAIN call: all sweeps but the last 1 to 4 run in them."""
+    return (iters - 1) // 4 * 2
+
+
+def himeno_bytes(iters, size):
+    """Bytes that a PLAIN call moves per point and sweep: a launch, of one sweep or of two, reads
+    11 coefficients, wrk1 and p and writes p, `size` bytes each."""
+    return 14.0 * size * (iters - himeno_pairs(iters)) / iters
+
+
+def himeno_dc_bytes(K):
+    """The same on average over an outer cycle of K sweeps of the defect correction: K-1 FP32 inner
+    sweeps, two to a launch but for the one left over (11 coefficients, read from a copy blocked by
+    64 points, r, q read, q written: 56 B a launch), and one FP64 rebase (11 coefficients, wrk1, B
+    read, q read 4 B, B / r / q written 8 + 4 + 4 B: 124 B)."""
+    return (((K - 1) // 2 + (K - 1) % 2) * 56.0 + 124.0) / K
+
+
 def bench_himeno(ctx, hip, nx=257, ny=257, nz=513, iters=200):
     out = {"workload": f"Himeno 19-point {nx}x{ny}x{nz} (incl. shell), {iters} sweeps + gosa"}
     lups = (nx - 2) * (ny - 2) * (nz - 2) * iters
     gosas = {}
-    for name, dt, variant, bpl in (("f32", hip.F32, hip.PLAIN, 56), ("f64", hip.F64, hip.PLAIN, 112),
-                                   ("dc", hip.F64, hip.CHOSEN, None)):
+    for name, dt, variant, size in (("f32", hip.F32, hip.PLAIN, 4), ("f64", hip.F64, hip.PLAIN, 8),
+                                    ("dc", hip.F64, hip.CHOSEN, None)):
         arrs, p = _himeno_dev(ctx, hip, nx, ny, nz, dt)
         ctx.himeno(arrs, nx, ny, nz, 0.8, 3, variant)  # warm-up
         arrs[0].upload(p)
@@ -504,22 +523,15 @@ def bench_himeno(ctx, hip, nx=257, ny=257, nz=513, iters=200):
         d = int(shape.split()[1][1:])
         ry = int(shape.split()[2][2:]) if len(shape.split()) > 2 else 2
         r["tiling"] = shape
-        if bpl:
-            # the sweeps but the last 1 to 4 run two to a launch (k_himeno_two): launches per sweep
+        if size:
             t, rows = ("float", 2) if dt == hip.F32 else ("double", 1)
-            pairs = (iters - 1) // 4 * 2
-            r["roofline"] = roofline(float(bpl) * pts, ms / iters,
+            pairs = himeno_pairs(iters)
+            r["roofline"] = roofline(himeno_bytes(iters, size) * pts, ms / iters,
                                      {f"k_himeno_two<{t}, 0, 256, 4, {rows}>": pairs / iters,
                                       f"k_himeno<{t}, 0, {d}, {ry}>": (iters - 2 * pairs) / iters})
         else:
-            # defect correction, per sweep on average over one outer cycle of K sweeps
-            # (the library's default K = 16): K-1 FP32 inner sweeps (11 coefficients, read
-            # from a copy blocked by 64 points, r, q read, q written: 56 B/LUP) and one FP64
-            # rebase (11 coefficients, wrk1, B read, q read 4 B, B / r / q written
-            # 8 + 4 + 4 B: 124 B/LUP)
-            K = HIMENO_DC_OUTER
-            # The inner sweeps run two to a launch, but for the one left over.
-            r["roofline"] = roofline(((K - 1) * 56.0 + 124.0) / K * pts, ms / iters,
+            K = HIMENO_DC_OUTER  # the library's default
+            r["roofline"] = roofline(himeno_dc_bytes(K) * pts, ms / iters,
                                      {"k_himeno_two<float, 2, 256, 4, 2>": (K - 1) // 2 / K,
                                       f"k_himeno<float, 2, {d}, {ry}>": (K - 1) % 2 / K,
                                       f"k_himeno<double, 1, {d}, {ry}>": 1 / K})

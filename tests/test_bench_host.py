@@ -115,3 +115,12 @@ def test_kernel_names_of_the_candidates_the_library_lists():
     assert bench.gol_kernel_name("win k8 g16 w16") == "k_step_win<1, 8, 16, 16>"
     assert "k_step_win<1, 8, 16, 16>" in json.load(open(os.path.join(ROOT, "profiles", "traffic.json")))
     assert bench.heat_kernel_name("whole 64x80 k5 w16", "float") == "k_heat2d_whole<float, 5, 16, 1>"
+
+
+def test_himeno_bytes_count_a_pair_of_sweeps_once():
+    # 200 sweeps: 98 launches of two and 4 of one, 14 streams each
+    assert bench.himeno_pairs(200) == 98
+    assert bench.himeno_bytes(200, 4) == 56.0 * 102 / 200
+    assert bench.himeno_bytes(4, 8) == 112.0  # all single
+    # 15 inner sweeps in 7 pairs and one single launch, and the rebase
+    assert bench.himeno_dc_bytes(16) == (8 * 56.0 + 124.0) / 16
