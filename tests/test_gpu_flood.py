@@ -86,6 +86,53 @@ def test_flood_strip_heights_bit_exact(ctx, n):
     assert np.allclose(vg, vc, rtol=1e-13, atol=0)
 
 
+# A call's strips have one height, which follows the sum of its grids: beside a dry grid of these
+# sides (0: alone) a small grid is marched in strips of 1, 2, 3, 5, 14 and 32 rows (on 256 CUs).
+FLOOD_BESIDE = {hip.F64: [0, 465, 713, 1240, 1581, 2387], hip.F32: [0, 775, 1426, 1674, 1581, 2387]}
+FLOOD_HEIGHTS = [1, 2, 3, 5, 14, 32]
+
+
+def _strip_rows(dt, sides):
+    """The height by the rule of csrc/flood_impl.hpp on 256 CUs, for grids of (nx, ny)."""
+    few, more = (2.1, 0.4) if dt == hip.F64 else (2.2, 0.2)
+
+    def cost(rows):
+        strips = sum(-(-nx // 62) * -(-ny // rows) for nx, ny in sides)
+        return max(-(-(-(-strips // 4)) // 256), few) * (rows + more)
+
+    return min([32, 28, 24, 20, 16, 14, 12, 10, 8, 7, 6, 5, 4, 3, 2, 1], key=cost)
+
+
+@pytest.mark.parametrize("dt", [hip.F64, hip.F32])
+def test_flood_strips_of_every_height(ctx, dt):
+    # 70 x 67 cells: two strips wide, and the last strip of each height but 1 has fewer rows.  FP64
+    # without friction equals the oracle bit for bit at every height; FP32 gives the bits of the
+    # strips of one row
+    nx, ny, steps = 70, 67, 9
+    npdt = np.float64 if dt == hip.F64 else np.float32
+    z = oracle.flood_dem(nx, ny, DX, 3300)
+    h = np.zeros_like(z)
+    h[1:-1, 1:-1] = np.maximum(np.percentile(z[1:-1, 1:-1], 40) - z[1:-1, 1:-1], 0.0) + 0.1
+    h[20:30, 10:40] = 0.0
+    arrs = [x.astype(npdt) for x in (h, np.zeros_like(z), np.zeros_like(z), z, np.zeros_like(z))]
+    c = [x.astype(np.float64) for x in arrs]
+    tc, vc, _ = oracle.flood_run(*c, nx, ny, DX, CN, HEXTRA, DT_FALLBACK, 0.0, RAIN, 0.0, steps)
+    keys = ("h", "qx", "qy", "z", "n2")
+    first = None
+    for side, height in zip(FLOOD_BESIDE[dt], FLOOD_HEIGHTS):
+        sides = [(nx, ny)] + ([(side, side)] if side else [])
+        assert _strip_rows(dt, sides) == height
+        scen = [{"nx": nx, "ny": ny, **{k: ctx.from_numpy(x, dt) for k, x in zip(keys, arrs)}}]
+        if side:
+            scen.append({"nx": side, "ny": side, **{k: ctx.array((side + 2, side + 2), dt) for k in keys}})
+        t, v = ctx.flood_ensemble_run(scen, params(), steps, dt)
+        got = [scen[0][k].download() for k in keys[:3]] + [t[0]]
+        first = first or got
+        for x, y in zip(got, c[:3] + [tc] if dt == hip.F64 else first):
+            assert np.array_equal(x, y), height
+        assert np.allclose(v[0], vc, rtol=1e-13 if dt == hip.F64 else 1e-4, atol=0)
+
+
 # dx on both sides of the range in which dt * d / dx is taken by the reciprocal and its remainder,
 # some with inexact reciprocals; a dam breaks onto shallow and onto dry ground, so edges with the
 # entropy fix and with a dry side meet edges without in one wave
