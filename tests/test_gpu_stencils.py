@@ -329,6 +329,25 @@ def test_gol_windows_of_any_width(ctx, nx, ny, gens):
         assert np.array_equal((d0, d1)[(gens + 1) % 2].download(), prev), variant
 
 
+@pytest.mark.parametrize("nx,ny,gens", [(32, 3, 20), (33, 5, 9), (63, 64, 17), (65, 17, 25), (1000, 77, 49),
+                                        (1984, 33, 9), (1985, 50, 18), (4031, 49, 34), (6144, 30, 19)])
+def test_gol_windows_write_every_cell(ctx, nx, ny, gens):
+    # as above with both buffers filled anew before each form: a cell left out, in either buffer or
+    # its ring, keeps a value that no board holds
+    a, d0, d1 = _gol_pair(ctx, nx, ny, seed=nx * 13 + gens)
+    ref = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens)
+    prev = oracle.gol_u8(a.copy(), np.zeros_like(a), nx, ny, gens - 1)
+    wins = [hip.CANDIDATE0 + i for i, name in enumerate(hip.gol_candidates()) if name.startswith("win ")]
+    b = a.copy()
+    b[[0, -1], :] = b[:, [0, -1]] = 9
+    for variant in [hip.PLAIN, hip.CHOSEN] + wins:
+        d0.upload(a if variant == hip.PLAIN else b)  # the packed forms read no ring
+        d1.upload(np.full_like(a, 7))
+        ctx.gol(d0, d1, nx, ny, gens, variant)
+        assert np.array_equal((d0, d1)[gens % 2].download(), ref), variant
+        assert np.array_equal((d0, d1)[(gens + 1) % 2].download(), prev), variant
+
+
 @pytest.mark.parametrize("gens", [2, 7, 8, 9, 16, 17, 24, 25])
 def test_gol_full_row_launch_split(ctx, gens):
     # the full-row form runs a call's generations in at least two launches, the first
@@ -531,6 +550,25 @@ def test_fdtd3d_tilings_by_size(ctx, dt, n):
     for variant in (hip.PLAIN, hip.CHOSEN):
         ctx.fdtd3d(d0, d1, nx, ny, nz, coeff, 1, variant)
         assert np.array_equal(d1.download(), ref)
+
+
+@pytest.mark.parametrize("dt", [hip.F32, hip.F64, hip.F16, hip.BF16])
+@pytest.mark.parametrize("n", [(5, 3, 1), (64, 32, 2), (66, 9, 3), (40, 33, 61), (100, 101, 103), (127, 131, 140),
+                               (162, 161, 163), (257, 130, 301), (256, 264, 260), (321, 330, 340)])
+def test_fdtd3d_tilings_write_every_point(ctx, dt, n):
+    # NaN in the target before each form: a point that a dropped plane, chunk or tile leaves out
+    # stays one.  One plane, two, odd counts that the chunks do not divide, the sizes between which
+    # PLAIN's tilings change
+    nx, ny, nz = n
+    coeff = FDTD_COEFF if dt != hip.F16 else [c / 2.0625 for c in FDTD_COEFF]
+    a, d0, d1 = _fdtd_pair(ctx, n, dt)
+    ref = oracle.fdtd3d(a.copy(), np.zeros_like(a), nx, ny, nz, coeff, 1, bf16=(dt == hip.BF16))
+    blank = np.zeros_like(a)
+    blank[4:-4, 4:-4, 4:-4] = 0x7FC0 if dt == hip.BF16 else np.nan
+    for variant in (hip.PLAIN, hip.CHOSEN):
+        d1.upload(blank)
+        ctx.fdtd3d(d0, d1, nx, ny, nz, coeff, 1, variant)
+        assert np.array_equal(d1.download().view(np.uint8), ref.view(np.uint8)), variant
 
 
 def test_fdtd3d_chosen_call_costs_the_host_no_tuning(ctx):
