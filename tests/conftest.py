@@ -12,6 +12,16 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (runs the HIP kernels through the C ABI)")
 
 
+def pytest_collection_modifyitems(items):
+    # test_apps_build.py compiles the reference's sources and asks for their directory only, which
+    # may be there and empty
+    if not os.path.exists("/root/reference/HeatDiffusion/src/main.cpp"):
+        skip = pytest.mark.skip(reason="the reference sources are not on this machine")
+        for item in items:
+            if item.path.name == "test_apps_build.py":
+                item.add_marker(skip)
+
+
 @pytest.fixture(scope="session")
 def ctx():
     """One HIP context (device 0, one stream) for every GPU test of the session."""
