@@ -5,6 +5,9 @@ Execute*Reduce box reductions: bit-exact wherever the result is integer/byte wor
 pure data movement; compensated sums within a few ulps of math.fsum.
 """
 import math
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -14,6 +17,7 @@ from appfis_amd import hip
 
 pytestmark = pytest.mark.gpu
 
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 FDTD_COEFF = [0.5, 0.125, 0.125 / 2, 0.125 / 3, 0.125 / 4]
 NPDT = {hip.U8: np.uint8, hip.I32: np.int32, hip.F32: np.float32, hip.F64: np.float64, hip.F16: np.float16}
 
@@ -261,6 +265,37 @@ def test_captured_calls_outlive_a_larger_workspace_and_scratch():
             assert out.download()[0] == int(ref[1:-1, 1:-1].sum())
             assert all((x.download() == 173).all() for x in held)
         c.graph_destroy(g)
+
+
+_CAPTURE_FIRST = """
+import numpy as np, oracle
+from appfis_amd import hip
+n, coeff = (40, 33, 61), {coeff}
+with hip.Context(0) as c:
+    for dt in (hip.F32, hip.F64):
+        a = np.zeros(tuple(x + 8 for x in n[::-1]), dtype=np.float32 if dt == hip.F32 else np.float64)
+        oracle.fill_uniform(a, 4, 5)
+        d0, d1 = c.from_numpy(a, dt), c.array(a.shape, dt)
+        c.graph_begin()
+        c.fdtd3d(d0, d1, *n, coeff, 3, hip.PLAIN)
+        g = c.graph_end()
+        ref = oracle.fdtd3d(a.copy(), np.zeros_like(a), *n, coeff, 3)
+        for rep in range(3):
+            d0.upload(a)
+            c.graph_launch(g, 1)
+            c.sync()
+            assert np.array_equal(d1.download(), ref), (dt, rep)
+        c.graph_destroy(g)
+print("captured first: ok")
+"""
+
+
+def test_plain_fdtd3d_captured_as_a_process_first_call():
+    # PLAIN's rule asks the runtime how many blocks of a tiling a CU holds, once a process; the call
+    # that asks may be under capture
+    r = subprocess.run([sys.executable, "-u", "-c", _CAPTURE_FIRST.format(coeff=FDTD_COEFF)], cwd=ROOT,
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "captured first: ok" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
 
 
 def test_kernel_timing_of_gol_calls(ctx):
