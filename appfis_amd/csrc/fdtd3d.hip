@@ -798,10 +798,10 @@ extern "C" int appfis_fdtd3d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1,
         // A fixed tiling by size and by what the shape and the buffers admit: low tiles of few
         // rows per thread where the field is small (they make the most blocks), tall ones where
         // it streams from memory and the tile's halo rows count.  Each with its planes by the
-        // rule above (us a sweep, this tiling / the other side of the line): FP32 256^3 ty4 27,
-        // dma 28, 320^3 76 / 61, 449^3 ty16 224, ty8 241; FP64 128^3 ty4 12.1, vx2 ty16 12.8,
-        // 200^3 30.5 / 29.2, 257^3 ty8 84, ty16 86, 321^3 165 / 148; BF16 65^3 ty4 ry2 5.2, ry4
-        // 5.6, 129^3 12.0 / 10.9, 320^3 vx2 ty4 47.8, ty8 49.5, 384^3 72.3 / 69.8.
+        // rule above (us a sweep, this tiling / the other side of the line): FP32 256^3 ty4 29.4,
+        // dma 28.3, 320^3 75 / 61, 400 x 401 x 402 ty16 168, ty8 178; FP64 128^3 ty4 11.6, vx2 ty16
+        // 11.8, 200^3 33.2 / 30.7, 511 x 301 x 257 ty16 168, ty8 171; BF16 65 x 63 x 61 ty4 ry2 4.5,
+        // ry4 4.9, 128^3 8.4 / 7.5, 320^3 vx2 ty4 48.9, ty8 49.8, 384^3 66.3 / 67.1.
         const bool pair = nx % 2 == 0 && aligned4;
         const double cells = (double)nx * ny * nz;
         const double M = 1 << 20;

@@ -198,9 +198,9 @@ int appfis_reduce_device_noalloc(appfis_ctx* ctx, const void* data, int dtype, i
  * buffered.  bufs[0] holds the field at entry; after `iters` sweeps the field is in
  * bufs[iters % 2] (the Grid::Swap parity).  dtype F64 or F32.
  * variant PLAIN: one sweep per launch.  CHOSEN: `tsteps` sweeps per launch with a
- * register-resident tile (temporal blocking); tsteps <= 0 picks the tuned depth.  The
- * ghost rings of the two buffers hold the same values: a launch of CHOSEN reads one of them
- * for all of its sweeps. */
+ * register-resident tile (temporal blocking); tsteps <= 0 picks the tuned depth (and one
+ * sweep per launch for calls of one or two).  The ghost rings of the two buffers hold the
+ * same values: a launch of CHOSEN reads one of them for all of its sweeps. */
 int appfis_heat2d(appfis_ctx* ctx, int dtype, void* buf0, void* buf1, int nx, int ny, double c,
                   int iters, int variant, int tsteps);
 
